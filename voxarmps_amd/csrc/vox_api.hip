@@ -448,7 +448,7 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
         (rc = dalloc(&c->pos_rec, n)) || (rc = dalloc(&c->blockmax, (size_t)grid_for(n))) ||
         (rc = dalloc(&c->blockmax2, (size_t)grid_for(n))))
         return bail(rc);
-    if ((rc = dalloc(&c->uorder, n)) || (rc = dalloc(&c->uscan, n))) return bail(rc);
+    if ((rc = dalloc(&c->uscan, n))) return bail(rc);
     if ((rc = dalloc(&c->uidx, n)) || (rc = dalloc(&c->urow, n)) || (rc = dalloc(&c->uflag, n)) ||
         (rc = dalloc(&c->rowlen, n)) || (rc = dalloc(&c->adiag, n)) || (rc = dalloc(&c->rhs, n)) ||
         (rc = dalloc(&c->cg_x, n)) || (rc = dalloc(&c->cg_r, n)) || (rc = dalloc(&c->cg_p, n)) ||
@@ -487,7 +487,7 @@ int vox_destroy(vox_ctx* c)
     }
     for (int k = 0; k < 6; ++k) dfree(c->sps_s[k]);
     dfree(c->scratch_d); dfree(c->pred_rec); dfree(c->pt_sorted); dfree(c->pos_rec); dfree(c->blockmax); dfree(c->blockmax2);
-    dfree(c->uidx); dfree(c->urow); dfree(c->uflag); dfree(c->uorder); dfree(c->uscan); dfree(c->zcell); dfree(c->rowlen); dfree(c->acol); dfree(c->dcol); dfree(c->cbase); dfree(c->wcol); dfree(c->wuniq); dfree(c->wn);
+    dfree(c->uidx); dfree(c->urow); dfree(c->uflag); dfree(c->uscan); dfree(c->rowlen); dfree(c->acol); dfree(c->dcol); dfree(c->cbase); dfree(c->wcol); dfree(c->wuniq); dfree(c->wn);
     dfree(c->aval); dfree(c->adiag); dfree(c->rhs);
     dfree(c->cg_x); dfree(c->cg_r); dfree(c->cg_p); dfree(c->cg_q); dfree(c->cg_d); dfree(c->cg_e);
     dfree(c->cg_x32); dfree(c->cg_r32); dfree(c->cg_p32); dfree(c->cg_q32); dfree(c->aval32);
@@ -840,7 +840,14 @@ int vox_get_cells(vox_ctx* c, int which, int32_t* cell)
 {
     VOX_TRY(check_ctx(c));
     if (!cell || (which != VOX_LIST_S && which != VOX_LIST_L)) return fail(VOX_ERR_ARG, "bad args");
-    VOX_HIP(hipMemcpy(cell, list_of(c, which).cell, sizeof(int32_t) * c->tp, hipMemcpyDeviceToHost));
+    const DevList& L = list_of(c, which);
+    VOX_HIP(hipMemcpy(cell, L.cell, sizeof(int32_t) * c->tp, hipMemcpyDeviceToHost));
+    if (!L.sorted) return VOX_OK;
+    const Grid& g = L.g;               // the reference numbers the cells x fastest
+    for (int i = 0; i < c->tp; ++i) {
+        const int k = cell[i], iz = k % g.ncz, iy = k / g.ncz % g.ncy, ix = k / g.ncz / g.ncy;
+        cell[i] = ix + iy * g.ncx + iz * g.ncx * g.ncy;
+    }
     return VOX_OK;
 }
 

@@ -20,9 +20,9 @@
 //
 // Pipeline per list: key+count (atomic histogram) -> exclusive scan (cell
 // start) -> atomic scatter -> per-cell rank sort by id (one wave per cell,
-// LDS tile) with position records copied into cell order -> per-particle stencil
-// walk (one thread per particle, or a wave per 64 sorted particles) writing sliced rows
-// (sl_index). With two radii the two lists' pipelines run on two streams.
+// LDS tile) with position records copied into cell order -> stencil walk (one
+// thread per particle, or a wave per 64 sorted particles on the matrix cores) writing
+// sliced rows (sl_index). With two radii the two lists' pipelines run on two streams.
 #include <utility>
 
 #include "vox_internal.hpp"
@@ -183,6 +183,22 @@ __device__ __forceinline__ bool cell_coords(const Grid& g, double x, double y, d
     return ic >= 1 && ic <= g.ncx && jc >= 1 && jc <= g.ncy && kc >= 1 && kc <= g.ncz;
 }
 
+// Cell number with the innermost stencil axis fastest (z in 3D, y in 2D; then
+// y, then x), the order the reference walks a stencil in (functions.cu:2871-2890):
+// the cells of one (x, y) column of a stencil are one contiguous run of the
+// cell-sorted records, and a row's entries ascend in position. Before, cells
+// were numbered x fastest, as the reference does (2826-2834; vox_get_cells
+// still reports that number).
+__host__ __device__ __forceinline__ int cell_key(const Grid& g, int ix, int iy, int iz)
+{
+    return (ix * g.ncy + iy) * g.ncz + iz;
+}
+// Cells along the innermost axis: key = row * inner_cells + inner.
+__host__ __device__ __forceinline__ int inner_cells(const Grid& g)
+{
+    return g.dim == 3 ? g.ncz : g.ncy;
+}
+
 // ctr[key] += 1 for every active lane of the wave, with one atomic per
 // distinct key: consecutive particles mostly share a cell, so per-lane atomics
 // on one counter serialise. Returns the lane's slot among the key's
@@ -220,7 +236,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_keys(Grid g, int n, const doubl
         int ic, jc, kc;
         double zi = (g.dim == 3) ? z[i] : 0.0;
         if (cell_coords(g, x[i], y[i], zi, ic, jc, kc)) {
-            key = (ic - 1) + (jc - 1) * g.ncx + (kc - 1) * g.ncx * g.ncy;   // 2826-2834, 0-based
+            key = cell_key(g, ic - 1, jc - 1, kc - 1);
         } else {
             atomicAdd(&flags[FLAG_DOMAIN], 1);
             atomicMin(&flags[FLAG_DOMAIN_FIRST], i);
@@ -353,52 +369,51 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
     if (t < n) {
         const PosRec me = rec[t];
         const int i = me.id;
-        const int32_t key = me.aux;
-        const int ncxy = g.ncx * g.ncy;
-        const int ic = key % g.ncx + 1;
-        const int jc = (key / g.ncx) % g.ncy + 1;
-        const int kc = key / ncxy + 1;
-        const int m1 = (ic == 1) ? 0 : -1, m2 = (ic == g.ncx) ? 0 : 1;
-        const int m3 = (jc == 1) ? 0 : -1, m4 = (jc == g.ncy) ? 0 : 1;
-        int m5 = 0, m6 = 0;
-        if (g.dim == 3) { m5 = (kc == 1) ? 0 : -1; m6 = (kc == g.ncz) ? 0 : 1; }
+        const int ni = inner_cells(g);
+        const int row = me.aux / ni, in = me.aux % ni;
+        const int ix = (g.dim == 3) ? row / g.ncy : row, iy = (g.dim == 3) ? row % g.ncy : 0;
+        const int x1 = max(ix - 1, 0), x2 = min(ix + 1, g.ncx - 1);
+        const int y1 = (g.dim == 3) ? max(iy - 1, 0) : 0;
+        const int y2 = (g.dim == 3) ? min(iy + 1, g.ncy - 1) : 0;
+        const int ny = (g.dim == 3) ? g.ncy : 1;
+        const int i1 = max(in - 1, 0), i2 = min(in + 1, ni - 1) + 1;
         const double xi = me.x, yi = me.y, zi = me.z;
         const double R2 = R * R;
         const double lo = R2 * (1.0 - 1e-10), hi = R2 * (1.0 + 1e-10);
         const long rb = sl_index(i, 0, cap);
-        for (int row = m1; row <= m2; ++row)
-            for (int col = m3; col <= m4; ++col)
-                for (int dep = m5; dep <= m6; ++dep) {
-                    int cn = (ic - 1 + row) + (jc - 1 + col) * g.ncx + (kc - 1 + dep) * ncxy;
-                    const int s = start[cn], e = start[cn + 1];
-                    // chunks of 8 candidates: loads first, then the ordered
-                    // accept/store pass (stores would serialise later loads)
-                    constexpr int U = 8;
-                    for (int j0 = s; j0 < e; j0 += U) {
-                        PosRec cr[U];
+        for (int xb = x1; xb <= x2; ++xb)
+            for (int yb = y1; yb <= y2; ++yb) {
+                // the innermost axis' cells are one run of records
+                const int cn = (xb * ny + yb) * ni;
+                const int s = start[cn + i1], e = start[cn + i2];
+                // chunks of 8 candidates: loads first, then the ordered
+                // accept/store pass (stores would serialise later loads)
+                constexpr int U = 8;
+                for (int j0 = s; j0 < e; j0 += U) {
+                    PosRec cr[U];
 #pragma unroll
-                        for (int u = 0; u < U; ++u) cr[u] = rec[(j0 + u < e) ? j0 + u : s];
-                        const int k0 = k;
+                    for (int u = 0; u < U; ++u) cr[u] = rec[(j0 + u < e) ? j0 + u : s];
+                    const int k0 = k;
 #pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            // branch-free test (the loads above stay unconditional)
-                            // z is 0 in 2D records: dx^2+dy^2+0 equals the 2D sum
-                            const PosRec cu = cr[u];
-                            const double dx = cu.x - xi, dy = cu.y - yi, dz = cu.z - zi;
-                            const double d2 = dx * dx + dy * dy + dz * dz;
-                            bool acc = d2 < lo;
-                            if (!acc && !(d2 > hi))   // rare band: exact sqrt decides
-                                acc = g.incl ? (sqrt(d2) <= R) : (sqrt(d2) < R);
-                            acc = acc && (j0 + u < e) && (g.incl || cu.id != i);
-                            if (acc) {
-                                ring[k & 15] = cu.id;
-                                ++k;
-                            }
+                    for (int u = 0; u < U; ++u) {
+                        // branch-free test (the loads above stay unconditional)
+                        // z is 0 in 2D records: dx^2+dy^2+0 equals the 2D sum
+                        const PosRec cu = cr[u];
+                        const double dx = cu.x - xi, dy = cu.y - yi, dz = cu.z - zi;
+                        const double d2 = dx * dx + dy * dy + dz * dz;
+                        bool acc = d2 < lo;
+                        if (!acc && !(d2 > hi))   // rare band: exact sqrt decides
+                            acc = g.incl ? (sqrt(d2) <= R) : (sqrt(d2) < R);
+                        acc = acc && (j0 + u < e) && (g.incl || cu.id != i);
+                        if (acc) {
+                            ring[k & 15] = cu.id;
+                            ++k;
                         }
-                        // at most 8 accepts per chunk: at most one group completed
-                        if ((k0 >> 3) != (k >> 3)) flush_ids(ring, k0 >> 3, cap, ids + rb);
                     }
+                    // at most 8 accepts per chunk: at most one group completed
+                    if ((k0 >> 3) != (k >> 3)) flush_ids(ring, k0 >> 3, cap, ids + rb);
                 }
+            }
         if (k & 7) flush_ids(ring, k >> 3, cap, ids + rb);
         cnt[i] = k;
         if (k > cap) atomicAdd(&flags[flag_overflow], 1);
@@ -416,116 +431,281 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
     (void)flag_max;
 }
 
-// Stencil walk for large cells (3D list L: 64-80 particles per cell). A wave
-// takes 64 consecutive particles of the cell-sorted order - one to a few
-// cells of one x-row of the grid - and streams the union of their stencils
-// once: x-blocks from the first lane's cell - 1 to the last lane's + 1, in
-// each the (y, z) cells of the row's stencil in reference order, each cell's
-// records in chunks of 64 through LDS, every lane testing every candidate
-// (broadcast reads). A lane takes the candidates of its own three x-blocks
-// only; its candidate sequence is therefore exactly its stencil in reference
-// order (x outer, then y, then z, ascending id inside a cell). Lanes of
-// another grid row, or more than one cell further along x than the group's
-// first lane, are served by the next pass of the same wave, so a pass never
-// streams more than four x-blocks. Against one wave per cell, lanes stay
-// filled where a cell holds more than 64 particles or fewer.
-// The accept test screens with a fused distance (within a few ulps of the
-// reference's unfused sum); only inside the +-1e-10 band around R, where the
-// two could disagree, does the reference's own expression and sqrt decide.
-// The order and the row storage are those of k_build_list.
+// Stencil walk for cells that hold many particles (3D list L: 64-80 a cell),
+// on the matrix cores. A wave takes 64 consecutive particles of the
+// cell-sorted order: one or a few cells of one row of cells along the innermost
+// axis. The lanes of one row form a group (a wave that straddles rows makes a
+// pass per row) and share its stencil: three runs of records in 2D, nine in
+// 3D, streamed in blocks of 64 candidates. The squared distances of a block
+// are a product: with positions relative to the group's first particle in
+// units of R,
+//   |p - c|^2 = |c|^2 + [c_x c_y c_z 1] . [-2p_x -2p_y -2p_z |p|^2],
+// so one v_mfma_f32_16x16x4_f32 gives 16 candidates x 16 particles and a
+// compare with 1 - |c|^2 decides each pair, where the vector units took
+// 14 instructions a pair (3 differences, 3 products, the band tests, the
+// append) in the walk this replaced.
+// What FP32 cannot decide is decided as the reference does: every pair within
+// kMmEps (|p|max + |c|)^2 of the radius (the rounding of the coordinates, of the
+// product's five terms and of the threshold stays below a quarter of it) goes to
+// a queue in LDS, evaluated 64 at a time with the reference's own expression in
+// FP64 (functions.cu:2886, 2907), together with the cell test that a pair two
+// cells apart needs. Such pairs are about 0.1 a particle in a moving fluid and
+// the six at exactly 4 spacings on a lattice.
+// A lane then walks its particle's accepted bits in candidate order (x outer,
+// then y, then z, ascending id inside a cell: the reference's order) into a
+// ring of 32 entries and stores completed groups of 8.
+// Bound by VALU issue (15,600 instructions a wave on list L, 70% busy).
+// Measured against the walk on vector units it replaced: list L of 199,000
+// particles 554 -> 205 us, 305,000 particles on one 3.2 spacings radius
+// 574 -> 284 us; at 1,180,000 particles both lists beside each other on two
+// streams 2.0 -> 1.2 ms.
 // kPos: the rows hold each neighbour's position in rec instead of its id.
+typedef float v4fm __attribute__((ext_vector_type(4)));
+constexpr float kMmEps = 1.9073486328125e-6f;      // 2^-19
+constexpr int kMmRing = 32;                        // entries: 7 waiting + 16 accepted
+
+__device__ __forceinline__ v4fm mfma_f32_k4(float a, float b, v4fm c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Entries 8 grp .. 8 grp + 7 of a lane's ring (slot-major: a lane's bank is
+// its own) to its row; positions become ids where the rows hold ids. Only the
+// first k entries of the row are positions: slots past them are not read as such.
 template <bool kPos>
-__global__ __launch_bounds__(kWave) void k_build_list_xrow(
+__device__ __forceinline__ void mm_flush(const int32_t* ring, int grp, int k, int cap,
+                                         const PosRec* __restrict__ rec, int32_t* __restrict__ row)
+{
+    if ((grp << 3) >= cap) return;
+    const int s0 = (grp & (kMmRing / 8 - 1)) * 8;
+    int32_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = ring[(s0 + u) * kWave];
+    if (!kPos) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = rec[8 * grp + u < k ? v[u] : 0].id;
+    }
+    v4i* o = reinterpret_cast<v4i*>(row + ((long)grp << 9));
+    o[0] = v4i{v[0], v[1], v[2], v[3]};
+    o[1] = v4i{v[4], v[5], v[6], v[7]};
+}
+
+template <bool kPos>
+__global__ __launch_bounds__(kWave, 4) void k_build_list_mm(
     Grid g, int n, double R, const int32_t* __restrict__ start, const PosRec* __restrict__ rec,
     int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ flags,
     int flag_overflow, int flag_max)
 {
-    __shared__ PosRec tile[kWave];
-    __shared__ int32_t ring_all[kWave * kIdRing];
-    int32_t* ring = ring_all + threadIdx.x * kIdRing;
+    __shared__ __align__(16) float comp[4][kWave];      // candidates: x, y, z and 1
+    __shared__ __align__(16) float thr[kWave];          // |c|^2 - 1
+    __shared__ __align__(8) uint32_t mask[kWave][2];    // a particle's accepted candidates:
+                                                        // 16 bits a tile, the first highest
+    __shared__ __align__(8) uint32_t flip[kWave][2];    // and those the exact test decides otherwise
+    __shared__ uint16_t queue[2 * kWave];               // particle | candidate << 6 | accepted << 12
+    __shared__ int32_t ring_all[kMmRing * kWave];
     const int lane = threadIdx.x;
-    const long t = (long)xcd_block() * kWave + lane;
+    int32_t* ring = ring_all + lane;
+    char* const slots = reinterpret_cast<char*>(ring_all);
+    constexpr uint32_t kSlotMask = kMmRing * kWave * 4 - 1;
+    static_assert(4 * kWave == 256, "a ring slot holds 64 lanes' entries");
+    const int t0 = xcd_block() * kWave;
+    const int t = t0 + lane;
     const bool valid = t < n;
     const PosRec me = rec[valid ? t : 0];
-    const int i = me.id;
-    const int key = me.aux;                           // cell, 0-based
-    const int ix = key % g.ncx;
-    const int rowkey = key / g.ncx;                   // y + ncy z
-    const long ncxy = (long)g.ncx * g.ncy;
+    const int ni = inner_cells(g), ny = (g.dim == 3) ? g.ncy : 1;
+    const int myrow = me.aux / ni, myin = me.aux % ni;
+    const double invR = 1.0 / R;
+    const float wide = fmaxf((float)(fmax(g.hx, g.hz) * invR), 1.f);   // a cell, in units of R
     // rows of positions are stored at the particle's own position too
-    const long rb = sl_index(kPos ? t : (long)i, 0, cap);
-    const double R2 = R * R;
-    const double lo = R2 * (1.0 - 1e-10), hi = R2 * (1.0 + 1e-10);
-    int k = 0;
-    const int tt = (int)t;
+    const long rb = sl_index(kPos ? t : (long)me.id, 0, cap);
+    const int cl = lane & 15, cg = lane >> 4;
+    int k = 0, kf = 0;                                  // entries accepted, entries stored
+    uint32_t at = 4u * lane;                            // byte of the next free ring slot
+    mask[lane][0] = mask[lane][1] = flip[lane][0] = flip[lane][1] = 0u;
     unsigned long long todo = __ballot(valid);
     while (todo) {
-        // the group's cell row and x-range are the same for every lane: kept
-        // in scalar registers, so the walk's cell bounds and the candidate
-        // index are scalar too
         const int lead = __ffsll(todo) - 1;
-        const int grow = __builtin_amdgcn_readfirstlane(__shfl(rowkey, lead));
-        const int gx = __builtin_amdgcn_readfirstlane(__shfl(ix, lead));
-        const bool mine = valid && rowkey == grow && ix <= gx + 1 && ((todo >> lane) & 1ull);
+        const int row = __builtin_amdgcn_readfirstlane(__shfl(myrow, lead));
+        const bool mine = valid && myrow == row;
         const unsigned long long m = __ballot(mine);
         todo &= ~m;
         const int last = 63 - __clzll(m);
-        const int x_lo = max(gx - 1, 0);
-        const int x_hi = min(__builtin_amdgcn_readfirstlane(__shfl(ix, last)) + 1, g.ncx - 1);
-        const int gy = grow % g.ncy, gz = grow / g.ncy;
-        const int y_lo = max(gy - 1, 0), y_hi = min(gy + 1, g.ncy - 1);
-        const int z_lo = (g.dim == 3) ? max(gz - 1, 0) : 0;
-        const int z_hi = (g.dim == 3) ? min(gz + 1, g.ncz - 1) : 0;
-        for (int xb = x_lo; xb <= x_hi; ++xb) {
-            const bool on = mine && xb >= ix - 1 && xb <= ix + 1;
-            for (int yb = y_lo; yb <= y_hi; ++yb)
-                for (int zb = z_lo; zb <= z_hi; ++zb) {
-                    const long cn = xb + yb * (long)g.ncx + zb * ncxy;
-                    const int cs = __builtin_amdgcn_readfirstlane(start[cn]);
-                    const int ce = __builtin_amdgcn_readfirstlane(start[cn + 1]);
-                    for (int j0 = cs; j0 < ce; j0 += kWave) {
-                        const int nc = min(kWave, ce - j0);
-                        __syncthreads();                   // last chunk's reads are done
-                        if (lane < nc) tile[lane] = rec[j0 + lane];
-                        __syncthreads();
-                        // groups of 8 candidates: at most one group of 8
-                        // accepts completes per group. Slots past nc hold
-                        // stale records and are never accepted.
-                        for (int u0 = 0; u0 < nc; u0 += 8) {
-                            const int k0 = k;
+        const int in_lo = __builtin_amdgcn_readfirstlane(__shfl(myin, lead));
+        const int in_hi = __builtin_amdgcn_readfirstlane(__shfl(myin, last));
+        const double ox = __shfl(me.x, lead), oy = __shfl(me.y, lead), oz = __shfl(me.z, lead);
+        const float px = mine ? (float)((me.x - ox) * invR) : 0.f;
+        const float py = mine ? (float)((me.y - oy) * invR) : 0.f;
+        const float pz = mine ? (float)((me.z - oz) * invR) : 0.f;
+        const float p2 = px * px + py * py + pz * pz;
+        // the group's largest distance from its origin and its bounding box
+        // (the lead itself sits at 0, the value of the other lanes)
+        float pm = p2, bx = px, by = py, bz = pz, Bx = px, By = py, Bz = pz;
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            pm = fmaxf(pm, __shfl_xor(pm, off));
+            bx = fminf(bx, __shfl_xor(bx, off)); Bx = fmaxf(Bx, __shfl_xor(Bx, off));
+            by = fminf(by, __shfl_xor(by, off)); By = fmaxf(By, __shfl_xor(By, off));
+            bz = fminf(bz, __shfl_xor(bz, off)); Bz = fmaxf(Bz, __shfl_xor(Bz, off));
+        }
+        pm = sqrtf(pm);
+        // no candidate is more than two cells along an axis from a particle of
+        // the group: |c| <= |p|max + 2 sqrt(3) cells
+        const float reach = 2.f * pm + 4.f * wide + 1.f;
+        const float eps = kMmEps * reach * reach;
+        __syncthreads();
+        comp[0][lane] = -2.f * px;
+        comp[1][lane] = -2.f * py;
+        comp[2][lane] = -2.f * pz;
+        comp[3][lane] = mine ? p2 : 1e30f;              // no candidate is near another row's lanes
+        __syncthreads();
+        float bp[4];
 #pragma unroll
-                            for (int uu = 0; uu < 8; ++uu) {
-                                const int u = u0 + uu;
-                                // z is 0 in 2D records
-                                const double dx = tile[u].x - me.x, dy = tile[u].y - me.y,
-                                             dz = tile[u].z - me.z;
-                                const double d2f = fma(dz, dz, fma(dy, dy, dx * dx));
-                                const bool sure = d2f < lo;
-                                const bool near = d2f <= hi;
-                                bool acc = sure;
-                                if (near != sure) {          // rare band: the reference's expression
-                                    const double d2 = dx * dx + dy * dy + dz * dz;
-                                    acc = g.incl ? (sqrt(d2) <= R) : (sqrt(d2) < R);
-                                }
-                                // the particle itself: by its position in rec (rows
-                                // of positions), else by id
-                                const bool other = kPos ? (j0 + u != tt) : (tile[u].id != i);
-                                acc = acc && on && (u < nc) && (g.incl || other);
-                                // the next free slot takes every candidate; only
-                                // an accepted one advances past it
-                                ring[k & 15] = kPos ? j0 + u : tile[u].id;
-                                k += acc ? 1 : 0;
+        for (int q = 0; q < 4; ++q) bp[q] = comp[cg][16 * q + cl];
+        __syncthreads();
+        comp[3][lane] = 1.f;
+        const int ix = (g.dim == 3) ? row / g.ncy : row, iy = (g.dim == 3) ? row % g.ncy : 0;
+        const int x1 = max(ix - 1, 0), x2 = min(ix + 1, g.ncx - 1);
+        const int y1 = (g.dim == 3) ? max(iy - 1, 0) : 0;
+        const int y2 = (g.dim == 3) ? min(iy + 1, g.ncy - 1) : 0;
+        const int i1 = max(in_lo - 1, 0), i2 = min(in_hi + 1, ni - 1) + 1;
+        for (int xb = x1; xb <= x2; ++xb)
+            for (int yb = y1; yb <= y2; ++yb) {
+                const int cn = (xb * ny + yb) * ni;
+                const int cs = __builtin_amdgcn_readfirstlane(start[cn + i1]);
+                const int ce = __builtin_amdgcn_readfirstlane(start[cn + i2]);
+                PosRec nx = rec[min(cs + lane, n - 1)];
+                for (int b0 = cs; b0 < ce; b0 += kWave) {
+                    const int nc = min(kWave, ce - b0);
+                    const PosRec cr = nx;
+                    nx = rec[min(b0 + kWave + lane, n - 1)];                  // the next block's
+                    const float cx = (float)((cr.x - ox) * invR);
+                    const float cy = (float)((cr.y - oy) * invR);
+                    const float cz = (float)((cr.z - oz) * invR);
+                    const float c2 = cx * cx + cy * cy + cz * cz;
+                    const bool in = lane < nc;
+                    // tiles whose candidates are all out of reach of the
+                    // group's box are left out
+                    const float gx = fmaxf(fmaxf(bx - cx, cx - Bx), 0.f);
+                    const float gy = fmaxf(fmaxf(by - cy, cy - By), 0.f);
+                    const float gz = fmaxf(fmaxf(bz - cz, cz - Bz), 0.f);
+                    const unsigned long long near =
+                        __ballot(in && gx * gx + gy * gy + gz * gz < 1.f + eps);
+                    if (!near) continue;
+                    __syncthreads();                    // the last block's reads are done
+                    comp[0][lane] = in ? cx : 0.f;
+                    comp[1][lane] = in ? cy : 0.f;
+                    comp[2][lane] = in ? cz : 0.f;
+                    thr[lane] = in ? c2 - 1.f : 1e30f;
+                    __syncthreads();
+                    int nq = 0;
+                    bool took = false;
+                    // the exact test of the first `count` queued pairs
+                    auto drain = [&](int count) {
+                        __syncthreads();
+                        if (lane < count) {
+                            const uint32_t it = queue[lane];
+                            const int pl = it & 63, c = (it >> 6) & 63;
+                            const PosRec P = rec[t0 + pl], C = rec[b0 + c];
+                            const double dx = C.x - P.x, dy = C.y - P.y, dz = C.z - P.z;
+                            const double d = sqrt(dx * dx + dy * dy + dz * dz);
+                            const int away = C.aux % ni - P.aux % ni;
+                            const bool acc = (g.incl ? d <= R : d < R) && away >= -1 && away <= 1;
+                            if (acc != ((it >> 12) != 0u))
+                                atomicOr(&flip[pl][c >> 5], 0x8000u >> (c & 15) << (c & 16));
+                        }
+                        __syncthreads();
+                    };
+#pragma unroll 1
+                    for (int tile = 0; tile < 4; ++tile) {
+                        if (!((near >> (16 * tile)) & 0xffffull)) continue;
+                        const int c0 = 16 * tile + 4 * cg;          // this lane's candidates
+                        const float a = comp[cg][16 * tile + cl];
+                        const v4fm t4 = *reinterpret_cast<const v4fm*>(&thr[c0]);
+                        v4fm d[4];                                  // |p - c|^2 - 1
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) d[q] = mfma_f32_k4(a, bp[q], t4);
+                        const int sh = 12 - 4 * cg + 16 * (tile & 1);
+                        float least = 1e30f;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            uint32_t nib = 0u;                      // the four sign bits
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                nib = (nib << 1) | (__float_as_uint(d[q][i]) >> 31);
+                                least = fminf(least, fabsf(d[q][i]));
                             }
-                            if ((k0 >> 3) != (k >> 3)) flush_ids(ring, k0 >> 3, cap, ids + rb);
+                            atomicOr(&mask[16 * q + cl][tile >> 1], nib << sh);
+                        }
+                        if (__any(least < eps)) {
+                            took = true;
+                            uint32_t ub = 0u, sg = 0u;              // bit 4 q + i
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    ub |= (fabsf(d[q][i]) < eps) ? 1u << (4 * q + i) : 0u;
+                                    sg |= (__float_as_uint(d[q][i]) >> 31) << (4 * q + i);
+                                }
+                            for (;;) {
+                                const unsigned long long um = __ballot(ub != 0u);
+                                if (!um) break;
+                                if (ub) {
+                                    const int b = __ffs(ub) - 1;
+                                    ub &= ub - 1u;
+                                    queue[nq + __popcll(um & ((1ull << lane) - 1ull))] =
+                                        (uint16_t)((16 * (b >> 2) + cl) | ((c0 + (b & 3)) << 6) |
+                                                   (((sg >> b) & 1u) << 12));
+                                }
+                                nq += __popcll(um);
+                                if (nq >= kWave) {
+                                    drain(kWave);
+                                    const uint16_t left = queue[kWave + lane];
+                                    __syncthreads();
+                                    queue[lane] = left;
+                                    nq -= kWave;
+                                }
+                            }
+                        }
+                    }
+                    if (nq) drain(nq);
+                    __syncthreads();
+                    uint32_t own[2] = {mask[lane][0], mask[lane][1]};
+                    mask[lane][0] = mask[lane][1] = 0u;
+                    if (took) {
+                        own[0] ^= flip[lane][0];
+                        own[1] ^= flip[lane][1];
+                        flip[lane][0] = flip[lane][1] = 0u;
+                    }
+                    const int self = t - b0;
+                    if (!g.incl && self >= 0 && self < nc) {        // the particle itself
+                        const uint32_t bit = 0x8000u >> (self & 15) << (self & 16);
+                        if (self >> 5) own[1] &= ~bit;
+                        else own[0] &= ~bit;
+                    }
+#pragma unroll 1
+                    for (int tile = 0; tile < 4; ++tile) {
+                        const uint32_t h = (((tile & 2) ? own[1] : own[0]) >> (16 * (tile & 1))) & 0xffffu;
+                        if (!__any(h != 0u)) continue;
+                        // the next free slot takes every candidate; only an
+                        // accepted one advances past it
+                        const int base = b0 + 16 * tile;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            *reinterpret_cast<int32_t*>(slots + at) = base + e;
+                            at = (at + (__builtin_amdgcn_ubfe(h, 15 - e, 1) << 8)) & kSlotMask;
+                        }
+                        k += __popc(h);
+                        while ((kf >> 3) < (k >> 3)) {
+                            mm_flush<kPos>(ring, kf >> 3, k, cap, rec, ids + rb);
+                            kf += 8;
                         }
                     }
                 }
-        }
+            }
     }
-    if (valid && (k & 7)) flush_ids(ring, k >> 3, cap, ids + rb);
+    if (valid && (k & 7)) mm_flush<kPos>(ring, k >> 3, k, cap, rec, ids + rb);
     int kmax = 0;
     if (valid) {
-        cnt[kPos ? t : (long)i] = k;
+        cnt[kPos ? t : (long)me.id] = k;
         if (k > cap) atomicAdd(&flags[flag_overflow], 1);
         kmax = k;
     }
@@ -667,8 +847,12 @@ static int search_one(vox_ctx* c, int which, double re)
     const double R = gg.incl ? re + c->p.delta : re;
     L.compact = compact;
     L.epoch = c->pos_epoch;
-    // Walk per cell when cells hold enough particles to fill most of a wave
-    // (expected count = cell volume / DL^dim), else per particle.
+    // The matrix-core walk where a cell is expected (cell volume / DL^dim) to
+    // hold 24 particles or more, else the walk per particle. NEIGHBOR calls
+    // measured with either, matrix against per particle, us: 3D 67 a cell 1500
+    // against 2480 (1,185,000 particles), 330 against 590 (201,000), 200 against
+    // 270 (15,500); 35 a cell 1005 / 1420, 250 / 370, 170 / 190; 10 a cell 650 /
+    // 630, 200 / 190, 150 / 104; 2D 16 a cell 354 / 296 (979,000), 4 a cell 395 / 210.
     const double per_cell = (c->p.dim == 3)
         ? L.g.hx * L.g.hx * L.g.hz / (c->p.dl * c->p.dl * c->p.dl)
         : L.g.hx * L.g.hx / (c->p.dl * c->p.dl);
@@ -684,10 +868,10 @@ static int search_one(vox_ctx* c, int which, double re)
     if (cell_walk) {
         VOX_TRY(fill_i32(c, c->dflags + fm, 0, 1));
         if (L.pos_rows)
-            k_build_list_xrow<true><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
+            k_build_list_mm<true><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
                 gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
         else
-            k_build_list_xrow<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
+            k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
                 gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
     } else {
         const int nb = grid_for(n);
@@ -752,7 +936,7 @@ int ensure_reference_list(vox_ctx* c, int which)
     for (int attempt = 0; attempt < 4; ++attempt) {
         VOX_TRY(fill_i32(c, c->dflags + fo, 0, 1));
         VOX_TRY(fill_i32(c, c->dflags + fm, 0, 1));
-        k_build_list_xrow<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
+        k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
             L.g, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
         VOX_HIP(hipGetLastError());
         L.pos_rows = false;

@@ -36,47 +36,27 @@ __global__ void k_umap(int n, const int32_t* __restrict__ bcon, int32_t* __restr
 }
 
 // ---- numbering of the unknowns -------------------------------------------------------
-// The unknowns are the bcon = 0 particles, numbered in the cell order of list
-// L's grid with z fastest (then y, then x; inside a cell by particle id), so
-// the assembly's rows and the solver's vectors run through space cell by
-// cell: a wave's 64 rows are neighbours, and so are most of their columns.
-// The reference numbers them in particle order (functions.cu:869-925); the
-// export maps back to it. Before the first NEIGHBOR, and for a dump of the
-// learned network's training systems, particle order is used.
-__device__ __forceinline__ int zkey(const Grid& g, int c)
-{
-    const int ix = c % g.ncx, iy = (c / g.ncx) % g.ncy, iz = c / (g.ncx * g.ncy);
-    return iz + g.ncz * (iy + g.ncy * ix);
-}
-
-__global__ void k_zcount(Grid g, const int32_t* __restrict__ start, int32_t* __restrict__ zcnt)
-{
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < g.tnc) zcnt[zkey(g, (int)c)] = start[c + 1] - start[c];
-}
-
-// Position t of the list's cell-sorted records goes to its cell's start in
-// z-fastest order plus its rank inside the cell.
-__global__ void k_uorder(int n, Grid g, const PosRec* __restrict__ rec,
-                         const int32_t* __restrict__ start, const int32_t* __restrict__ zstart,
-                         const int32_t* __restrict__ bcon, int32_t* __restrict__ uflag,
-                         int32_t* __restrict__ uorder)
+// The unknowns are the bcon = 0 particles, numbered in the cell-sorted order of
+// list L (innermost axis fastest; inside a cell by particle id), so the
+// assembly's rows and the solver's vectors run through space cell by cell: a
+// wave's 64 rows are neighbours, and so are most of their columns. The
+// reference numbers them in particle order (functions.cu:869-925); the export
+// maps back to it. Before the first NEIGHBOR, and for a dump of the learned
+// network's training systems, particle order is used.
+__global__ void k_uflag_order(int n, const PosRec* __restrict__ rec,
+                              const int32_t* __restrict__ bcon, int32_t* __restrict__ uflag)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const PosRec r = rec[t];
-    const int np = zstart[zkey(g, r.aux)] + (t - start[r.aux]);
-    uorder[np] = r.id;
-    uflag[np] = (bcon[r.id] == 0) ? 1 : 0;
+    if (t < n) uflag[t] = (bcon[rec[t].id] == 0) ? 1 : 0;
 }
 
-__global__ void k_umap_order(int n, const int32_t* __restrict__ uorder,
+__global__ void k_umap_order(int n, const PosRec* __restrict__ rec,
                              const int32_t* __restrict__ uflag, const int32_t* __restrict__ uscan,
                              int32_t* __restrict__ uidx, int32_t* __restrict__ urow)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    const int id = uorder[t];
+    const int id = rec[t].id;
     if (uflag[t]) {
         const int r = uscan[t];
         uidx[id] = r;
@@ -98,21 +78,9 @@ static int number_unknowns(vox_ctx* c)
         c->uorder_cells = false;
         return VOX_OK;
     }
-    const long tnc = L.g.tnc;
-    if (c->zcell_alloc < tnc) {
-        if (c->zcell) (void)hipFree(c->zcell);
-        c->zcell = nullptr;
-        VOX_HIP(hipMalloc(&c->zcell, sizeof(int32_t) * 2 * (size_t)(tnc + 1)));
-        c->zcell_alloc = tnc;
-    }
-    int32_t* zcnt = c->zcell;
-    int32_t* zstart = c->zcell + (tnc + 1);
-    k_zcount<<<grid_for(tnc), kBlock, 0, c->stream>>>(L.g, L.cell_start, zcnt);
-    VOX_TRY(scan_exclusive(c, zcnt, zstart, tnc, zstart + tnc));
-    k_uorder<<<grid_for(n), kBlock, 0, c->stream>>>(n, L.g, L.rec, L.cell_start, zstart, c->bcon,
-                                                     c->uflag, c->uorder);
+    k_uflag_order<<<grid_for(n), kBlock, 0, c->stream>>>(n, L.rec, c->bcon, c->uflag);
     VOX_TRY(scan_exclusive(c, c->uflag, c->uscan, n, c->dflags + FLAG_NU));
-    k_umap_order<<<grid_for(n), kBlock, 0, c->stream>>>(n, c->uorder, c->uflag, c->uscan, c->uidx,
+    k_umap_order<<<grid_for(n), kBlock, 0, c->stream>>>(n, L.rec, c->uflag, c->uscan, c->uidx,
                                                          c->urow);
     VOX_HIP(hipGetLastError());
     c->uorder_cells = true;
