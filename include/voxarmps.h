@@ -121,7 +121,7 @@ typedef struct vox_params {
                              0: from zero, as the reference (functions.cu:2503) */
     int32_t list_mode;    /* neighbour search: 0 auto, 1 one thread per particle,
                              2 one wave per 64 cell-sorted particles on the
-                             matrix cores (same lists either way)                                 */
+                             matrix cores (same lists either way)              */
     int32_t lpc_cap_pct;  /* learned FCG: iteration cap in percent of the Jacobi-CG
                              baseline before the fallback (200: twice)         */
     int32_t method;       /* PRESSURECALC: 1 PPE (incompressible), 3 weakly

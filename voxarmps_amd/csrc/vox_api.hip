@@ -81,12 +81,23 @@ int prof_drain(vox_ctx* c)
 
 int read_flags(vox_ctx* c)
 {
-    VOX_HIP(hipMemcpyAsync(c->hflags, c->dflags, sizeof(int32_t) * FLAG_COUNT,
-                           hipMemcpyDeviceToHost, c->stream));
-    VOX_HIP(hipMemcpyAsync(c->hscal, c->dscal, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost,
-                           c->stream));
+    VOX_HIP(hipMemcpyAsync(c->hstat, c->dstat, kStatBytes, hipMemcpyDeviceToHost, c->stream));
     VOX_HIP(hipStreamSynchronize(c->stream));
     return VOX_OK;
+}
+
+int32_t spread_max(const vox_ctx* c, int slot)
+{
+    int32_t m = 0;
+    for (int k = 0; k < kSpread; ++k) m = std::max(m, c->hspread[k * kSpreadLine + slot]);
+    return m;
+}
+
+int32_t spread_sum(const vox_ctx* c, int slot)
+{
+    int32_t m = 0;
+    for (int k = 0; k < kSpread; ++k) m += c->hspread[k * kSpreadLine + slot];
+    return m;
 }
 
 // Lattice count of neighbours inside the accept radius, used to size rows
@@ -445,8 +456,7 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
     for (int k = 0; k < 6; ++k)
         if ((rc = dalloc(&c->sps_s[k], n))) return bail(rc);
     if ((rc = dalloc(&c->scratch_d, n)) || (rc = dalloc(&c->pred_rec, n)) || (rc = dalloc(&c->pt_sorted, n)) ||
-        (rc = dalloc(&c->pos_rec, n)) || (rc = dalloc(&c->blockmax, (size_t)grid_for(n))) ||
-        (rc = dalloc(&c->blockmax2, (size_t)grid_for(n))))
+        (rc = dalloc(&c->pos_rec, n)))
         return bail(rc);
     if ((rc = dalloc(&c->uscan, n))) return bail(rc);
     if ((rc = dalloc(&c->uidx, n)) || (rc = dalloc(&c->urow, n)) || (rc = dalloc(&c->uflag, n)) ||
@@ -461,14 +471,18 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
         (rc = dalloc(&c->coll_act, n)) || (rc = dalloc(&c->coll_cnt2, n)) || (rc = dalloc(&c->coll_off2, n + 1)) ||
         (rc = dalloc(&c->coll_logn, 1)))
         return bail(rc);
-    if ((rc = dalloc(&c->partials, kPartialSlots * (size_t)kMaxPartials)) || (rc = dalloc(&c->dscal, SC_COUNT)) ||
-        (rc = dalloc(&c->dflags, FLAG_COUNT)))
+    if ((rc = dalloc(&c->partials, kPartialSlots * (size_t)kMaxPartials)) ||
+        (rc = dalloc(&c->dstat, kStatBytes)))
         return bail(rc);
-    if (hipHostMalloc((void**)&c->hflags, sizeof(int32_t) * FLAG_COUNT, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&c->hscal, sizeof(double) * SC_COUNT, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc((void**)&c->hstat, kStatBytes, hipHostMallocDefault) != hipSuccess)
         return bail(fail(VOX_ERR_HIP, "hipHostMalloc"));
-    std::memset(c->hflags, 0, sizeof(int32_t) * FLAG_COUNT);
-    std::memset(c->hscal, 0, sizeof(double) * SC_COUNT);
+    std::memset(c->hstat, 0, kStatBytes);
+    c->dscal = reinterpret_cast<double*>(c->dstat);
+    c->dflags = reinterpret_cast<int32_t*>(c->dstat + kStatFlags);
+    c->dspread = reinterpret_cast<int32_t*>(c->dstat + kStatSpread);
+    c->hscal = reinterpret_cast<double*>(c->hstat);
+    c->hflags = reinterpret_cast<int32_t*>(c->hstat + kStatFlags);
+    c->hspread = reinterpret_cast<int32_t*>(c->hstat + kStatSpread);
     if (hipDeviceSynchronize() != hipSuccess) return bail(fail(VOX_ERR_HIP, "initial sync"));
     *out = c;
     return VOX_OK;
@@ -486,7 +500,7 @@ int vox_destroy(vox_ctx* c)
         dfree(L.order_raw); dfree(L.rec); dfree(L.pos_of);
     }
     for (int k = 0; k < 6; ++k) dfree(c->sps_s[k]);
-    dfree(c->scratch_d); dfree(c->pred_rec); dfree(c->pt_sorted); dfree(c->pos_rec); dfree(c->blockmax); dfree(c->blockmax2);
+    dfree(c->scratch_d); dfree(c->pred_rec); dfree(c->pt_sorted); dfree(c->pos_rec);
     dfree(c->uidx); dfree(c->urow); dfree(c->uflag); dfree(c->uscan); dfree(c->rowlen); dfree(c->acol); dfree(c->dcol); dfree(c->cbase); dfree(c->wcol); dfree(c->wuniq); dfree(c->wn);
     dfree(c->aval); dfree(c->adiag); dfree(c->rhs);
     dfree(c->cg_x); dfree(c->cg_r); dfree(c->cg_p); dfree(c->cg_q); dfree(c->cg_d); dfree(c->cg_e);
@@ -494,10 +508,9 @@ int vox_destroy(vox_ctx* c)
     dfree(c->coll_cnt); dfree(c->coll_off); dfree(c->coll_i); dfree(c->coll_j);
     dfree(c->coll_act); dfree(c->coll_cnt2); dfree(c->coll_off2); dfree(c->coll_i2); dfree(c->coll_j2);
     dfree(c->coll_stamp); dfree(c->coll_root); dfree(c->region); dfree(c->rbox); dfree(c->coll_logidx); dfree(c->coll_log); dfree(c->coll_logn);
-    dfree(c->scan_blocks); dfree(c->scan_blocks2); dfree(c->partials); dfree(c->dscal); dfree(c->dflags);
+    dfree(c->scan_blocks); dfree(c->scan_blocks2); dfree(c->partials); dfree(c->dstat);
     lpc_free_ctx(c);
-    if (c->hflags) (void)hipHostFree(c->hflags);
-    if (c->hscal) (void)hipHostFree(c->hscal);
+    if (c->hstat) (void)hipHostFree(c->hstat);
     for (auto& r : c->prof_pending) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto e : c->prof_free) (void)hipEventDestroy(e);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);

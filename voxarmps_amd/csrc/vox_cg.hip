@@ -325,7 +325,7 @@ struct WinArgs {
     v4u* wcol;
     int32_t* wuniq;
     int32_t* wn;
-    int32_t* flags;
+    int32_t* spread;
 };
 
 // The windows of the LDS-gather product, one block per chunk of 256 rows
@@ -334,7 +334,7 @@ struct WinArgs {
 // the assembly's bound on how far the rows reach below and above their own
 // index), the prefix of its popcounts per word, the distinct columns in
 // ascending order and each entry's rank among them. A chunk with a column
-// past the bitmap or more distinct columns than kWinMax raises FLAG_WIN_N
+// past the bitmap or more distinct columns than kWinMax raises SPR_WIN_N
 // past kWinMax, and the product then reads the column steps. Each lane walks
 // its row 4 chunks (32 entries) per round trip.
 __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
     if (cw >= 0) atomicOr(&bits[cw], cm);
     __syncthreads();
     if (outside) {                                     // uniform
-        if (t == 0) { a.wn[ch] = -1; atomicMax(&a.flags[FLAG_WIN_N], kWinMax + 1); }
+        if (t == 0) { a.wn[ch] = -1; atomicMax(spread_at(a.spread, SPR_WIN_N), kWinMax + 1); }
         return;
     }
     // exclusive prefix of the words' popcounts: thread t owns words [w0, w1)
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
     }
     const int total = red[kBlock - 1];
     if (total > kWinMax) {                             // uniform
-        if (t == 0) { a.wn[ch] = -1; atomicMax(&a.flags[FLAG_WIN_N], kWinMax + 1); }
+        if (t == 0) { a.wn[ch] = -1; atomicMax(spread_at(a.spread, SPR_WIN_N), kWinMax + 1); }
         return;
     }
     int run = red[t] - sum;
@@ -466,8 +466,8 @@ __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
     }
     if (t == 0) {
         a.wn[ch] = total;
-        atomicMax(&a.flags[FLAG_WIN_N], total);
-        atomicAdd(&a.flags[FLAG_WIN_SUM], total);
+        atomicMax(spread_at(a.spread, SPR_WIN_N), total);
+        atomicAdd(spread_at(a.spread, SPR_WIN_SUM), total);
     }
 }
 
@@ -1013,11 +1013,10 @@ static int ensure_window(vox_ctx* c)
     const long span = (long)c->col_below + c->col_above + kBlock;
     const int words = (int)((span + 31) / 32);
     if (words > kWinSpanWords) return VOX_OK;
-    VOX_TRY(fill_i32(c, c->dflags + FLAG_WIN_N, 0, 2));          // and FLAG_WIN_SUM
     WinArgs w;
     w.nu = c->nu; w.cap = c->a_cap; w.words = words; w.rowlen = c->rowlen;
     w.dcol = reinterpret_cast<const v4u*>(c->dcol); w.cbase = c->cbase;
-    w.wcol = reinterpret_cast<v4u*>(c->wcol); w.wuniq = c->wuniq; w.wn = c->wn; w.flags = c->dflags;
+    w.wcol = reinterpret_cast<v4u*>(c->wcol); w.wuniq = c->wuniq; w.wn = c->wn; w.spread = c->dspread;
     {
         ProfScope ps(c, KC_ASSEMBLE);
         const size_t lds = sizeof(uint32_t) * (size_t)words + sizeof(uint16_t) * (size_t)(words + 1);
@@ -1025,8 +1024,8 @@ static int ensure_window(vox_ctx* c)
         VOX_HIP(hipGetLastError());
     }
     VOX_TRY(read_flags(c));
-    c->win_n = c->hflags[FLAG_WIN_N];
-    c->win_sum = c->hflags[FLAG_WIN_SUM];
+    c->win_n = spread_max(c, SPR_WIN_N);
+    c->win_sum = spread_sum(c, SPR_WIN_SUM);
     c->win_ok = c->win_n <= kWinMax;
     return VOX_OK;
 }

@@ -63,10 +63,6 @@ inline int grid_for(long n, int block = kBlock)
 // ---- device flags (int32 slots of ctx->dflags) -------------------------------
 enum DevFlag {
     FLAG_DOMAIN = 0,      // particle outside neighbour grid
-    FLAG_OVERFLOW_S,      // list S row longer than capacity
-    FLAG_OVERFLOW_L,
-    FLAG_MAXCNT_S,        // longest row (atomicMax)
-    FLAG_MAXCNT_L,
     FLAG_NAN,             // PREPDATA ERROR#1 count
     FLAG_OOB,             // PREPDATA ERROR#2 count
     FLAG_COLL_HITS,       // applied collision impulses
@@ -81,15 +77,31 @@ enum DevFlag {
     FLAG_CG_BREAK,
     FLAG_DOMAIN_FIRST,    // smallest index of a particle outside the grid (atomicMin)
     FLAG_DCOL_BAD,        // a PPE row's column steps do not fit 16 bits (see dcol)
-    FLAG_WIN_N,           // most distinct columns of a PPE chunk (atomicMax; see wcol)
-    FLAG_WIN_SUM,         // distinct columns over all chunks (atomicAdd)
-    FLAG_COL_BELOW,       // max over PPE rows of row - first column (atomicMax)
-    FLAG_COL_ABOVE,       // max over PPE rows of last column - row (atomicMax)
     FLAG_COUNT
 };
 
+// Counters that every block of a kernel raises: kSpread copies, each on a
+// cache line of its own (block b uses copy b % kSpread), combined on the host.
+// Atomics of 27,000 blocks on one address took 0.3 ms of a 0.7 ms kernel.
+enum SpreadSlot {
+    SPR_MAXCNT_S = 0,      // longest row of list S (max)
+    SPR_MAXCNT_L,
+    SPR_COL_BELOW,         // over PPE rows: row - first column (max)
+    SPR_COL_ABOVE,         //                last column - row (max)
+    SPR_WIN_N,             // most distinct columns of a PPE chunk (max; see wcol)
+    SPR_WIN_SUM,           // distinct columns over all chunks (sum)
+    SPR_COUNT
+};
+constexpr int kSpread = 32;
+constexpr int kSpreadLine = 32;        // int32 per copy: 128 bytes
+// The status block that read_flags copies to the host in one piece: scalars,
+// flags, spread counters.
+constexpr int kStatFlags = 128, kStatSpread = 256;        // byte offsets
+constexpr int kStatBytes = kStatSpread + 4 * kSpread * kSpreadLine;
+
 // device scalar slots of ctx->dscal (double); the solver names its own
 constexpr int SC_COUNT = 12;
+static_assert(SC_COUNT * 8 <= kStatFlags && FLAG_COUNT * 4 <= kStatSpread - kStatFlags, "status block");
 
 // ---- neighbour grid + list ------------------------------------------------------
 struct Grid {
@@ -231,6 +243,7 @@ struct vox_ctx {
     int32_t* bcon = nullptr;
 
     vox::DevList list[2];
+    int max_count[2] = {0, 0};     // longest row of each list's last search
     int tuned_mode[2] = {0, 0};    // neighbour walk chosen by the autotuner (0: none)
     int tune_pred = 6;             // predictor variant (vox::kPredVariants): 8 records,
                                    // 256 threads, gradient deferred unless tuned
@@ -358,21 +371,23 @@ struct vox_ctx {
     // scan scratch
     int32_t* scan_blocks = nullptr;
     long scan_blocks_cap = 0;
-    int32_t* blockmax = nullptr;   // one slot per 256-particle block
     // side stream of the neighbour build (list L beside list S), with its own
-    // scan scratch and block-maximum slots, and the events joining the streams
+    // scan scratch, and the events joining the streams
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int32_t* scan_blocks2 = nullptr;
     long scan_blocks2_cap = 0;
-    int32_t* blockmax2 = nullptr;
 
     // reductions
     double* partials = nullptr;    // 8 * kMaxPartials
-    double* dscal = nullptr;       // SC_COUNT
-    int32_t* dflags = nullptr;     // FLAG_COUNT
-    int32_t* hflags = nullptr;     // pinned mirror
-    double* hscal = nullptr;       // pinned mirror
+    char* dstat = nullptr;         // the status block and, in it,
+    double* dscal = nullptr;       //   SC_COUNT scalars
+    int32_t* dflags = nullptr;     //   FLAG_COUNT flags
+    int32_t* dspread = nullptr;    //   kSpread copies of the spread counters
+    char* hstat = nullptr;         // pinned mirror
+    double* hscal = nullptr;
+    int32_t* hflags = nullptr;
+    int32_t* hspread = nullptr;
 
     vox_status st{};
 
@@ -427,7 +442,9 @@ int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t*
 int ensure_acol(vox_ctx* c);                                    // vox_ppe.hip
 int fill_i32(vox_ctx* c, int32_t* p, int32_t v, long n);
 int fill_f64(vox_ctx* c, double* p, double v, long n);
-int read_flags(vox_ctx* c);   // D2H of dflags + dscal into pinned mirrors (syncs)
+int read_flags(vox_ctx* c);   // D2H of the status block into its pinned mirror (syncs)
+int32_t spread_max(const vox_ctx* c, int slot);       // of the last read_flags
+int32_t spread_sum(const vox_ctx* c, int slot);
 
 int autotune_lists(vox_ctx* c, int reps, int32_t* modes);
 int build_neighbors(vox_ctx* c);
@@ -561,8 +578,82 @@ __device__ __forceinline__ double wfun_k(double r, int ktype, double re, double 
     }
 }
 
+// sqrt(x) correctly rounded, and h, 1 / (2 sqrt(x)) to a few units in the last
+// place: Goldschmidt's iteration on the hardware's reciprocal square root and
+// two residual corrections (Markstein), the steps of sqrt() without its scaling,
+// so x must be normal and far from the ends of the range; other x (0, a
+// denormal, infinity, NaN) take sqrt() itself and a full division.
+__device__ __forceinline__ double sqrt_h(double x, double& h)
+{
+    // (biased exponent below 93 or above 1953; negative x and NaN as well)
+    if (__builtin_expect((uint32_t)__double2hiint(x) - 0x05d00000u > 0x74400000u, 0)) {
+        const double s = sqrt(x);
+        h = 0.5 / s;
+        return s;
+    }
+    const double y = __builtin_amdgcn_rsq(x);
+    double s = x * y;
+    h = 0.5 * y;
+    const double r = fma(-h, s, 0.5);
+    s = fma(s, r, s);
+    h = fma(h, r, h);
+    s = fma(fma(-s, s, x), h, s);
+    return fma(fma(-s, s, x), h, s);
+}
+
+// 1 / q correctly rounded from an approximation y good to a few units in the
+// last place: a Newton step brings y within one unit, the second rounds
+// correctly (Markstein) unless q's significand is all ones, where the quotient
+// lies next to a tie: those q (1 - 2^-53 occurs on lattices) take the division.
+__device__ __forceinline__ double recip_from(double q, double y)
+{
+    y = fma(fma(-q, y, 1.0), y, y);
+    y = fma(fma(-q, y, 1.0), y, y);
+    const uint32_t lo = (uint32_t)__double2loint(q), hi = (uint32_t)__double2hiint(q);
+    if (__builtin_expect((lo & (hi | 0xfff00000u)) == 0xffffffffu, 0)) y = 1.0 / q;
+    return y;
+}
+
+// The weight W(r) of a distance r = sqrt_h(r^2, h): wfun_k with the
+// reciprocal of q = r / re taken from h instead of a division (the same bits).
+template <int KT>
+__device__ __forceinline__ double wfun_h(double r, double h, int ktype, double re, double inv_re)
+{
+    if constexpr (KT == 2) {
+        const double q = div_by(r, re, inv_re);
+        return (q < 1.0) ? recip_from(q, (2.0 * re) * h) - 1 : 0.0;
+    } else {
+        return wfun_k<KT>(r, ktype, re, inv_re);
+    }
+}
+
+// s + v_0 + v_1 + ... + v_15 over the lanes of a row of 16, added in lane
+// order (every lane of the row holds the same s and gets the same sum). One
+// instruction a term: v_j * 1 + s rounds as the sum does, and the multiply-add
+// takes lane j's value by DPP. The leading s_nop covers the wait states
+// between the write of v and a DPP read of it.
+__device__ __forceinline__ double row16_add(double s, double v)
+{
+    const double one = 1.0;
+#define VOX_ADD16(j) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #j " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t"
+        VOX_ADD16(0) VOX_ADD16(1) VOX_ADD16(2) VOX_ADD16(3)
+        VOX_ADD16(4) VOX_ADD16(5) VOX_ADD16(6) VOX_ADD16(7)
+        VOX_ADD16(8) VOX_ADD16(9) VOX_ADD16(10) VOX_ADD16(11)
+        VOX_ADD16(12) VOX_ADD16(13) VOX_ADD16(14) VOX_ADD16(15)
+        : "+v"(s) : "v"(v), "v"(one));
+#undef VOX_ADD16
+    return s;
+}
+
 // The compile-time kernel type of a run (0: any other, read at run time).
 inline int kt_of(int ktype) { return (ktype == 2 || ktype == 6) ? ktype : 0; }
+
+// This block's copy of a spread counter.
+__device__ __forceinline__ int32_t* spread_at(int32_t* spread, int slot)
+{
+    return spread + (blockIdx.x & (kSpread - 1)) * kSpreadLine + slot;
+}
 
 // Fixed-order block sum of one double per thread (blockDim == kBlock).
 __device__ __forceinline__ double block_sum(double v, double* lds)

@@ -359,8 +359,8 @@ __device__ __forceinline__ void flush_ids(const int32_t* ring, int c, int cap,
 // that hit the same lines.
 __global__ __launch_bounds__(kBlock) void k_build_list(
     Grid g, int n, double R, const int32_t* __restrict__ start, const PosRec* __restrict__ rec,
-    int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ flags,
-    int flag_overflow, int flag_max, int32_t* __restrict__ blockmax)
+    int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ spread,
+    int slot_max)
 {
     __shared__ int32_t ring_all[kBlock * kIdRing];
     int32_t* ring = ring_all + threadIdx.x * kIdRing;
@@ -416,9 +416,8 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
             }
         if (k & 7) flush_ids(ring, k >> 3, cap, ids + rb);
         cnt[i] = k;
-        if (k > cap) atomicAdd(&flags[flag_overflow], 1);
     }
-    // longest row: wave max -> block max -> one slot per block (no atomics)
+    // longest row: wave max -> block max
     __shared__ int wmax[kBlock / kWave];
     int m = wave_max_i32(k);
     if ((threadIdx.x % kWave) == 0) wmax[threadIdx.x / kWave] = m;
@@ -426,9 +425,8 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
     if (threadIdx.x == 0) {
         int b = wmax[0];
         for (int w = 1; w < kBlock / kWave; ++w) b = max(b, wmax[w]);
-        blockmax[blockIdx.x] = b;
+        atomicMax(spread_at(spread, slot_max), b);
     }
-    (void)flag_max;
 }
 
 // Stencil walk for cells that hold many particles (3D list L: 64-80 a cell),
@@ -493,8 +491,8 @@ __device__ __forceinline__ void mm_flush(const int32_t* ring, int grp, int k, in
 template <bool kPos>
 __global__ __launch_bounds__(kWave, 4) void k_build_list_mm(
     Grid g, int n, double R, const int32_t* __restrict__ start, const PosRec* __restrict__ rec,
-    int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ flags,
-    int flag_overflow, int flag_max)
+    int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ spread,
+    int slot_max)
 {
     __shared__ __align__(16) float comp[4][kWave];      // candidates: x, y, z and 1
     __shared__ __align__(16) float thr[kWave];          // |c|^2 - 1
@@ -706,25 +704,10 @@ __global__ __launch_bounds__(kWave, 4) void k_build_list_mm(
     int kmax = 0;
     if (valid) {
         cnt[kPos ? t : (long)me.id] = k;
-        if (k > cap) atomicAdd(&flags[flag_overflow], 1);
         kmax = k;
     }
     kmax = wave_max_i32(kmax);
-    if (lane == 0) atomicMax(&flags[flag_max], kmax);
-}
-
-__global__ void k_reduce_max(const int32_t* __restrict__ v, int n, int32_t* __restrict__ out)
-{
-    __shared__ int lds[kBlock];
-    int m = 0;
-    for (int k = threadIdx.x; k < n; k += kBlock) m = max(m, (int)v[k]);
-    lds[threadIdx.x] = m;
-    __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) lds[threadIdx.x] = max(lds[threadIdx.x], lds[threadIdx.x + s]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = lds[0];
+    if (lane == 0) atomicMax(spread_at(spread, slot_max), kmax);
 }
 
 // ---- host side --------------------------------------------------------------------------
@@ -741,6 +724,24 @@ int ensure_list_storage(vox_ctx* c, int which, int cap)
 }
 
 static int search_one(vox_ctx* c, int which, double re);
+
+// What a search reports: the domain flags, and the longest rows with the other
+// spread counters.
+__global__ void k_clear_search(int32_t* __restrict__ flags, int32_t* __restrict__ spread)
+{
+    for (int k = threadIdx.x; k < kSpread * kSpreadLine; k += blockDim.x) spread[k] = 0;
+    if (threadIdx.x == 0) {
+        flags[FLAG_DOMAIN] = 0;
+        flags[FLAG_DOMAIN_FIRST] = 0x7fffffff;
+    }
+}
+
+static int clear_search_status(vox_ctx* c)
+{
+    k_clear_search<<<1, kSpread * kSpreadLine, 0, c->stream>>>(c->dflags, c->dspread);
+    VOX_HIP(hipGetLastError());
+    return VOX_OK;
+}
 
 // List L in 3D can hold compact rows: the reference accepts d <= re + DELTA
 // with the particle itself (functions.cu:2886), but its consumers, PREDICTION
@@ -838,8 +839,7 @@ static int search_one(vox_ctx* c, int which, double re)
 {
     DevList& L = c->list[which];
     const int n = c->tp;
-    const int fo = which == 0 ? FLAG_OVERFLOW_S : FLAG_OVERFLOW_L;
-    const int fm = which == 0 ? FLAG_MAXCNT_S : FLAG_MAXCNT_L;
+    const int sm = which == 0 ? SPR_MAXCNT_S : SPR_MAXCNT_L;
     // compact rows (list L): d < re, the particle itself excluded
     const bool compact = (which == 1) && list_compact_ok(c);
     Grid gg = L.g;
@@ -859,25 +859,21 @@ static int search_one(vox_ctx* c, int which, double re)
     const int mode = c->tuned_mode[which] ? c->tuned_mode[which] : c->p.list_mode;
     const bool cell_walk = (mode == 2 || (mode == 0 && per_cell >= 24.0));
     ProfScope ps(c, which == 0 ? KC_LIST : KC_LIST_L);
-    VOX_TRY(fill_i32(c, c->dflags + fo, 0, 1));
     // Compact rows of the cell walk hold positions in the cell-sorted records
     // (and sit at the particle's position): their consumers gather from
     // records in that order, where a row's consecutive entries (one cell's
     // particles) sit side by side.
     L.pos_rows = compact && cell_walk;
     if (cell_walk) {
-        VOX_TRY(fill_i32(c, c->dflags + fm, 0, 1));
         if (L.pos_rows)
             k_build_list_mm<true><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
-                gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
+                gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
         else
             k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
-                gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
+                gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
     } else {
-        const int nb = grid_for(n);
-        k_build_list<<<nb, kBlock, 0, c->stream>>>(gg, n, R, L.cell_start, L.rec, L.cap, L.ids,
-                                                    L.cnt, c->dflags, fo, fm, c->blockmax);
-        k_reduce_max<<<1, kBlock, 0, c->stream>>>(c->blockmax, nb, c->dflags + fm);
+        k_build_list<<<grid_for(n), kBlock, 0, c->stream>>>(gg, n, R, L.cell_start, L.rec, L.cap,
+                                                            L.ids, L.cnt, c->dspread, sm);
     }
     VOX_HIP(hipGetLastError());
     return VOX_OK;
@@ -907,12 +903,11 @@ static int domain_error(vox_ctx* c)
 // with wider rows (up to 3 more passes).
 static int regrow_one(vox_ctx* c, int which, double re)
 {
-    const int fo = which == 0 ? FLAG_OVERFLOW_S : FLAG_OVERFLOW_L;
-    const int fm = which == 0 ? FLAG_MAXCNT_S : FLAG_MAXCNT_L;
     for (int attempt = 0; attempt < 4; ++attempt) {
-        if (c->hflags[fo] == 0) return VOX_OK;
+        const int need = spread_max(c, which == 0 ? SPR_MAXCNT_S : SPR_MAXCNT_L);
+        c->max_count[which] = need;
+        if (need <= c->list[which].cap) return VOX_OK;
         if (attempt == 3) break;
-        int need = c->hflags[fm];
         int cap = ((need + need / 4) + 7) & ~7;
         VOX_TRY(ensure_list_storage(c, which, cap));
         VOX_TRY(search_one(c, which, re));
@@ -929,23 +924,21 @@ int ensure_reference_list(vox_ctx* c, int which)
 {
     DevList& L = c->list[which];
     if (!L.compact) return VOX_OK;
-    const int fo = which == 0 ? FLAG_OVERFLOW_S : FLAG_OVERFLOW_L;
-    const int fm = which == 0 ? FLAG_MAXCNT_S : FLAG_MAXCNT_L;
+    const int sm = which == 0 ? SPR_MAXCNT_S : SPR_MAXCNT_L;
     const double R = L.g.incl ? L.re + c->p.delta : L.re;
     const int n = c->tp;
     for (int attempt = 0; attempt < 4; ++attempt) {
-        VOX_TRY(fill_i32(c, c->dflags + fo, 0, 1));
-        VOX_TRY(fill_i32(c, c->dflags + fm, 0, 1));
+        VOX_TRY(fill_i32(c, c->dspread, 0, kSpread * kSpreadLine));
         k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
-            L.g, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dflags, fo, fm);
+            L.g, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
         VOX_HIP(hipGetLastError());
         L.pos_rows = false;
         VOX_TRY(read_flags(c));
-        if (c->hflags[fo] == 0) {
+        const int need = spread_max(c, sm);
+        if (need <= L.cap) {
             L.compact = false;
             return VOX_OK;
         }
-        const int need = c->hflags[fm];
         VOX_TRY(ensure_list_storage(c, which, ((need + need / 4) + 7) & ~7));
     }
     return fail(VOX_ERR_OVERFLOW, "neighbour row capacity could not be satisfied");
@@ -1011,26 +1004,23 @@ int autotune_lists(vox_ctx* c, int reps, int32_t* modes)
     return rc;
 }
 
-// List L on the side stream: the context's stream, scan scratch and
-// block-maximum slots are swapped for the side ones while its work is queued.
+// List L on the side stream: the context's stream and scan scratch are swapped
+// for the side ones while its work is queued.
 static int launch_side(vox_ctx* c, int which, double re)
 {
     std::swap(c->stream, c->stream2);
     std::swap(c->scan_blocks, c->scan_blocks2);
     std::swap(c->scan_blocks_cap, c->scan_blocks2_cap);
-    std::swap(c->blockmax, c->blockmax2);
     const int rc = launch_one(c, which, re);
     std::swap(c->stream, c->stream2);
     std::swap(c->scan_blocks, c->scan_blocks2);
     std::swap(c->scan_blocks_cap, c->scan_blocks2_cap);
-    std::swap(c->blockmax, c->blockmax2);
     return rc;
 }
 
 int build_neighbors(vox_ctx* c)
 {
-    VOX_TRY(fill_i32(c, c->dflags + FLAG_DOMAIN, 0, 1));
-    VOX_TRY(fill_i32(c, c->dflags + FLAG_DOMAIN_FIRST, 0x7fffffff, 1));
+    VOX_TRY(clear_search_status(c));
     if (c->two_lists && c->stream2) {
         // The two lists are independent: list L is built on a second stream
         // beside list S (the side stream first waits for everything queued so
@@ -1049,8 +1039,8 @@ int build_neighbors(vox_ctx* c)
         VOX_TRY(build_one(c, 0, c->p.re_s));
         if (c->two_lists) VOX_TRY(build_one(c, 1, c->p.re_l));
     }
-    c->st.max_count_s = c->hflags[FLAG_MAXCNT_S];
-    c->st.max_count_l = c->two_lists ? c->hflags[FLAG_MAXCNT_L] : c->hflags[FLAG_MAXCNT_S];
+    c->st.max_count_s = c->max_count[0];
+    c->st.max_count_l = c->max_count[c->two_lists ? 1 : 0];
     return VOX_OK;
 }
 

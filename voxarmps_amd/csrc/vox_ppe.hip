@@ -99,7 +99,7 @@ struct AsmArgs {
     int32_t *acol, *rowlen;                // acol null: the columns are not stored
     v4u* dcol;                             // 16-bit column steps (null: not stored)
     int32_t *cbase, *dbad;                 //   first columns; set when a step does not fit
-    int32_t* creach;                       //   max row - first column, max last column - row
+    int32_t* spread;                       //   max row - first column, max last column - row
     double *aval, *adiag, *rhs, *source;
     float* aval32;                         // FP32 values (mixed precision, learned network)
     PosRec* rec;                           // the records the row entries index
@@ -115,6 +115,12 @@ __global__ void k_pack_asm(AsmArgs a)
 {
     // threads in particle order (fields read in lines), whole records stored
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // what the assembly and the window build report
+    if (i < kSpread) {
+        int32_t* sp = a.spread + i * kSpreadLine;
+        sp[SPR_COL_BELOW] = sp[SPR_COL_ABOVE] = sp[SPR_WIN_N] = sp[SPR_WIN_SUM] = 0;
+        if (i == 0) *a.dbad = 0;
+    }
     if (i >= a.n) return;
     const int t = a.order ? a.pos_of[i] : i;
     PosRec r;
@@ -126,144 +132,182 @@ __global__ void k_pack_asm(AsmArgs a)
     a.source[i] = (bi == 0) ? a.inv_dt_dt * (a.pnd[i] - a.n0s) / a.n0s : 0.0;
 }
 
-// Per-thread ring of the last 16 outputs in LDS (strides of 17 keep the lanes'
-// equal-slot accesses on distinct banks).
-constexpr int kRing = 17;
-
-// One thread per unknown row r (particle urow[r]), so a wave is one SELL-64
-// slice: its lanes produce their rows' entries 8 at a time into LDS, and once
-// every lane holds its group g (or has run out of row), the wave stores entry
-// 8g + u of its 64 rows as one contiguous block for u = 0..7. Rows are written
-// in their final layout in one pass. Entries are processed strictly in list
-// order (the reference's), so the values and the diagonal are bit-identical
-// to the sequential MATRIX.
+// One block per 16 unknown rows (row r is particle urow[r]). Four waves evaluate,
+// 16 lanes per row: each lane takes one of the row's next 16 list entries and
+// the kept ones go to the row's slots of a ring in LDS in list order (their rank
+// among the row's lanes). Once every row holds its group g of 16 entries (or has
+// run out of list) a fifth wave stores it: entry k of the 16 rows is one
+// 128-byte line. The diagonal adds the lanes' terms in lane order, the list's:
+// values and diagonal are bit-identical to the sequential MATRIX.
+// Why: one thread per row (8 records in flight, 3 waves per SIMD) was bound by the
+// latency of its gathers. Consecutive entries of a row are mostly neighbouring
+// records, so 16 lanes per row touch half the lines, 24 evaluating waves per CU
+// hide the latency, and a system of few rows still fills the chip. The wave
+// that stores does not evaluate: loads and stores share one in-order counter, so
+// a wave that waits for its next record would wait for its stores too.
+// Measured, one thread per row -> this, us: 820,000 rows of 240 entries 1567 ->
+// 1299, 282,000 rows 698 -> 472, 105,000 rows 435 -> 172; 2D rows of 45 entries,
+// FP32 values: 866,000 rows 417 -> 383, 1,250 rows (FP64) 35 -> 8. At 820,000 rows
+// 16 lanes that store their entries themselves (32-byte pieces of lines) took
+// 1545 us, 0.6 of it the stores; 32-row blocks that store between evaluations
+// 1480; four lanes per row with a ring per wave 1455.
 // SV = double: FP64 values (and their FP32 copy when aval32 is set, for the
 // learned preconditioner's network); SV = float: mixed precision, FP32 values
 // only (computed in FP64 and rounded once; the diagonal stays FP64).
+constexpr int kAsmLanes = 16;                       // lanes per row
+constexpr int kAsmRows = 16;                        // rows per block
+constexpr int kAsmEval = kAsmRows * kAsmLanes;      // evaluating threads
+constexpr int kAsmThreads = kAsmEval + kWave;
+constexpr int kAsmRing = 64;                        // slots: a group being stored, the next
+                                                    // one and what the one after gets early
+constexpr int kAsmStride = 20;                      // rows of a slot: 16 slots x 4 rows on
+                                                    // distinct banks
 template <class SV, int KT>
-__global__ __launch_bounds__(kBlock) void k_assemble_rows(AsmArgs a)
+__global__ __launch_bounds__(kAsmThreads, 8) void k_assemble_rows(AsmArgs a)
 {
-    __shared__ int32_t ring_c[kBlock * kRing];
-    __shared__ double ring_v[kBlock * kRing];
+    __shared__ double ring_v[kAsmRing * kAsmStride];
+    __shared__ int32_t ring_c[kAsmRing * kAsmStride];
+    __shared__ int32_t krow[kAsmRows];              // entries each row holds
     const int nu = *a.nu;
-    if ((long)blockIdx.x * blockDim.x >= nu) return;          // uniform over the block
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = r < nu;
-    const int i = live ? a.urow[r] : 0;
-    const int self = a.pos_of ? a.pos_of[i] : i;   // own index among the entries' records
-    int32_t* rc = ring_c + threadIdx.x * kRing;
-    double* rv = ring_v + threadIdx.x * kRing;
-    // rows of positions sit at the particle's position
-    const int32_t* __restrict__ row = a.L.ids + sl_index(self, 0, a.L.cap);
-    const PosRec me = a.rec[self];
-    const double xi = me.x, yi = me.y, zi = me.z;
-    const long ob = mx_index(r, 0, a.acap);                  // entry k at ob + 64 k
-    double diag = 0.0;
-    int k = 0, l0 = 0;
-    int first = 0, last = 0;                                  // column steps
-    bool bad = false;
-    const int cnt = live ? a.L.cnt[self] : 0;
-    constexpr int U = 8;
-    // the next chunk's ids are loaded while the current chunk's records are
-    // gathered and used
-    int32_t jn[U];
-    if (cnt > 0) load_chunk8(row, 0, jn);
-    for (int g = 0;; ++g) {
-        // this lane's rows until group g is complete or the row is done; a
-        // list chunk adds at most 8 entries, so the ring never holds more
-        // than groups g and g + 1
-        while (k < 8 * (g + 1) && l0 < cnt) {
-            int jj[U];
-            PosRec rr[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) jj[u] = jn[u];
-            if (l0 + U < cnt) load_chunk8(row, (l0 >> 3) + 1, jn);
-#pragma unroll
-            for (int u = 0; u < U; ++u) jj[u] = (l0 + u < cnt) ? jj[u] : self;
-#pragma unroll
-            for (int u = 0; u < U; ++u) rr[u] = a.rec[jj[u]];
-            // Branch-free per entry (a skipped entry keeps diag unchanged
-            // through a select), so no record load is sunk into a branch
-            // behind a full wait.
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const PosRec rj = rr[u];
-                const int bj = rj.id;
+    if ((long)blockIdx.x * kAsmRows >= nu) return;            // uniform over the block
+    const int lane = threadIdx.x & (kWave - 1);
+    if (threadIdx.x < kAsmEval) {
+        const int sub = threadIdx.x & (kAsmLanes - 1), lr = threadIdx.x / kAsmLanes;
+        const int r = blockIdx.x * kAsmRows + lr;
+        const bool live = r < nu;
+        const int i = live ? a.urow[r] : 0;
+        const int self = a.pos_of ? a.pos_of[i] : i;   // own index among the entries' records
+        // rows of positions sit at the particle's position; 16 entries on, a
+        // lane's entry is two chunks (1024 elements) away
+        const int32_t* __restrict__ row = a.L.ids + sl_index(self, 0, a.L.cap) + sl_step(sub);
+        const PosRec me = a.rec[self];
+        const unsigned long long seg = 0xffffull << (lane & 48);      // the row's lanes
+        const unsigned long long below = seg & ((1ull << lane) - 1ull);
+        double diag = 0.0;
+        int k = 0, left = (live ? a.L.cnt[self] : 0) - sub;   // entries from this lane's on
+        // the next entry's record and the id of the one after
+        int jn = (left > 0) ? *row : self;
+        PosRec rn = a.rec[jn];
+        row += 1024;
+        int jnn = (left > kAsmLanes) ? *row : self;
+        for (int g = 0;; ++g) {
+            while (k < 16 * (g + 1) && left + sub > 0) {
+                const int j = jn;
+                const PosRec rj = rn;
+                jn = jnn;
+                rn = a.rec[jn];
+                left -= kAsmLanes;
+                row += 1024;
+                jnn = (left > kAsmLanes) ? *row : self;
                 // z is 0 in 2D records, and adding 0*0 leaves the 2D sum
                 // unchanged, so one expression serves both dimensions
-                const double dx = rj.x - xi, dy = rj.y - yi, dz = rj.z - zi;
-                const double d = sqrt(dx * dx + dy * dy + dz * dz);
-                // jj == self: the particle itself, or padding past the row end
-                const bool use = (jj[u] != self) && (bj != -1) && !(fabs(d) <= 1.0e-15);
+                const double dx = rj.x - me.x, dy = rj.y - me.y, dz = rj.z - me.z;
+                double h;
+                const double d = sqrt_h(dx * dx + dy * dy + dz * dz, h);
+                const int bj = rj.id;
+                // j == self: the particle itself, or padding past the row end
+                const bool use = (j != self) && (bj != -1) && !(fabs(d) <= 1.0e-15);
                 // (= c0 * W(d) / n0l / rho1 with IEEE divisions, see div_by);
                 // matopt: hl / d^3 / n0l / rho1 (functions.cu:903-913)
-                const double val = a.matopt
-                    ? div_by(div_by(a.hl / (d * d * d), a.n0l, a.inv_n0l), a.rho1, a.inv_rho1)
-                    : div_by(div_by(a.c0 * wfun_k<KT>(d, a.ktype, a.re, a.inv_re), a.n0l, a.inv_n0l),
-                             a.rho1, a.inv_rho1);
-                if (use && bj == 0 && val != 0.0) {
-                    rc[k & 15] = rj.aux;
-                    rv[k & 15] = -val;
-                    ++k;
+                double val = a.matopt ? a.hl / (d * d * d)
+                                      : a.c0 * wfun_h<KT>(d, h, a.ktype, a.re, a.inv_re);
+                val = div_by(div_by(val, a.n0l, a.inv_n0l), a.rho1, a.inv_rho1);
+                const bool keep = use && bj == 0 && val != 0.0;
+                const unsigned long long kept = __ballot(keep);
+                if (keep) {
+                    const int s = ((k + __popcll(kept & below)) & (kAsmRing - 1)) * kAsmStride + lr;
+                    ring_c[s] = rj.aux;
+                    ring_v[s] = -val;
                 }
-                diag = use ? diag + val : diag;
+                k += __popcll(kept & seg);
+                diag = row16_add(diag, use ? val : 0.0);      // + 0 leaves its bits
             }
-            l0 += U;
+            if (sub == 0) krow[lr] = k;
+            __syncthreads();
+            // (a wave that is a group ahead may have raised krow meanwhile:
+            // only of rows that hold more than group g anyway)
+            if (!__any(krow[lane & (kAsmRows - 1)] > 16 * g)) break;
         }
-        const bool has = k > 8 * g;
-        if (!__any(has)) break;                                // every row is written
-        if (has) {
-            const int s0 = (g & 1) * 8;
-            // the group's columns also as steps from the previous column
-            // (entry 0 from itself: its column is the row's base); steps past
-            // the row's end are 0
-            int prev = (g == 0) ? rc[s0] : last;
-            if (g == 0) first = prev;
+        if (live && sub == 0) {
+            a.adiag[r] = diag + a.dshift;
+            a.rowlen[r] = k;
+            a.rhs[r] = a.source[i];
+        }
+        return;
+    }
+    const int srow = lane & (kAsmRows - 1), part = lane / kAsmRows;
+    const int sr = blockIdx.x * kAsmRows + srow;
+    const long ob = mx_index(sr, 0, a.acap);                  // entry k at ob + 64 k
+    bool bad = false;
+    int first = 0, last = 0;                                  // columns of the row's first and
+                                                              // last entry so far (parts 0, 1)
+    for (int g = 0;; ++g) {
+        __syncthreads();
+        const int have = krow[srow];
+        if (!__any(have > 16 * g)) break;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int kk = 16 * g + 4 * u + part;
+            const int s = (kk & (kAsmRing - 1)) * kAsmStride + srow;
+            const double v = ring_v[s];
+            const long o = ob + 64L * kk;
+            if (kk < have) {
+                if constexpr (sizeof(SV) == 8) {
+                    a.aval[o] = v;
+                    if (a.aval32) a.aval32[o] = (float)v;
+                } else {
+                    a.aval32[o] = (float)v;
+                }
+                if (a.acol) a.acol[o] = ring_c[s];
+            }
+        }
+        if (a.dcol) {
+            // the group's columns as steps from the previous column (entry 0
+            // from itself: its column is the row's base), a chunk of 8 for
+            // each of lane parts 0 and 1
+            const int half = part & 1, e0 = 16 * g + 8 * half;
+            int32_t cu[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                cu[u] = ring_c[((e0 + u) & (kAsmRing - 1)) * kAsmStride + srow];
+            // the column before the chunk: the previous group's last for the
+            // first half, entry e0 - 1 for the second
+            const int mid = __shfl(cu[7], srow), tail = __shfl(last, srow + kAsmRows);
+            int prev = half ? mid : (g == 0 ? cu[0] : tail);
+            if (g == 0) first = cu[0];
             uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int kk = 8 * g + u;
-                if (kk < k) {
-                    const long o = ob + 64L * kk;
-                    const int cu = rc[s0 + u];
-                    if (a.acol) a.acol[o] = cu;
-                    const int d = cu - prev;
+                if (e0 + u < have) {
+                    const int d = cu[u] - prev;
                     bad = bad || d < 0 || d > 0xffff;
                     w[u >> 1] |= (uint32_t)(d & 0xffff) << (16 * (u & 1));
-                    prev = cu;
-                    if constexpr (sizeof(SV) == 8) {
-                        a.aval[o] = rv[s0 + u];
-                        if (a.aval32) a.aval32[o] = (float)rv[s0 + u];
-                    } else {
-                        a.aval32[o] = (float)rv[s0 + u];
-                    }
+                    prev = cu[u];
                 }
             }
-            last = prev;
-            if (a.dcol) a.dcol[dc_index(r, g, a.acap)] = v4u{w[0], w[1], w[2], w[3]};
+            if (e0 < have) {
+                last = prev;
+                if (part < 2) {
+                    if (e0 == 0) a.cbase[sr] = first;
+                    a.dcol[dc_index(sr, 2 * g + half, a.acap)] = v4u{w[0], w[1], w[2], w[3]};
+                }
+            }
         }
     }
-    if (a.dcol) {
-        // how far the rows' columns reach below and above the row (every lane
-        // of the wave is here: the loop above ends for all of them together)
-        int below = (live && k > 0) ? r - first : 0;
-        int above = (live && k > 0) ? last - r : 0;
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-            below = max(below, __shfl_xor(below, o));
-            above = max(above, __shfl_xor(above, o));
-        }
-        if ((threadIdx.x & (kWave - 1)) == 0) {
-            atomicMax(&a.creach[0], below);
-            atomicMax(&a.creach[1], above);
-        }
+    if (!a.dcol) return;
+    if (__any(bad) && lane == 0) atomicOr(a.dbad, 1);
+    // how far the rows' columns reach below and above the row (a row's last
+    // column is the larger of its halves': columns ascend where steps fit)
+    const int have = krow[srow];
+    int under = (have > 0 && !(part & 1)) ? sr - first : 0;
+    int over = (have > 8 * (part & 1)) ? last - sr : 0;
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        under = max(under, __shfl_xor(under, o));
+        over = max(over, __shfl_xor(over, o));
     }
-    if (!live) return;
-    a.adiag[r] = diag + a.dshift;
-    a.rowlen[r] = k;
-    a.rhs[r] = a.source[i];
-    if (a.dcol) {
-        a.cbase[r] = first;
-        if (bad) atomicOr(a.dbad, 1);
+    if (lane == 0) {
+        atomicMax(spread_at(a.spread, SPR_COL_BELOW), under);
+        atomicMax(spread_at(a.spread, SPR_COL_ABOVE), over);
     }
 }
 
@@ -385,14 +429,14 @@ __global__ void k_rhs_from_source(int nu, const int32_t* __restrict__ urow, cons
 
 static void launch_assemble_rows(vox_ctx* c, const AsmArgs& a, bool fp32_only)
 {
-    const int n = c->tp;
+    const int nb = grid_for(c->tp, kAsmRows);
     switch (kt_of(c->p.ktype) * 2 + (fp32_only ? 1 : 0)) {
-    case 4: k_assemble_rows<double, 2><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
-    case 5: k_assemble_rows<float, 2><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
-    case 12: k_assemble_rows<double, 6><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
-    case 13: k_assemble_rows<float, 6><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
-    case 1: k_assemble_rows<float, 0><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
-    default: k_assemble_rows<double, 0><<<grid_for(n), kBlock, 0, c->stream>>>(a); break;
+    case 4: k_assemble_rows<double, 2><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
+    case 5: k_assemble_rows<float, 2><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
+    case 12: k_assemble_rows<double, 6><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
+    case 13: k_assemble_rows<float, 6><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
+    case 1: k_assemble_rows<float, 0><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
+    default: k_assemble_rows<double, 0><<<nb, kAsmThreads, 0, c->stream>>>(a); break;
     }
 }
 
@@ -452,9 +496,7 @@ int ppe_assemble(vox_ctx* c)
     if (!c->dcol) VOX_HIP(hipMalloc(&c->dcol, sizeof(uint16_t) * (size_t)sl_size(n, c->a_cap)));
     if (!c->cbase) VOX_HIP(hipMalloc(&c->cbase, sizeof(int32_t) * (size_t)n));
     a.dcol = reinterpret_cast<v4u*>(c->dcol); a.cbase = c->cbase; a.dbad = c->dflags + FLAG_DCOL_BAD;
-    a.creach = c->dflags + FLAG_COL_BELOW;
-    VOX_TRY(fill_i32(c, a.dbad, 0, 1));
-    VOX_TRY(fill_i32(c, a.creach, 0, 2));
+    a.spread = c->dspread;
     a.aval32 = mixed ? c->aval32 : nullptr;
     a.adiag = c->adiag; a.rhs = c->rhs;
     a.source = c->f[VOX_F_SOURCE];
@@ -464,6 +506,7 @@ int ppe_assemble(vox_ctx* c)
     // the search: list_l_for_consumer)
     a.order = L.pos_rows ? L.rec : nullptr;
     a.pos_of = L.pos_rows ? L.pos_of : nullptr;
+    static_assert(kBlock >= kSpread, "one block clears the counters");
     k_pack_asm<<<grid_for(n), kBlock, 0, c->stream>>>(a);
     // rows: a grid for every particle, of which the blocks past nu (read on
     // the device) return at once
@@ -482,8 +525,8 @@ int ppe_assemble(vox_ctx* c)
         VOX_HIP(hipGetLastError());
         c->acol_ok = true;
     }
-    c->col_below = c->hflags[FLAG_COL_BELOW];
-    c->col_above = c->hflags[FLAG_COL_ABOVE];
+    c->col_below = spread_max(c, SPR_COL_BELOW);
+    c->col_above = spread_max(c, SPR_COL_ABOVE);
     c->asm_count += 1;
     c->aval32_ok = mixed;
     c->aval64_ok = !fp32_only;
