@@ -285,8 +285,8 @@ int vox_set_regions(vox_ctx* ctx, int nregion, const int32_t* region, const doub
  * list (modes[2] receives the choice for lists S and L); then runs the step's
  * stages up to MATRIX once and times the predictor's variants (FP64: records
  * gathered per group 4, 8 or 2 with 256 threads per block, 4 or 8 with 128;
- * variants 5-8: 8 or 4 records with 128 or 256 threads and the gradient terms
- * deferred to a queue)
+ * variants 5-7: 8 records with 128 or 256 threads, 4 with 128, and the gradient
+ * terms deferred to a queue; 8: 16 lanes per particle)
  * and the PPE product's (0: 8 entries per load batch with p gathered from a
  * per-block LDS window of the block's distinct columns; 1, 2, 3: 4, 16 and 8
  * entries on the 32-bit columns; 4: 8 entries on 16-bit column steps; 0 and 4

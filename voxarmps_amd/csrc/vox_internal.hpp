@@ -18,7 +18,8 @@ constexpr int kBlock = 256;          // threads per workgroup (4 waves)
 constexpr int kWave = 64;            // CDNA wavefront width
 constexpr int kMaxPartials = 8192;   // reduction partial slots per scalar
 constexpr int kPartialSlots = 10;    // scalars reduced through ctx->partials
-constexpr int kPredVariants = 9;     // predictor: records per group x block size x deferred gradient
+constexpr int kPredVariants = 9;     // predictor: records per group x block size x deferred
+                                     // gradient, and 16 lanes per particle
 constexpr int kSpmvVariants = 5;     // PPE product: 8 entries per batch gathered from an LDS
                                      // window; 4, 16, 8 on 32-bit columns; 8 on 16-bit steps
 constexpr int kWinMax = 7936;        // distinct columns of a 256-row PPE chunk in the window
@@ -245,8 +246,8 @@ struct vox_ctx {
     vox::DevList list[2];
     int max_count[2] = {0, 0};     // longest row of each list's last search
     int tuned_mode[2] = {0, 0};    // neighbour walk chosen by the autotuner (0: none)
-    int tune_pred = 6;             // predictor variant (vox::kPredVariants): 8 records,
-                                   // 256 threads, gradient deferred unless tuned
+    int tune_pred = 8;             // predictor variant (vox::kPredVariants): 16 lanes per
+                                   // particle unless tuned
     int tune_spmv = 0;             // PPE product variant (vox::kSpmvVariants)
     bool two_lists = false;
     double n0s = 0.0, n0l = 0.0;
@@ -644,6 +645,13 @@ __device__ __forceinline__ double row16_add(double s, double v)
         : "+v"(s) : "v"(v), "v"(one));
 #undef VOX_ADD16
     return s;
+}
+
+// The wave's largest of a value that is the same in each row of 16 lanes.
+__device__ __forceinline__ int row16_max(int v)
+{
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
 // The compile-time kernel type of a run (0: any other, read at run time).

@@ -705,6 +705,165 @@ __global__ __launch_bounds__(BS) void k_prediction_dg(PredArgs a)
     }
 }
 
+// The predictor with 16 lanes per particle, four particles per wave: a lane
+// evaluates one of the row's next 16 entries and each sum adds the lanes' terms
+// in lane order (row16_add), which is the list's; the entries within re_s go to
+// the row's queue in LDS in list order and their gradient terms are added 16 at
+// a time when it fills and at the end. The same bits as the walks above.
+// Why: one thread per particle (188 VGPRs, 2 waves per SIMD) waits for its
+// gathers; the lanes of a row gather records that lie side by side, and a
+// small system still fills the chip. The ordered sums cost 16 multiply-adds
+// each; those weighted with the eddy viscosity are left out where every
+// particle of the wave has none.
+// Measured against the walk of variant 6: 820k rows of 122 entries 1544 us
+// (1690), 103k rows 233 us (324), 2D two-phase of 12k particles 20 us (41), 2D
+// of 3k 6.4 us (31). Bound by the FP64 instructions (73 % of the cycles) and
+// the L1 lookups of the gathers (83 %); records brought to LDS four lanes a
+// record need a third of those lookups and were slower (1690 us, 267 us), and
+// 96 registers for a fifth wave spill (3566 us).
+constexpr int kPredSlots = 80;                     // queued entries of a row
+constexpr int kPredStride = kBlock / 16 + 4;       // rows of a slot, padded
+
+template <bool kUniform, int KT>
+__global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
+{
+    __shared__ int32_t queue[kPredSlots * kPredStride];
+    const int lane = threadIdx.x & (kWave - 1), sub = threadIdx.x & 15, lr = threadIdx.x >> 4;
+    const int t = xcd_block() * (kBlock / 16) + lr;
+    const bool live = t < a.n;
+    const int i = live ? sorted_particle(a.order, t) : 0;
+    const int self = !live ? 0 : a.pos ? t : i;
+    const int32_t* __restrict__ rpt = a.pos ? a.rpt : a.pt;
+    const int dim = a.dim;
+    const int ti = a.pt[i];
+    const bool fluid = live && ti > 0;
+    if (live && !fluid && sub == 0) {
+        a.xs[i] = a.x[i]; a.ys[i] = a.y[i]; a.us[i] = a.u[i]; a.vs[i] = a.v[i];
+        if (dim == 3) { a.zs[i] = a.z[i]; a.ws[i] = a.w[i]; }
+    }
+    if (!__any(fluid)) return;
+    const PredRec me = a.rec[self];
+    const double xi = me.x, yi = me.y, zi = me.z, ui = me.u, vi = me.v, wi = me.w;
+    const double mi = me.meu, phi_ = a.ph[i], nt = a.neut[i];
+    const double rhoN = (ti == 1) ? a.rho1 : a.rho2;
+    const double inv_rhoN = 1.0 / rhoN;
+    const double inv_re_s = 1.0 / a.re_s, inv_re_l = 1.0 / a.re_l;
+    const bool eddy = __any(fluid && nt != 0.0);
+    double s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0, s6 = 0, s7 = 0, s8 = 0, s9 = 0;
+    const unsigned long long seg = 0xffffull << (lane & 48);
+    const unsigned long long below = seg & ((1ull << lane) - 1ull);
+    int32_t* const gq = queue + lr;
+    int nq = 0;
+    // adds the queued gradient terms of up to `most` entries a row
+    auto drain = [&](int most) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int q = sub; q < most + sub; q += 16) {
+            double g1 = 0.0, g2 = 0.0, g3 = 0.0;
+            if (q < nq) {
+                const PredRec* rj = a.rec + gq[q * kPredStride];
+                const double dx = rj->x - xi, dy = rj->y - yi, dz = rj->z - zi;
+                double h;
+                const double D = sqrt_h(dx * dx + dy * dy + dz * dz, h);
+                const double dp = rj->pn - phi_;
+                const double inv_D = 1.0 / D;
+                const double wg = wfun_h<KT>(D, h, a.ktype, a.re_s, inv_re_s);
+                g1 = div_by(div_by(dp * dx * wg, D, inv_D), D, inv_D);
+                g2 = div_by(div_by(dp * dy * wg, D, inv_D), D, inv_D);
+                g3 = div_by(div_by(dp * dz * wg, D, inv_D), D, inv_D);
+            }
+            s1 = row16_add(s1, g1);
+            s2 = row16_add(s2, g2);
+            if (dim == 3) s3 = row16_add(s3, g3);
+        }
+        nq = 0;
+        __builtin_amdgcn_wave_barrier();
+    };
+    // rows of positions sit at positions; 16 entries on, a lane's entry is two
+    // chunks (1024 elements) away
+    const int32_t* __restrict__ row = a.L.ids + sl_index(self, 0, a.L.cap) + sl_step(sub);
+    const int cnt = fluid ? a.L.cnt[self] : 0;
+    const int most = row16_max(cnt);
+    int left = cnt - sub;                              // entries from this lane's on
+    struct Entry { double x, y, z, u, v, w, meu; };
+    auto load = [&](int j) {
+        const PredRec* r = a.rec + j;
+        return Entry{r->x, r->y, r->z, r->u, r->v, r->w, kUniform ? 0.0 : r->meu};
+    };
+    auto next_id = [&](int ahead) {
+        const int j = (left > ahead) ? row[(ahead >> 4) * 1024] : self;
+        return j;
+    };
+    auto step = [&](int j, const Entry& rj) {
+        // z, w are 0 in 2D records: the 3-term distance equals the 2D one
+        // bit for bit
+        const double dx = rj.x - xi, dy = rj.y - yi, dz = rj.z - zi;
+        double h;
+        const double D = sqrt_h(dx * dx + dy * dy + dz * dz, h);
+        const bool use = (j != self) && (D > 0);
+        const double NEU = (kUniform || ti == rpt[j])
+                               ? div_by(mi, rhoN, inv_rhoN)
+                               : div_by(2 * mi * rj.meu / (mi + rj.meu), rhoN, inv_rhoN);
+        // W(D; re_s) is 0 beyond re_s (every kernel type), where the
+        // gradient terms are +-0 and leave the sums' bits unchanged
+        const bool close = use && D <= a.re_s;
+        const unsigned long long kept = __ballot(close);
+        if (close) gq[(nq + __popcll(kept & below)) * kPredStride] = j;
+        nq += __popcll(kept & seg);
+        // a skipped entry adds +0, which leaves each sum's bits unchanged (a
+        // sum that starts at +0 is never -0)
+        const double wl = wfun_h<KT>(D, h, a.ktype, a.re_l, inv_re_l);
+        const double tu = wl * (rj.u - ui), tv = wl * (rj.v - vi), tw = wl * (rj.w - wi);
+        s4 = row16_add(s4, use ? tu * NEU : 0.0);
+        s5 = row16_add(s5, use ? tv * NEU : 0.0);
+        if (dim == 3) s6 = row16_add(s6, use ? tw * NEU : 0.0);
+        if (eddy) {
+            s7 = row16_add(s7, use ? tu : 0.0);
+            s8 = row16_add(s8, use ? tv : 0.0);
+            if (dim == 3) s9 = row16_add(s9, use ? tw : 0.0);
+        }
+    };
+    if (most > 0) {
+        // two groups a turn, each group's records on the way during the other
+        int ja = next_id(0), jb = next_id(16);
+        Entry ra = load(ja);
+        for (int g = 0;; g += 32) {
+            const Entry rb = load(jb);
+            const int jc = next_id(32);
+            step(ja, ra);
+            if (g + 16 >= most) break;
+            ra = load(jc);
+            const int jd = next_id(48);
+            step(jb, rb);
+            if (g + 32 >= most) break;
+            ja = jc;
+            jb = jd;
+            left -= 32;
+            row += 2048;
+            const int longest = row16_max(nq);
+            if (longest > kPredSlots - 32) drain(longest);
+        }
+    }
+    drain(row16_max(nq));
+    // lane c of the row finishes component c (with no eddy viscosity its
+    // product is 0 times the other sum: 0, or NaN where that one is not finite)
+    if (!fluid || sub >= dim) return;
+    const double sl = (sub == 0) ? s4 : (sub == 1) ? s5 : s6;
+    const double se = !eddy ? sl : (sub == 0) ? s7 : (sub == 1) ? s8 : s9;
+    const double sg = (sub == 0) ? s1 : (sub == 1) ? s2 : s3;
+    const double v0 = (sub == 0) ? ui : (sub == 1) ? vi : wi;
+    const double x0 = (sub == 0) ? xi : (sub == 1) ? yi : zi;
+    const double gr = (sub == 0) ? a.gx : (sub == 1) ? a.gy : a.gz;
+    const double* const tt = (sub == 0) ? a.t1 : (sub == 1) ? a.t2 : a.t3;
+    double* const os = (sub == 0) ? a.us : (sub == 1) ? a.vs : a.ws;
+    double* const ox = (sub == 0) ? a.xs : (sub == 1) ? a.ys : a.zs;
+    const double gc = a.relax1 * (a.gcoef_num * a.dt / a.n0s / a.rho[i]);
+    const double dt = a.dt;
+    const double vel = v0 + gr * dt + a.lapc * dt * (sl + nt * se) / a.ln0 + dt * tt[i] - gc * sg;
+    os[i] = vel;
+    ox[i] = x0 + dt * vel;
+}
+
 // Every MEU equals nu1 rho1 (Newtonian viscosity and no PTYPE 2 particle:
 // functions.cu:2073-2085) and the harmonic mean 2 m m / (m + m) of that value
 // rounds back to it, so NEU does not depend on the neighbour's type.
@@ -716,19 +875,27 @@ bool uniform_meu(const vox_ctx* c)
     return hm == m;
 }
 
-// Predictor variants for the autotuner: (records per group, block size), the
-// gradient terms in the row walk (0-4) or deferred to a queue (5-8).
-static const int kPredR[kPredVariants] = {4, 8, 2, 4, 8, 8, 8, 4, 4};
+// Predictor variants for the autotuner: one thread per particle with (records
+// per group, block size), the gradient terms in the row walk (0-4) or deferred
+// to a queue (5-7), and 16 lanes per particle (8).
+static const int kPredR[kPredVariants] = {4, 8, 2, 4, 8, 8, 8, 4, 1};
 static const int kPredBS[kPredVariants] = {256, 256, 256, 128, 128, 128, 256, 128, 256};
 
 template <bool kU>
 static void launch_pred_u(const PredArgs& a, int v, int n, hipStream_t s)
 {
+    const int nb = grid_for(16L * n);
     switch (v) {
+    case 8:
+        switch (kt_of(a.ktype)) {
+        case 2: k_prediction_l16<kU, 2><<<nb, kBlock, 0, s>>>(a); break;
+        case 6: k_prediction_l16<kU, 6><<<nb, kBlock, 0, s>>>(a); break;
+        default: k_prediction_l16<kU, 0><<<nb, kBlock, 0, s>>>(a); break;
+        }
+        break;
     case 5: k_prediction_dg<kU, 8, 128><<<grid_for(n, 128), 128, 0, s>>>(a); break;
     case 6: k_prediction_dg<kU, 8, 256><<<grid_for(n, 256), 256, 0, s>>>(a); break;
     case 7: k_prediction_dg<kU, 4, 128><<<grid_for(n, 128), 128, 0, s>>>(a); break;
-    case 8: k_prediction_dg<kU, 4, 256><<<grid_for(n, 256), 256, 0, s>>>(a); break;
     case 1: k_prediction<kU, 8, 256><<<grid_for(n, 256), 256, 0, s>>>(a); break;
     case 2: k_prediction<kU, 2, 256><<<grid_for(n, 256), 256, 0, s>>>(a); break;
     case 3: k_prediction<kU, 4, 128><<<grid_for(n, 128), 128, 0, s>>>(a); break;
@@ -749,10 +916,11 @@ static int launch_prediction(vox_ctx* c, const PredArgs& a, int variant)
 
 const char* pred_variant_name(int v)
 {
-    static char buf[kPredVariants][48];
+    static char buf[kPredVariants][80];
     if (v < 0 || v >= kPredVariants) return "?";
-    std::snprintf(buf[v], sizeof buf[v], "%d records per group, %d threads per block%s", kPredR[v],
-                  kPredBS[v], v >= 5 ? ", gradient deferred" : "");
+    std::snprintf(buf[v], sizeof buf[v], "%s%d records per group, %d threads per block%s",
+                  v == 8 ? "16 lanes per particle, " : "", kPredR[v], kPredBS[v],
+                  v >= 5 ? ", gradient deferred" : "");
     return buf[v];
 }
 
