@@ -464,7 +464,7 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
         (rc = dalloc(&c->cg_x, n)) || (rc = dalloc(&c->cg_r, n)) || (rc = dalloc(&c->cg_p, n)) ||
         (rc = dalloc(&c->cg_q, n)) || (rc = dalloc(&c->cg_x32, n)) || (rc = dalloc(&c->cg_r32, n)) ||
         (rc = dalloc(&c->cg_p32, n)) || (rc = dalloc(&c->cg_q32, n)) || (rc = dalloc(&c->cg_d, n)) ||
-        (rc = dalloc(&c->cg_e, n)))
+        (rc = dalloc(&c->cg_e, n)) || (rc = dalloc(&c->cg_pn, n)) || (rc = dalloc(&c->cg_zj, n)))
         return bail(rc);
     if ((rc = dalloc(&c->coll_cnt, n)) || (rc = dalloc(&c->coll_off, n + 1)) ||
         (rc = dalloc(&c->coll_stamp, n)) || (rc = dalloc(&c->coll_root, n)) || (rc = dalloc(&c->coll_logidx, n)) ||
@@ -503,6 +503,7 @@ int vox_destroy(vox_ctx* c)
     dfree(c->scratch_d); dfree(c->pred_rec); dfree(c->pt_sorted); dfree(c->pos_rec);
     dfree(c->uidx); dfree(c->urow); dfree(c->uflag); dfree(c->uscan); dfree(c->rowlen); dfree(c->acol); dfree(c->dcol); dfree(c->cbase); dfree(c->wcol); dfree(c->wuniq); dfree(c->wn);
     dfree(c->aval); dfree(c->adiag); dfree(c->rhs);
+    dfree(c->cg_pn); dfree(c->cg_zj);
     dfree(c->cg_x); dfree(c->cg_r); dfree(c->cg_p); dfree(c->cg_q); dfree(c->cg_d); dfree(c->cg_e);
     dfree(c->cg_x32); dfree(c->cg_r32); dfree(c->cg_p32); dfree(c->cg_q32); dfree(c->aval32);
     dfree(c->coll_cnt); dfree(c->coll_off); dfree(c->coll_i); dfree(c->coll_j);

@@ -38,7 +38,6 @@
 //      -alpha q); p = z + beta p
 // which stays a conjugate-direction method when M varies between solves or
 // is not exactly symmetric positive definite.
-#include <type_traits>
 
 #include "vox_internal.hpp"
 
@@ -51,23 +50,6 @@ namespace vox {
 constexpr int kVecThreads = 1024;
 constexpr int kVecBlocks = 512;
 
-// Fixed-order sum over a block of NT threads (LDS tree of NT doubles).
-template <int NT>
-__device__ __forceinline__ double block_sum_n(double v, double* lds)
-{
-    const int t = threadIdx.x;
-    lds[t] = v;
-    __syncthreads();
-#pragma unroll
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if (t < s) lds[t] = lds[t] + lds[t + s];
-        __syncthreads();
-    }
-    const double r = lds[0];
-    __syncthreads();
-    return r;
-}
-
 template <int NT>
 __device__ __forceinline__ double sum_partials_n(const double* part, int n, double* lds)
 {
@@ -76,16 +58,47 @@ __device__ __forceinline__ double sum_partials_n(const double* part, int n, doub
     return block_sum_n<NT>(s, lds);
 }
 
+// The same sum (that of NT = kVecThreads) by one wave, the result in every lane;
+// J = 8 for n <= 512, 16 for any n.
+template <int J>
+__device__ __forceinline__ double wave_partials(const double* part, int n)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    double w[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) w[j] = 0.0;
+    for (int base = 0; base < n; base += kVecThreads)
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int k = base + kWave * j + lane;
+            if (k < n) w[j] = w[j] + part[k];
+        }
+#pragma unroll
+    for (int h = J / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int j = 0; j < h; ++j) w[j] = w[j] + w[j + h];
+    const double r = wave_tree(w[0]);
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(r)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(r)));
+}
+
+// and by all of a block's threads: up to 512 partials each wave adds for itself
+__device__ __forceinline__ double vec_partials(const double* part, int n, double* lds)
+{
+    return (n <= 512) ? wave_partials<8>(part, n) : sum_partials_n<kVecThreads>(part, n, lds);
+}
+
 // partial slots (kMaxPartials doubles each)
 enum { P_BB = 0, P_RZ0, P_NNZ, P_PQ, P_RR, P_RZ, P_RES, P_RHS, P_ZQ, P_COUNT };
 // scalar slots
-enum { S_BNORM = 0, S_RZ0, S_RZ1, S_RELRES, S_NNZ, S_RESN, S_RHSN, S_COUNT_ };
+enum { S_BNORM = 0, S_RZ0, S_RZ1, S_RELRES, S_NNZ, S_RESN, S_RHSN, S_PQ, S_COUNT_ };
 static_assert(S_COUNT_ <= SC_COUNT, "scalar slots");
 static_assert(P_COUNT <= kPartialSlots, "partial slots");
 
 template <class VT, class MT>
 struct CgArgs {
-    int nu, cap, maxit, it, npq;   // npq: blocks of the product kernel
+    int nu, cap, maxit, it;
+    int npq, nvb;                  // blocks of the product and of the vector kernels
     double tol;
     const int32_t* __restrict__ rowlen;
     const int32_t* __restrict__ acol;
@@ -101,8 +114,9 @@ struct CgArgs {
     VT* x;
     VT* r;
     VT* p;
+    const VT* pold;                   // the direction before p (see k_cg_spmv_win)
     VT* q;
-    VT* z;                            // flexible CG: z = M r
+    VT* z;                            // flexible CG: z = M r; CG: r / d where p is updated from it
     const int32_t* __restrict__ slen; // coupling operator (SELL-64, cap scap)
     const int32_t* __restrict__ scol;
     const float* __restrict__ sval;
@@ -149,24 +163,45 @@ __global__ __launch_bounds__(kVecThreads) void k_cg_init(CgArgs<VT, MT> a)
     }
 }
 
+// One thread: the scalars and flags a solve starts from.
+template <class VT, class MT>
+__device__ __forceinline__ void cg_start(const CgArgs<VT, MT>& a, double bn, double rz, double nz)
+{
+    a.scal[S_BNORM] = bn;
+    a.scal[S_RZ0] = rz;
+    a.scal[S_NNZ] = nz;
+    a.scal[S_RELRES] = 0.0;
+    a.flags[FLAG_CG_ITERS] = 0;
+    a.flags[FLAG_CG_BREAK] = 0;
+    a.flags[FLAG_CG_CONV] = (bn == 0.0) ? 1 : 0;
+    a.flags[FLAG_CG_DONE] = (bn == 0.0) ? 1 : 0;
+}
+
+// The end of iteration `it`: relative residual from ||r||^2 and, in the lead
+// thread, the flags; whether the solve goes on.
+template <class VT, class MT>
+__device__ __forceinline__ bool cg_goes_on(const CgArgs<VT, MT>& a, double rr, int it, bool lead)
+{
+    const double rel = sqrt(rr) / a.scal[S_BNORM];
+    const bool conv = rel <= a.tol;
+    const bool stop = it >= a.maxit || !isfinite(rel);
+    if (lead) {
+        a.scal[S_RELRES] = rel;
+        a.flags[FLAG_CG_ITERS] = it;
+        if (conv) a.flags[FLAG_CG_CONV] = 1;
+        if (conv || stop) a.flags[FLAG_CG_DONE] = 1;
+    }
+    return !conv && !stop;
+}
+
 template <class VT, class MT>
 __global__ __launch_bounds__(kBlock) void k_cg_init_fin(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kBlock];
-    double bb = sum_partials(PSLOT(a, P_BB), kVecBlocks, lds);
-    double rz = sum_partials(PSLOT(a, P_RZ0), kVecBlocks, lds);
-    double nz = sum_partials(PSLOT(a, P_NNZ), kVecBlocks, lds);
-    if (threadIdx.x == 0) {
-        double bn = sqrt(bb);
-        a.scal[S_BNORM] = bn;
-        a.scal[S_RZ0] = rz;
-        a.scal[S_NNZ] = nz;
-        a.scal[S_RELRES] = 0.0;
-        a.flags[FLAG_CG_ITERS] = 0;
-        a.flags[FLAG_CG_BREAK] = 0;
-        a.flags[FLAG_CG_CONV] = (bn == 0.0) ? 1 : 0;
-        a.flags[FLAG_CG_DONE] = (bn == 0.0) ? 1 : 0;
-    }
+    double bb = sum_partials(PSLOT(a, P_BB), a.nvb, lds);
+    double rz = sum_partials(PSLOT(a, P_RZ0), a.nvb, lds);
+    double nz = sum_partials(PSLOT(a, P_NNZ), a.nvb, lds);
+    if (threadIdx.x == 0) cg_start(a, sqrt(bb), rz, nz);
 }
 
 // Row products over the SELL-64 matrix, entries in row order after the
@@ -260,6 +295,15 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(CgArgs<VT, MT> a)
     if (threadIdx.x == 0) PSLOT(a, P_PQ)[blockIdx.x] = pq;
 }
 
+// A load of matrix data: kKeep for a matrix that the caches hold from one
+// product to the next, else it passes by them.
+template <bool kKeep, class T>
+__device__ __forceinline__ T stream_load(const T* p)
+{
+    if constexpr (kKeep) return *p;
+    else return __builtin_nontemporal_load(p);
+}
+
 // Step or rank u (0..7) of a 16-byte chunk of 16-bit values.
 __device__ __forceinline__ int u16_of(const v4u& w, int u)
 {
@@ -273,39 +317,98 @@ __device__ __forceinline__ int u16_of(const v4u& w, int u)
 // global memory, one cache-line lookup per distinct line touched by each
 // wave-wide load, become one coalesced staging pass per block; the row sums
 // are the same operations in the same order, so q and p.q are the same bits.
-template <class VT, class MT>
+//
+// kF = 1 (CG) and 2 (flexible CG): the product also ends the iteration before
+// it, in place of k_cg_p / k_fcg_p: every block adds that iteration's partials,
+// tests it and stages p = z + beta pold at its window's columns; its own rows of
+// p go to the other of two buffers, since other blocks still read pold. The
+// first product of a CG solve starts it (k_cg_init_fin). The same operations,
+// so the same bits. A launch an iteration less, which is what small systems are
+// bound by; the window's second gather is about what k_cg_p read and wrote.
+// (updates_p has both sides measured.)
+template <class VT, class MT, int kF, bool kKeep>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv_win(CgArgs<VT, MT> a)
 {
     extern __shared__ __align__(16) unsigned char dyn_lds[];
     VT* win = reinterpret_cast<VT*>(dyn_lds);
     __shared__ double lds[kBlock];
-    if (a.flags[FLAG_CG_DONE]) return;
+    const int wave = threadIdx.x >> 6;
+    const bool lead = (blockIdx.x == 0 && threadIdx.x == 0);
+    const bool first = kF == 1 && a.it == 1;
+    if (!first && a.flags[FLAG_CG_DONE]) return;
     const int ch = xcd_block();
+    const int r = ch * kBlock + threadIdx.x;
+    const bool row = r < a.nu;
+    const v4u* __restrict__ wc = a.wcol + dc_index(r, 0, a.cap);
+    const MT* __restrict__ val = a.aval + mx_index(r, 0, a.cap);
+    const int len = row ? a.rowlen[r] : 0;
+    VT beta = (VT)0;
+    if (first) {
+        if (wave < 3) {
+            const double s = wave_partials<8>(wave == 0 ? PSLOT(a, P_BB) : wave == 1 ? PSLOT(a, P_RZ0)
+                                                                                    : PSLOT(a, P_NNZ), a.nvb);
+            lds[wave] = s;
+        }
+        __syncthreads();
+        const double bn = sqrt(lds[0]);
+        if (lead) cg_start(a, bn, lds[1], lds[2]);
+        if (bn == 0.0) return;
+    } else if (kF == 1) {
+        if (wave < 2) lds[wave] = wave_partials<8>(wave == 0 ? PSLOT(a, P_RR) : PSLOT(a, P_RZ), a.nvb);
+        __syncthreads();
+        const double rz = lds[1];
+        if (!cg_goes_on(a, lds[0], a.it - 1, lead)) return;
+        beta = (VT)(rz / a.scal[S_RZ0 + (a.it & 1)]);
+        if (lead) a.scal[S_RZ0 + ((a.it - 1) & 1)] = rz;
+    } else if (kF == 2 && a.it > 1) {
+        if (wave < 2) lds[wave] = wave_partials<16>(wave == 0 ? PSLOT(a, P_RZ) : PSLOT(a, P_ZQ), a.npq);
+        __syncthreads();
+        const double zr = lds[0], zq = lds[1];
+        if (!(zr > 0.0) || !isfinite(zr)) {
+            // M r is not a descent direction: the preconditioner is not positive here
+            if (lead) { a.flags[FLAG_CG_BREAK] = 1; a.flags[FLAG_CG_DONE] = 1; }
+            return;
+        }
+        const double rz_old = a.scal[S_RZ0 + (a.it & 1)];
+        const double alpha = rz_old / a.scal[S_PQ];
+        beta = (VT)(-alpha * zq / rz_old);
+        if (lead) a.scal[S_RZ0 + ((a.it - 1) & 1)] = zr;
+    }
+    const bool renew = kF != 0 && a.it > 1;
     const int n = a.wn[ch];
     const int32_t* __restrict__ uq = a.wuniq + (long)ch * kWinMax;
-    for (int t = threadIdx.x; t < n; t += kBlock) win[t] = a.p[uq[t]];
+    if (renew)
+        for (int t = threadIdx.x; t < n; t += kBlock) {
+            const int k = uq[t];
+            win[t] = a.z[k] + beta * a.pold[k];
+        }
+    else
+        for (int t = threadIdx.x; t < n; t += kBlock) win[t] = a.p[uq[t]];
     __syncthreads();
     double pq = 0.0;
-    const int r = ch * kBlock + threadIdx.x;
-    if (r < a.nu) {
-        // (issuing the first batch before the staging, and each batch before
-        // the previous one is consumed, measured the same)
-        const VT pr = a.p[r];
+    if (row) {
+        VT pr;
+        if (renew) {
+            pr = a.z[r] + beta * a.pold[r];
+            a.p[r] = pr;
+        } else {
+            pr = a.p[r];
+        }
         VT acc = (VT)a.diag[r] * pr;
-        const int len = a.rowlen[r];
-        const v4u* __restrict__ wc = a.wcol + dc_index(r, 0, a.cap);
-        const MT* __restrict__ val = a.aval + mx_index(r, 0, a.cap);
+        // (issuing the first batch before the staging, and each batch before
+        // the previous one is consumed, measured the same on large systems;
+        // 16 entries ahead, the first before the sums, slower on small ones)
         int k = 0;
         for (; k + 8 <= len; k += 8) {
-            const v4u w = __builtin_nontemporal_load(&wc[8L * k]);
+            const v4u w = stream_load<kKeep>(&wc[8L * k]);
             MT vv[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) vv[u] = __builtin_nontemporal_load(&val[64L * (k + u)]);
+            for (int u = 0; u < 8; ++u) vv[u] = stream_load<kKeep>(&val[64L * (k + u)]);
 #pragma unroll
             for (int u = 0; u < 8; ++u) acc = acc + (VT)vv[u] * win[u16_of(w, u)];
         }
         if (k < len) {
-            const v4u w = __builtin_nontemporal_load(&wc[8L * k]);
+            const v4u w = stream_load<kKeep>(&wc[8L * k]);
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (k + u < len) acc = acc + (VT)val[64L * (k + u)] * win[u16_of(w, u)];
@@ -343,14 +446,15 @@ __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
     uint32_t* bits = wlds;
     uint16_t* pre = reinterpret_cast<uint16_t*>(wlds + a.words);
     __shared__ int red[kBlock];
-    __shared__ int outside;
+    __shared__ int outside, chunks;
     const int ch = blockIdx.x, t = threadIdx.x;
     const int r = ch * kBlock + t;
     const int len = (r < a.nu) ? a.rowlen[r] : 0;
     const int first = (len > 0) ? a.cbase[r] : 0x7fffffff;
     red[t] = first;
-    if (t == 0) outside = 0;
+    if (t == 0) outside = chunks = 0;
     __syncthreads();
+    atomicAdd(&chunks, (len + 7) >> 3);
     for (int s = kBlock / 2; s > 0; s >>= 1) {
         if (t < s) red[t] = min(red[t], red[t + s]);
         __syncthreads();
@@ -468,6 +572,7 @@ __global__ __launch_bounds__(kBlock) void k_win_build(WinArgs a)
         a.wn[ch] = total;
         atomicMax(spread_at(a.spread, SPR_WIN_N), total);
         atomicAdd(spread_at(a.spread, SPR_WIN_SUM), total);
+        atomicAdd(spread_at(a.spread, SPR_CHUNKS), chunks);
     }
 }
 
@@ -476,7 +581,7 @@ __global__ __launch_bounds__(kVecThreads) void k_cg_update(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kVecThreads];
     if (a.flags[FLAG_CG_DONE]) return;
-    const double pq = sum_partials_n<kVecThreads>(PSLOT(a, P_PQ), a.npq, lds);
+    const double pq = vec_partials(PSLOT(a, P_PQ), a.npq, lds);
     const double rz_old = a.scal[S_RZ0 + ((a.it - 1) & 1)];
     if (!(pq > 0.0) || !isfinite(pq)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -494,6 +599,7 @@ __global__ __launch_bounds__(kVecThreads) void k_cg_update(CgArgs<VT, MT> a)
         const VT res = a.r[r] - alpha * a.q[r];
         a.r[r] = res;
         const VT z = res / (VT)a.diag[r];
+        if (a.z) a.z[r] = z;
         rr += (double)res * (double)res;
         rz += (double)res * (double)z;
     }
@@ -508,28 +614,24 @@ __global__ __launch_bounds__(kVecThreads) void k_cg_update(CgArgs<VT, MT> a)
 template <class VT, class MT>
 __global__ __launch_bounds__(kVecThreads) void k_cg_p(CgArgs<VT, MT> a)
 {
-    __shared__ double lds[kVecThreads];
     if (a.flags[FLAG_CG_DONE]) return;
-    const double rr = sum_partials_n<kVecThreads>(PSLOT(a, P_RR), kVecBlocks, lds);
-    const double rz = sum_partials_n<kVecThreads>(PSLOT(a, P_RZ), kVecBlocks, lds);
-    const double rel = sqrt(rr) / a.scal[S_BNORM];
+    const double rr = wave_partials<8>(PSLOT(a, P_RR), a.nvb);
+    const double rz = wave_partials<8>(PSLOT(a, P_RZ), a.nvb);
     const bool lead = (blockIdx.x == 0 && threadIdx.x == 0);
-    if (lead) {
-        a.scal[S_RELRES] = rel;
-        a.flags[FLAG_CG_ITERS] = a.it;
-    }
-    if (rel <= a.tol) {
-        if (lead) { a.flags[FLAG_CG_CONV] = 1; a.flags[FLAG_CG_DONE] = 1; }
-        return;
-    }
-    if (a.it >= a.maxit || !isfinite(rel)) {
-        if (lead) a.flags[FLAG_CG_DONE] = 1;
-        return;
-    }
+    if (!cg_goes_on(a, rr, a.it, lead)) return;
     const VT beta = (VT)(rz / a.scal[S_RZ0 + ((a.it - 1) & 1)]);
     if (lead) a.scal[S_RZ0 + (a.it & 1)] = rz;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < a.nu; r += gridDim.x * blockDim.x)
         a.p[r] = a.r[r] / (VT)a.diag[r] + beta * a.p[r];
+}
+
+// The end of the last iteration queued before the host reads the flags, where
+// the products update p (one wave).
+template <class VT, class MT>
+__global__ __launch_bounds__(kWave) void k_cg_test(CgArgs<VT, MT> a)
+{
+    if (a.flags[FLAG_CG_DONE]) return;
+    cg_goes_on(a, wave_partials<8>(PSLOT(a, P_RR), a.nvb), a.it, threadIdx.x == 0);
 }
 
 // ---- flexible CG ---------------------------------------------------------------------------
@@ -601,8 +703,8 @@ template <class VT, class MT>
 __global__ __launch_bounds__(kBlock) void k_fcg_init_fin(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kBlock];
-    const double bb = sum_partials(PSLOT(a, P_BB), kVecBlocks, lds);
-    const double nz = sum_partials(PSLOT(a, P_NNZ), kVecBlocks, lds);
+    const double bb = sum_partials(PSLOT(a, P_BB), a.nvb, lds);
+    const double nz = sum_partials(PSLOT(a, P_NNZ), a.nvb, lds);
     const double rz = sum_partials(PSLOT(a, P_RZ0), a.npq, lds);
     if (threadIdx.x == 0) {
         const double bn = sqrt(bb);
@@ -624,7 +726,7 @@ __global__ __launch_bounds__(kVecThreads) void k_fcg_update(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kVecThreads];
     if (a.flags[FLAG_CG_DONE]) return;
-    const double pq = sum_partials_n<kVecThreads>(PSLOT(a, P_PQ), a.npq, lds);
+    const double pq = vec_partials(PSLOT(a, P_PQ), a.npq, lds);
     const double rz_old = a.scal[S_RZ0 + ((a.it - 1) & 1)];
     if (!(pq > 0.0) || !isfinite(pq)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -635,6 +737,7 @@ __global__ __launch_bounds__(kVecThreads) void k_fcg_update(CgArgs<VT, MT> a)
         return;
     }
     const VT alpha = (VT)(rz_old / pq);
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.scal[S_PQ] = pq;
     double rr = 0.0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < a.nu; r += gridDim.x * blockDim.x) {
         a.x[r] = a.x[r] + alpha * a.p[r];
@@ -651,21 +754,8 @@ __global__ __launch_bounds__(kBlock) void k_fcg_prec(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kBlock];
     if (a.flags[FLAG_CG_DONE]) return;
-    const double rr = sum_partials(PSLOT(a, P_RR), kVecBlocks, lds);
-    const double rel = sqrt(rr) / a.scal[S_BNORM];
-    const bool lead = (blockIdx.x == 0 && threadIdx.x == 0);
-    if (lead) {
-        a.scal[S_RELRES] = rel;
-        a.flags[FLAG_CG_ITERS] = a.it;
-    }
-    if (rel <= a.tol) {
-        if (lead) { a.flags[FLAG_CG_CONV] = 1; a.flags[FLAG_CG_DONE] = 1; }
-        return;
-    }
-    if (a.it >= a.maxit || !isfinite(rel)) {
-        if (lead) a.flags[FLAG_CG_DONE] = 1;
-        return;
-    }
+    const double rr = sum_partials(PSLOT(a, P_RR), a.nvb, lds);
+    if (!cg_goes_on(a, rr, a.it, blockIdx.x == 0 && threadIdx.x == 0)) return;
     double zr = 0.0, zq = 0.0;
     const int r = xcd_tid();
     if (r < a.nu) {
@@ -687,7 +777,7 @@ __global__ __launch_bounds__(kVecThreads) void k_fcg_p(CgArgs<VT, MT> a)
 {
     __shared__ double lds[kVecThreads];
     if (a.flags[FLAG_CG_DONE]) return;
-    const double pq = sum_partials_n<kVecThreads>(PSLOT(a, P_PQ), a.npq, lds);
+    const double pq = a.scal[S_PQ];
     const double zr = sum_partials_n<kVecThreads>(PSLOT(a, P_RZ), a.npq, lds);
     const double zq = sum_partials_n<kVecThreads>(PSLOT(a, P_ZQ), a.npq, lds);
     const double rz_old = a.scal[S_RZ0 + ((a.it - 1) & 1)];
@@ -850,18 +940,51 @@ __global__ void k_scatter_x(int nu, const int32_t* __restrict__ urow, const doub
 }
 
 // ---- host ------------------------------------------------------------------------------------
+// Whether the products update p (k_cg_spmv_win). Measured per solve of 11 to 14
+// iterations, without and with: 2D rows 0.9k 192 -> 176 us, 12k 221 -> 180, 80k
+// 226 -> 194, 377k 449 -> 405; 3D rows 64k 617 -> 578, 139k 1028 -> 1010, 179k to
+// 272k equal, 820k 6.6 -> 6.8 ms: a 3D chunk stages 6 to 7 columns a row, whose
+// second gather costs what k_cg_p did, a 2D chunk 2 to 3.
+constexpr int kFusedBlocks = 768;
+template <class VT, class MT>
+static bool updates_p(const vox_ctx* c, const CgArgs<VT, MT>& a)
+{
+    return c->tune_spmv == 0 && a.wcol && a.maxit > 0 &&
+           (a.npq <= kFusedBlocks || c->win_sum <= 4L * c->nu);
+}
+
+// Whether the matrix's columns and values stay in the 256 MB cache between
+// products. Solves with loads that pass it by and with ordinary ones: 139 MB
+// 578 -> 524 us, 211 MB 792 -> 732, 278 MB 1010 -> 969 but 367 MB 1235 -> 1320 and
+// 598 MB 1864 -> 2132; FP32 values 167 MB 810 -> 737, 277 MB 1186 -> 1161 but
+// 359 MB 1523 -> 1626; 2D 37 MB 290 -> 260.
+constexpr long kKeepBytes = 288L << 20;
+template <class MT>
+static bool fits_caches(const vox_ctx* c)
+{
+    return 8L * c->win_chunks * (long)(sizeof(uint16_t) + sizeof(MT)) <= kKeepBytes;
+}
+
 // The product variant the autotuner chose (variant 0 unless tuned). Variant 0
 // gathers p from the blocks' LDS windows when they are built, variant 4 reads
 // the columns' 16-bit steps when the assembly stored them all; either falls
 // back to the next form (window -> steps -> 32-bit columns). Variants 1-3
 // read the 32-bit columns, 4, 16 and 8 entries per batch.
 template <class VT, class MT>
-static void launch_spmv(vox_ctx* c, const CgArgs<VT, MT>& a, int variant)
+static void launch_spmv(vox_ctx* c, const CgArgs<VT, MT>& a, int variant, int fused = 0)
 {
     if (variant == 0 && a.wcol) {
         c->st.product_col_bytes = 2;
         c->st.product_window_cols = c->win_sum;
-        k_cg_spmv_win<VT, MT><<<a.npq, kBlock, sizeof(VT) * (size_t)a.win_n, c->stream>>>(a);
+        const size_t lds = sizeof(VT) * (size_t)a.win_n;
+        auto go = [&](auto f) {
+            constexpr int F = decltype(f)::value;
+            if (fits_caches<MT>(c)) k_cg_spmv_win<VT, MT, F, true><<<a.npq, kBlock, lds, c->stream>>>(a);
+            else k_cg_spmv_win<VT, MT, F, false><<<a.npq, kBlock, lds, c->stream>>>(a);
+        };
+        if (fused == 1) go(std::integral_constant<int, 1>{});
+        else if (fused == 2) go(std::integral_constant<int, 2>{});
+        else go(std::integral_constant<int, 0>{});
         return;
     }
     const bool steps = (variant == 0 || variant == 4) && a.dcol != nullptr;
@@ -878,14 +1001,26 @@ static void launch_spmv(vox_ctx* c, const CgArgs<VT, MT>& a, int variant)
     }
 }
 
+// The two buffers of p swap with each iteration that updates p in its product.
+template <class VT, class MT>
+static void next_direction(CgArgs<VT, MT>& a, VT* const buf[2])
+{
+    a.p = buf[(a.it - 1) & 1];
+    a.pold = buf[a.it & 1];
+}
+
 // Runs CG on A x = rhs to ||r|| <= tol ||rhs||. Returns iterations; *conv, *brk.
 template <class VT, class MT>
 static int run_cg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
 {
+    // the products that gather from LDS windows update p themselves
+    const bool fused = updates_p(c, a);
+    VT* const buf[2] = {a.p, reinterpret_cast<VT*>(c->cg_pn)};
+    a.z = fused ? reinterpret_cast<VT*>(c->cg_zj) : nullptr;
     {
         ProfScope ps(c, KC_CG_INIT);
-        k_cg_init<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
-        k_cg_init_fin<VT, MT><<<1, kBlock, 0, c->stream>>>(a);
+        k_cg_init<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
+        if (!fused) k_cg_init_fin<VT, MT><<<1, kBlock, 0, c->stream>>>(a);
         VOX_HIP(hipGetLastError());
     }
     // Check schedule: the first batch runs the last solve's count (consecutive
@@ -905,16 +1040,21 @@ static int run_cg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
             a.it = ++it;
             {
                 ProfScope ps(c, KC_SPMV);
-                launch_spmv<VT, MT>(c, a, c->tune_spmv);
+                if (fused) next_direction(a, buf);
+                launch_spmv<VT, MT>(c, a, c->tune_spmv, fused ? 1 : 0);
             }
             {
                 ProfScope ps(c, KC_CG_UPDATE);
-                k_cg_update<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+                k_cg_update<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
             }
-            {
+            if (!fused) {
                 ProfScope ps(c, KC_CG_P);
-                k_cg_p<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+                k_cg_p<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
             }
+        }
+        if (fused) {
+            ProfScope ps(c, KC_CG_P);
+            k_cg_test<VT, MT><<<1, kWave, 0, c->stream>>>(a);
         }
         VOX_HIP(hipGetLastError());
         VOX_TRY(read_flags(c));
@@ -931,9 +1071,11 @@ static int run_cg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
 template <class VT, class MT>
 static int run_fcg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
 {
+    const bool fused = updates_p(c, a);
+    VT* const buf[2] = {a.p, reinterpret_cast<VT*>(c->cg_pn)};
     {
         ProfScope ps(c, KC_CG_INIT);
-        k_fcg_init<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+        k_fcg_init<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
     }
     {
         ProfScope ps(c, KC_LPC_APPLY);
@@ -956,19 +1098,20 @@ static int run_fcg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
             a.it = ++it;
             {
                 ProfScope ps(c, KC_SPMV);
-                launch_spmv<VT, MT>(c, a, c->tune_spmv);
+                if (fused) next_direction(a, buf);
+                launch_spmv<VT, MT>(c, a, c->tune_spmv, fused ? 2 : 0);
             }
             {
                 ProfScope ps(c, KC_CG_UPDATE);
-                k_fcg_update<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+                k_fcg_update<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
             }
             {
                 ProfScope ps(c, KC_LPC_APPLY);
                 k_fcg_prec<VT, MT><<<a.npq, kBlock, 0, c->stream>>>(a);
             }
-            {
+            if (!fused) {
                 ProfScope ps(c, KC_CG_P);
-                k_fcg_p<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+                k_fcg_p<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
             }
         }
         VOX_HIP(hipGetLastError());
@@ -1026,6 +1169,7 @@ static int ensure_window(vox_ctx* c)
     VOX_TRY(read_flags(c));
     c->win_n = spread_max(c, SPR_WIN_N);
     c->win_sum = spread_sum(c, SPR_WIN_SUM);
+    c->win_chunks = spread_sum(c, SPR_CHUNKS);
     c->win_ok = c->win_n <= kWinMax;
     return VOX_OK;
 }
@@ -1049,9 +1193,10 @@ static void fill_args(vox_ctx* c, CgArgs<VT, MT>& a, const MT* aval, VT* x, VT* 
     a.wuniq = c->wuniq; a.wn = c->wn; a.win_n = c->win_n;
     a.nu = c->nu; a.cap = c->a_cap; a.tol = tol; a.maxit = maxit; a.it = 0;
     a.npq = grid_for(c->nu > 0 ? c->nu : 1);
+    a.nvb = std::min(kVecBlocks, grid_for(c->nu > 0 ? c->nu : 1, kVecThreads));
     a.rowlen = c->rowlen; a.acol = c->acol; a.aval = aval; a.diag = c->adiag; a.rhs = rhs;
     a.dcol = c->dcol_ok ? reinterpret_cast<const v4u*>(c->dcol) : nullptr; a.cbase = c->cbase;
-    a.x = x; a.r = r; a.p = p; a.q = q;
+    a.x = x; a.r = r; a.p = p; a.pold = p; a.q = q;
     a.part = c->partials; a.scal = c->dscal; a.flags = c->dflags;
     a.z = nullptr; a.slen = c->lpc_slen; a.scol = c->lpc_scol; a.sval = c->lpc_sval; a.gd = c->lpc_gd;
     a.scap = c->lpc_scap;
@@ -1240,7 +1385,7 @@ static int solve_learned(vox_ctx* c, vox_solve_info* info)
 template <class VT, class MT>
 static int time_spmv_t(vox_ctx* c, CgArgs<VT, MT>& a, int reps, float* ms)
 {
-    k_cg_init<VT, MT><<<kVecBlocks, kVecThreads, 0, c->stream>>>(a);
+    k_cg_init<VT, MT><<<a.nvb, kVecThreads, 0, c->stream>>>(a);
     k_cg_init_fin<VT, MT><<<1, kBlock, 0, c->stream>>>(a);
     VOX_HIP(hipGetLastError());
     hipEvent_t e0, e1;

@@ -2,6 +2,7 @@
 // libvoxarmps. Everything here is gfx950 (wave64) code; no other target.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -91,6 +92,7 @@ enum SpreadSlot {
     SPR_COL_ABOVE,         //                last column - row (max)
     SPR_WIN_N,             // most distinct columns of a PPE chunk (max; see wcol)
     SPR_WIN_SUM,           // distinct columns over all chunks (sum)
+    SPR_CHUNKS,            // 8-entry chunks of the PPE's rows (sum)
     SPR_COUNT
 };
 constexpr int kSpread = 32;
@@ -292,6 +294,7 @@ struct vox_ctx {
     int wcap_alloc = 0;            // a_cap wcol was allocated for
     int win_n = 0;                 // most distinct columns of a chunk
     int win_sum = 0;               // distinct columns over all chunks
+    int win_chunks = 0;            // 8-entry chunks of all rows
     int col_below = 0, col_above = 0;   // every row's columns lie in [r - below, r + above]
     bool win_ok = false;
     long asm_count = 0;            // PPE assemblies and loads so far
@@ -311,6 +314,8 @@ struct vox_ctx {
     double* cg_x = nullptr;
     double* cg_r = nullptr;
     double* cg_p = nullptr;
+    double* cg_pn = nullptr;       // the other half of p and z = r / d, when the product
+    double* cg_zj = nullptr;       //   also updates p (floats in a mixed solve)
     double* cg_q = nullptr;
     double* cg_d = nullptr;        // FP64 inner solve of a warm-started solve: x
     double* cg_e = nullptr;        //   and residual
@@ -663,20 +668,51 @@ __device__ __forceinline__ int32_t* spread_at(int32_t* spread, int slot)
     return spread + (blockIdx.x & (kSpread - 1)) * kSpreadLine + slot;
 }
 
-// Fixed-order block sum of one double per thread (blockDim == kBlock).
-__device__ __forceinline__ double block_sum(double v, double* lds)
+// The last six levels of the sums' fixed tree, v_t + v_(t + s) for s = 32 .. 1,
+// within a wave; the result is in lane 0.
+__device__ __forceinline__ double wave_tree(double v)
 {
-    // wave-level tree through LDS keeps a fixed association order
-    int t = threadIdx.x;
+    v = v + __shfl_down(v, 32);
+    v = v + __shfl_down(v, 16);
+    auto from = [](double x, auto ctrl) {              // lane t takes lane t + n of its row of 16
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), decltype(ctrl)::value, 0xf, 0xf, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), decltype(ctrl)::value, 0xf, 0xf, true);
+        return __hiloint2double(hi, lo);
+    };
+    v = v + from(v, std::integral_constant<int, 0x108>{});
+    v = v + from(v, std::integral_constant<int, 0x104>{});
+    v = v + from(v, std::integral_constant<int, 0x102>{});
+    v = v + from(v, std::integral_constant<int, 0x101>{});
+    return v;
+}
+
+// Fixed-order sum of one double per thread over a block of NT threads: the tree
+// lds[t] + lds[t + s], s = NT / 2 .. 1, with its levels above a wave done by the
+// first wave in registers (two barriers instead of one a level).
+template <int NT>
+__device__ __forceinline__ double block_sum_n(double v, double* lds)
+{
+    constexpr int J = NT / kWave;
+    const int t = threadIdx.x;
     lds[t] = v;
     __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (t < s) lds[t] = lds[t] + lds[t + s];
-        __syncthreads();
+    if (t < kWave) {
+        double w[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) w[j] = lds[t + kWave * j];
+#pragma unroll
+        for (int h = J / 2; h > 0; h >>= 1)
+#pragma unroll
+            for (int j = 0; j < h; ++j) w[j] = w[j] + w[j + h];
+        const double r = wave_tree(w[0]);
+        if (t == 0) lds[0] = r;
     }
-    double r = lds[0];
+    __syncthreads();
+    const double r = lds[0];
     __syncthreads();
     return r;
 }
+
+__device__ __forceinline__ double block_sum(double v, double* lds) { return block_sum_n<kBlock>(v, lds); }
 
 }  // namespace vox

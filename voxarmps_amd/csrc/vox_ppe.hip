@@ -118,7 +118,8 @@ __global__ void k_pack_asm(AsmArgs a)
     // what the assembly and the window build report
     if (i < kSpread) {
         int32_t* sp = a.spread + i * kSpreadLine;
-        sp[SPR_COL_BELOW] = sp[SPR_COL_ABOVE] = sp[SPR_WIN_N] = sp[SPR_WIN_SUM] = 0;
+        sp[SPR_COL_BELOW] = sp[SPR_COL_ABOVE] = sp[SPR_WIN_N] = sp[SPR_WIN_SUM] =
+            sp[SPR_CHUNKS] = 0;
         if (i == 0) *a.dbad = 0;
     }
     if (i >= a.n) return;
