@@ -660,25 +660,38 @@ template <class VT, class MT>
 __device__ __forceinline__ VT apply_m(const CgArgs<VT, MT>& a, int r)
 {
     VT acc = (VT)a.gd[r] * a.r[r];
-    const long b = mx_index(r, 0, a.scap);
     const int len = a.slen[r];
+    if (len <= 0) return acc;
+    const long b = mx_index(r, 0, a.scap);
+    const int32_t* __restrict__ col = a.scol + b;
+    const float* __restrict__ val = a.sval + b;
+    // the next 8 entries are loaded before these are used (past the row's end its
+    // last entry again)
     constexpr int U = 8;
-    int k = 0;
-    for (; k + U <= len; k += U) {
-        int32_t cc[U];
-        float vv[U];
-        VT rr[U];
+    int32_t cc[U];
+    float vn[U];
+    auto next = [&](int k) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            cc[u] = __builtin_nontemporal_load(&a.scol[b + 64L * (k + u)]);
-            vv[u] = __builtin_nontemporal_load(&a.sval[b + 64L * (k + u)]);
+            const long i = 64L * min(k + u, len - 1);
+            cc[u] = col[i];
+            vn[u] = val[i];
         }
+    };
+    next(0);
+    for (int k = 0; k < len; k += U) {
+        VT rr[U];
+        float vv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) rr[u] = a.r[cc[u]];
+        for (int u = 0; u < U; ++u) {
+            rr[u] = a.r[cc[u]];
+            vv[u] = vn[u];
+        }
+        next(k + U);
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc = acc + (VT)vv[u] * rr[u];
+        for (int u = 0; u < U; ++u)
+            if (k + u < len) acc = acc + (VT)vv[u] * rr[u];
     }
-    for (; k < len; ++k) acc = acc + (VT)a.sval[b + 64L * k] * a.r[a.scol[b + 64L * k]];
     return acc;
 }
 

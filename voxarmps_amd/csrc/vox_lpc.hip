@@ -28,9 +28,15 @@
 // launch, the 16 x 64 output tile staged in LDS for the coalesced store and
 // for the message product that follows in the same kernel.
 //
-// Training (mean over probes w of ||A M w - w||^2 / ||w||^2, Adam): the
-// backward pass runs in FP32 on the vector units, one thread per row, with
-// weight gradients reduced per block in a fixed order (deterministic).
+// Row walks take 4 or 8 lanes per row, each with its own channels (or probe, or
+// moment): the lanes of a row read one gathered record side by side (one cache
+// lookup instead of one a lane), every sum stays one chain in the row's order,
+// and a system of a few thousand rows still fills the chip.
+//
+// Training (mean over probes w of ||A M w - w||^2 / ||w||^2, Adam): the four
+// probes go through one walk of each operator, and the backward pass runs in
+// FP32, its dense products and weight gradients on v_mfma_f32_16x16x4_f32, with
+// weight gradients reduced in a fixed order (deterministic).
 #include <algorithm>
 #include <cstring>
 #include <numeric>
@@ -52,7 +58,6 @@ constexpr float kCMax = 2.5f;
 constexpr float kBeta = -0.40546510810816438f;   // -ln(1.5): c = 1 at zero output
 constexpr int kProbes = 4;
 constexpr int kOuterBlocks = 256;
-constexpr int kOuterMax = LH * LH;
 
 // ---- bf16 (round to nearest even; inputs are finite) -----------------------
 __device__ __forceinline__ uint16_t f2bf(float x)
@@ -72,6 +77,49 @@ __device__ __forceinline__ double rademacher(uint64_t seed, int probe, int r)
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z = z ^ (z >> 31);
     return (z >> 63) ? -1.0 : 1.0;
+}
+
+// ---- row walks ---------------------------------------------------------------
+// The first `len` entries of a SELL-64 row in order: f(column, value, gathered)
+// for each, gathered = get(column). U entries' gathers are in flight together,
+// and the next U columns and values are loaded before they are used; loads past
+// the row's end take its last entry again, so none sits in a branch.
+template <int U, class Get, class F>
+__device__ __forceinline__ void walk_row(const int32_t* __restrict__ col, const float* __restrict__ val,
+                                         int len, Get get, F f)
+{
+    if (len <= 0) return;
+    int32_t c[U], cn[U];
+    float v[U], vn[U];
+    auto next = [&](int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long i = 64L * min(k + u, len - 1);
+            cn[u] = col[i];
+            vn[u] = val[i];
+        }
+    };
+    decltype(get(0)) x[U];
+    auto gather = [&]() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            c[u] = cn[u];
+            v[u] = vn[u];
+            x[u] = get(c[u]);
+        }
+    };
+    next(0);
+    int k = 0;
+    for (; k + U <= len; k += U) {
+        gather();
+        next(k + U);
+#pragma unroll
+        for (int u = 0; u < U; ++u) f(c[u], v[u], x[u]);
+    }
+    gather();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (k + u < len) f(c[u], v[u], x[u]);
 }
 
 // ---- features and strong couplings ------------------------------------------
@@ -125,51 +173,61 @@ struct FeatArgs {
     float* sval;
 };
 
+// Four lanes per row: x, y, z moments and the sum of magnitudes. Strong
+// couplings wait in LDS for whole-line stores at the end (a wave's stores hold up
+// its next gathers); a row's 49th and later are stored as they come.
+// 240 -> 154 us at 107k rows of 215 entries (254 with the stores in the walk).
+constexpr int kStrongLds = 48;
 __global__ __launch_bounds__(kBlock) void k_lpc_features(FeatArgs a)
 {
-    const int r = xcd_tid();
-    if (r >= a.nu) return;
-    const v4f pr = a.upos[r];
-    float osum = 0.f, mx = 0.f, my = 0.f, mz = 0.f;
-    const long b = mx_index(r, 0, a.cap);
-    const int len = a.rowlen[r];
-    int n = 0;
-    constexpr int U = 8;
-    for (int k = 0; k < len; k += U) {
-        int32_t cc[U];
-        float oo[U];
-        v4f pp[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool ok = (k + u) < len;
-            cc[u] = ok ? __builtin_nontemporal_load(&a.acol[b + 64L * (k + u)]) : r;
-            oo[u] = ok ? -__builtin_nontemporal_load(&a.aval[b + 64L * (k + u)]) : 0.f;
+    __shared__ int32_t qc[kStrongLds][kWave];
+    __shared__ float qv[kStrongLds][kWave];
+    __shared__ int sn[kWave];
+    const int q = threadIdx.x & 3, lr = threadIdx.x >> 2;
+    const int row0 = xcd_block() * kWave, r = row0 + lr;
+    if (r < a.nu) {
+        const float* __restrict__ pos = reinterpret_cast<const float*>(a.upos);
+        const float own = pos[4L * r + q];
+        const long b = mx_index(r, 0, a.cap);
+        float acc = 0.f;
+        int n = 0;
+        walk_row<8>(a.acol + b, a.aval + b, a.rowlen[r], [&](int c) { return pos[4L * c + q]; },
+                    [&](int c, float v, float x) {
+                        const float o = -v;
+                        acc = fmaf(o, q < 3 ? x - own : 1.f, acc);
+                        if ((double)o >= a.thr) {
+                            if (n < kStrongLds) {
+                                if (q == 0) qc[n][lr] = c;
+                                if (q == 1) qv[n][lr] = o;
+                            } else {
+                                if (q == 0) a.scol[b + 64L * n] = c;
+                                if (q == 1) a.sval[b + 64L * n] = o;
+                            }
+                            ++n;
+                        }
+                    });
+        const float osum = __shfl(acc, 3, 4);
+        const float inv = (osum > 0.f) ? 1.f / osum : 0.f;
+        float* f = a.feat + 8L * r;
+        if (q < 3) {
+            f[3 + q] = acc * inv * a.inv_re;
+            if (q < 2) f[6 + q] = 0.f;
+        } else {
+            a.slen[r] = n;
+            f[2] = osum * a.invd[r];
+            a.inv_osum[r] = inv;
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u) pp[u] = a.upos[cc[u]];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            osum += oo[u];
-            mx = fmaf(oo[u], pp[u].x - pr.x, mx);
-            my = fmaf(oo[u], pp[u].y - pr.y, my);
-            mz = fmaf(oo[u], pp[u].z - pr.z, mz);
-            if ((double)oo[u] >= a.thr) {   // padding has oo = 0 < thr
-                a.scol[b + 64L * n] = cc[u];
-                a.sval[b + 64L * n] = oo[u];
-                ++n;
-            }
-        }
+        if (q == 0) sn[lr] = min(n, kStrongLds);
+    } else if (q == 0) {
+        sn[lr] = 0;
     }
-    a.slen[r] = n;
-    const float inv = (osum > 0.f) ? 1.f / osum : 0.f;
-    float* f = a.feat + 8L * r;
-    f[2] = osum * a.invd[r];
-    f[3] = mx * inv * a.inv_re;
-    f[4] = my * inv * a.inv_re;
-    f[5] = mz * inv * a.inv_re;
-    f[6] = 0.f;
-    f[7] = 0.f;
-    a.inv_osum[r] = inv;
+    __syncthreads();
+    const int i = threadIdx.x & (kWave - 1), n = sn[i];
+    const long b = mx_index(row0 + i, 0, a.cap);
+    for (int k = threadIdx.x >> 6; k < n; k += kBlock / kWave) {
+        a.scol[b + 64L * k] = qc[k][i];
+        a.sval[b + 64L * k] = qv[k][i];
+    }
 }
 
 // Training-set coupling values: O_rk / (A_rr A_kk) as (O_rk * (1/A_rr)) * (1/A_kk).
@@ -205,56 +263,37 @@ struct AggArgs {
     uint16_t* m;
 };
 
-// m_r = (sum_k O_rk s_k) / sum_k O_rk over the matrix row; one thread per row,
-// 8 entries' 32-byte message gathers in flight.
+// m_r = (sum_k O_rk s_k) / sum_k O_rk over the matrix row: G lanes per row, each
+// with 16 / G of the message's channels.
+// Bound by the gathers' cache lookups: one thread per row, 32 bytes an entry,
+// made two a row and entry, the lanes of a row make one between them. 107k rows
+// of 215 entries 176 -> 103 us (8 lanes: the same within 3 %), 14.6k rows 134 ->
+// 21 us. 16 entries a batch measured the same, 4 slower.
+template <int G>
 __global__ __launch_bounds__(kBlock) void k_lpc_agg(AggArgs a)
 {
-    const int r = xcd_tid();
+    constexpr int D = LM / G / 2;                      // dwords (channel pairs) of a lane
+    const int q = threadIdx.x & (G - 1);
+    const int r = xcd_block() * (kBlock / G) + threadIdx.x / G;
     if (r >= a.nu) return;
-    float acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.f;
+    struct Part { uint32_t w[D]; };
+    const Part* __restrict__ s = reinterpret_cast<const Part*>(a.s);
     const long b = mx_index(r, 0, a.cap);
-    const int len = a.rowlen[r];
-    constexpr int U = 8;
-    for (int k = 0; k < len; k += U) {
-        int32_t cc[U];
-        float oo[U];
-        v4i x[U][2];
+    float acc[2 * D] = {};
+    walk_row<8>(a.acol + b, a.aval + b, a.rowlen[r], [&](int c) { return s[(long)G * c + q]; },
+                [&](int, float v, const Part& x) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool ok = (k + u) < len;
-            cc[u] = ok ? __builtin_nontemporal_load(&a.acol[b + 64L * (k + u)]) : r;
-            oo[u] = ok ? -__builtin_nontemporal_load(&a.aval[b + 64L * (k + u)]) : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const v4i* p = reinterpret_cast<const v4i*>(a.s + 16L * cc[u]);
-            x[u][0] = p[0];
-            x[u][1] = p[1];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4i v = x[u][h];
-                const int32_t e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    acc[8 * h + 2 * t] = fmaf(oo[u], bf_lo(e[t]), acc[8 * h + 2 * t]);
-                    acc[8 * h + 2 * t + 1] = fmaf(oo[u], bf_hi(e[t]), acc[8 * h + 2 * t + 1]);
-                }
-            }
-        }
-    }
+                    for (int t = 0; t < D; ++t) {
+                        acc[2 * t] = fmaf(-v, bf_lo(x.w[t]), acc[2 * t]);
+                        acc[2 * t + 1] = fmaf(-v, bf_hi(x.w[t]), acc[2 * t + 1]);
+                    }
+                });
     const float io = a.inv_osum[r];
-    int32_t w[8];
+    Part o;
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
-        w[t] = (int32_t)((uint32_t)f2bf(acc[2 * t] * io) | ((uint32_t)f2bf(acc[2 * t + 1] * io) << 16));
-    v4i* o = reinterpret_cast<v4i*>(a.m + 16L * r);
-    o[0] = v4i{w[0], w[1], w[2], w[3]};
-    o[1] = v4i{w[4], w[5], w[6], w[7]};
+    for (int t = 0; t < D; ++t)
+        o.w[t] = (uint32_t)f2bf(acc[2 * t] * io) | ((uint32_t)f2bf(acc[2 * t + 1] * io) << 16);
+    reinterpret_cast<Part*>(a.m)[(long)G * r + q] = o;
 }
 
 // Inference: t_r = sqrt(c_r) / A_rr, gd_r = g_r / A_rr from the network
@@ -270,15 +309,18 @@ __global__ void k_lpc_gc_inf(int nu, const float* __restrict__ o, const float* _
     t[r] = sqrtf(cv) * invd[r];
 }
 
+// (4 threads per row, 64 rows side by side; 31 -> 20 us at 107k rows)
 __global__ __launch_bounds__(kBlock) void k_lpc_scale(int nu, int cap, const int32_t* __restrict__ slen,
                                                       const int32_t* __restrict__ scol,
                                                       const float* __restrict__ t, float* sval)
 {
-    const int r = xcd_tid();
+    const int r = xcd_block() * kWave + (threadIdx.x & (kWave - 1));
     if (r >= nu) return;
     const long b = mx_index(r, 0, cap);
     const float tr = t[r];
-    for (int k = 0; k < slen[r]; ++k) sval[b + 64L * k] = (sval[b + 64L * k] * tr) * t[scol[b + 64L * k]];
+    const int len = slen[r];
+    for (int k = threadIdx.x >> 6; k < len; k += kBlock / kWave)
+        sval[b + 64L * k] = (sval[b + 64L * k] * tr) * t[scol[b + 64L * k]];
 }
 
 struct DenseArgs {
@@ -433,46 +475,55 @@ __global__ void k_lpc_gc(int nu, const float* __restrict__ o, float* g, float* c
 }
 
 // ---- training: probes and the loss gradient with respect to g and c --------
-enum { LS_NN = 0, LS_COEF, LS_LOSS, LS_EPOCH, LS_COUNT };
+// Vectors of the four probes are interleaved: element 4 r + p.
+enum { LS_NN = 0, LS_COEF = kProbes, LS_LOSS = 2 * kProbes, LS_EPOCH, LS_COUNT };
 
-__global__ void k_lpc_probe(int nu, int probe, uint64_t seed, const float* __restrict__ rhs, float* w)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nu) return;
-    w[r] = probe == 0 ? rhs[r] : (float)rademacher(seed, probe, r);
-}
-
-__global__ __launch_bounds__(kBlock) void k_lpc_dot(int nu, const float* __restrict__ x, double* part)
+// w = right-hand side, then three Rademacher vectors; v = sc w; partial ||rhs||^2.
+__global__ __launch_bounds__(kBlock) void k_lpc_probe(int nu, uint64_t seed, const float* __restrict__ rhs,
+                                                      const float* __restrict__ sc, v4f* w, v4f* v,
+                                                      double* part)
 {
     __shared__ double lds[kBlock];
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
     double s = 0.0;
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nu; r += gridDim.x * blockDim.x)
-        s += (double)x[r] * (double)x[r];
+    if (r < nu) {
+        const v4f x = {rhs[r], (float)rademacher(seed, 1, r), (float)rademacher(seed, 2, r),
+                       (float)rademacher(seed, 3, r)};
+        w[r] = x;
+        v[r] = x * sc[r];
+        s = (double)x.x * (double)x.x;
+    }
     s = block_sum(s, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// mode 0: scal[LS_NN] = sum, scal[LS_COEF] = 2 / (probes * sum)
-// mode 1: scal[LS_LOSS] += sum / (probes * scal[LS_NN])
-// mode 2: scal[LS_EPOCH] += scal[LS_LOSS]
-__global__ __launch_bounds__(kBlock) void k_lpc_fin(const double* part, int n, double* scal, int mode)
+// From the partial ||rhs||^2 (n1) and ||A M w - w||^2 (n2 a probe): each probe's
+// norm and gradient factor 2 / (probes ||w||^2), and the loss.
+__global__ __launch_bounds__(kBlock) void k_lpc_fin(int nu, const double* __restrict__ part, int n1,
+                                                    const double* __restrict__ epart, int n2, double* scal)
 {
     __shared__ double lds[kBlock];
-    double s = 0.0;
-    for (int k = threadIdx.x; k < n; k += kBlock) s = s + part[k];
-    s = block_sum(s, lds);
-    if (threadIdx.x != 0) return;
-    if (mode == 0) {
-        scal[LS_NN] = s;
-        scal[LS_COEF] = s > 0 ? 2.0 / (kProbes * s) : 0.0;
-    } else if (mode == 1) {
-        scal[LS_LOSS] += scal[LS_NN] > 0 ? s / (kProbes * scal[LS_NN]) : 0.0;
-    } else {
-        scal[LS_EPOCH] += scal[LS_LOSS];
+    double loss = 0.0;
+    for (int p = 0; p < kProbes; ++p) {
+        double s = 0.0, e = 0.0;
+        if (p == 0) {
+            for (int k = threadIdx.x; k < n1; k += kBlock) s = s + part[k];
+            s = block_sum(s, lds);
+        } else {
+            s = (double)nu;
+        }
+        for (int k = threadIdx.x; k < n2; k += kBlock) e = e + epart[(long)p * n2 + k];
+        e = block_sum(e, lds);
+        if (threadIdx.x != 0) continue;
+        scal[LS_NN + p] = s;
+        scal[LS_COEF + p] = s > 0 ? 2.0 / (kProbes * s) : 0.0;
+        loss += s > 0 ? e / (kProbes * s) : 0.0;
     }
+    if (threadIdx.x == 0) scal[LS_LOSS] = loss;
 }
 
 __global__ void k_lpc_set(double* scal, int slot, double v) { scal[slot] = v; }
+__global__ void k_lpc_epoch(double* scal) { scal[LS_EPOCH] += scal[LS_LOSS]; }
 
 struct OpView {   // a SELL-64 operator: rows, cap, lengths, columns, values
     int nu, cap;
@@ -481,133 +532,174 @@ struct OpView {   // a SELL-64 operator: rows, cap, lengths, columns, values
     const float* __restrict__ val;
 };
 
+// init + sum_k a_rk x_k of row r for probe p.
+__device__ __forceinline__ float row_product(const OpView& A, int r, int p, const float* __restrict__ x,
+                                             float init)
+{
+    const long b = mx_index(r, 0, A.cap);
+    float acc = init;
+    walk_row<8>(A.col + b, A.val + b, A.len[r], [&](int c) { return x[4L * c + p]; },
+                [&](int, float v, float y) { acc = fmaf(v, y, acc); });
+    return acc;
+}
+
+// One lane per row and probe in the kernels that follow, so that an operator is
+// walked once for the four probes and a gather takes their 16 bytes together.
+// 14.6k rows of 215 entries, all four probes: residual 4 x 87 -> 20 us, adjoint
+// 4 x 87 -> 17, mprobe 4 x 22 -> 7, dgc 4 x 36 -> 8.
 // t = Oh (sc w); z = g w / A_rr + sc t
 __global__ __launch_bounds__(kBlock) void k_lpc_mprobe(OpView S, const float* __restrict__ sc,
                                                        const float* __restrict__ g,
                                                        const float* __restrict__ inv_d,
-                                                       const float* __restrict__ w, float* t, float* z)
+                                                       const float* __restrict__ w,
+                                                       const float* __restrict__ v, float* t, float* z)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = xcd_tid(), r = e >> 2;
     if (r >= S.nu) return;
-    const long b = mx_index(r, 0, S.cap);
-    float acc = 0.f;
-    for (int k = 0; k < S.len[r]; ++k) {
-        const int cc = S.col[b + 64L * k];
-        acc = fmaf(S.val[b + 64L * k], sc[cc] * w[cc], acc);
-    }
-    t[r] = acc;
-    z[r] = fmaf(sc[r], acc, (g[r] * inv_d[r]) * w[r]);
+    const float acc = row_product(S, r, e & 3, v, 0.f);
+    t[e] = acc;
+    z[e] = fmaf(sc[r], acc, (g[r] * inv_d[r]) * w[e]);
 }
 
-// out = A x - sub (partial ||out||^2 per block), or out = coef * A x (sub null)
-__global__ __launch_bounds__(kBlock) void k_lpc_spmv(OpView A, const float* __restrict__ diag,
-                                                     const float* __restrict__ x,
-                                                     const float* __restrict__ sub,
-                                                     const double* __restrict__ scal, float* out,
-                                                     double* part)
+// e = A z - w, partial ||e||^2 per block and probe
+__global__ __launch_bounds__(kBlock) void k_lpc_residual(OpView A, const float* __restrict__ diag,
+                                                         const float* __restrict__ z,
+                                                         const float* __restrict__ w, float* out,
+                                                         double* epart)
 {
     __shared__ double lds[kBlock];
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = xcd_tid(), r = e >> 2, t = threadIdx.x;
     double ee = 0.0;
     if (r < A.nu) {
-        const long b = mx_index(r, 0, A.cap);
-        float acc = diag[r] * x[r];
-        for (int k = 0; k < A.len[r]; ++k) acc = fmaf(A.val[b + 64L * k], x[A.col[b + 64L * k]], acc);
-        if (sub) {
-            const float e = acc - sub[r];
-            out[r] = e;
-            ee = (double)e * (double)e;
-        } else {
-            out[r] = (float)(scal[LS_COEF] * (double)acc);
-        }
+        const float d = row_product(A, r, e & 3, z, diag[r] * z[e]) - w[e];
+        out[e] = d;
+        ee = (double)d * (double)d;
     }
-    if (sub) {
-        ee = block_sum(ee, lds);
-        if (threadIdx.x == 0) part[blockIdx.x] = ee;
+    lds[t] = ee;
+    __syncthreads();
+    for (int s = kBlock / 2; s >= kProbes; s >>= 1) {
+        if (t < s) lds[t] = lds[t] + lds[t + s];
+        __syncthreads();
     }
+    if (t < kProbes) epart[(long)t * gridDim.x + blockIdx.x] = lds[t];
 }
 
-// u = Oh (sc y); dL/dg += y w / A_rr; dL/dc += (y t + w u) / (2 sc)
+// y = coef A e and sc y
+__global__ __launch_bounds__(kBlock) void k_lpc_adjoint(OpView A, const float* __restrict__ diag,
+                                                        const float* __restrict__ x,
+                                                        const float* __restrict__ sc,
+                                                        const double* __restrict__ scal, float* y, float* ys)
+{
+    const int e = xcd_tid(), r = e >> 2;
+    if (r >= A.nu) return;
+    const float acc = row_product(A, r, e & 3, x, diag[r] * x[e]);
+    const float v = (float)(scal[LS_COEF + (e & 3)] * (double)acc);
+    y[e] = v;
+    ys[e] = sc[r] * v;
+}
+
+// u = Oh (sc y); dL/dg = sum over probes of y w / A_rr; dL/dc = (y t + w u) / (2 sc);
+// then through the output functions (dO) and the head's weights (dh).
 __global__ __launch_bounds__(kBlock) void k_lpc_dgc(OpView S, const float* __restrict__ sc,
                                                     const float* __restrict__ inv_d,
                                                     const float* __restrict__ w,
                                                     const float* __restrict__ t,
-                                                    const float* __restrict__ y, float* dgdc, int first)
+                                                    const float* __restrict__ y,
+                                                    const float* __restrict__ ys,
+                                                    const float* __restrict__ w32,
+                                                    const float* __restrict__ o,
+                                                    const float* __restrict__ g, float* dO, float* dh)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = xcd_tid(), r = e >> 2, p = e & 3;
     if (r >= S.nu) return;
-    const long b = mx_index(r, 0, S.cap);
-    float u = 0.f;
-    for (int k = 0; k < S.len[r]; ++k) {
-        const int cc = S.col[b + 64L * k];
-        u = fmaf(S.val[b + 64L * k], sc[cc] * y[cc], u);
+    const float u = row_product(S, r, p, ys, 0.f);
+    const float dgp = y[e] * w[e] * inv_d[r];
+    const float dcp = (0.5f / sc[r]) * (y[e] * t[e] + w[e] * u);
+    float dg = __shfl(dgp, 0, 4), dc = __shfl(dcp, 0, 4);
+#pragma unroll
+    for (int k = 1; k < kProbes; ++k) {
+        dg += __shfl(dgp, k, 4);
+        dc += __shfl(dcp, k, 4);
     }
-    const float dg = y[r] * w[r] * inv_d[r];
-    const float dc = (0.5f / sc[r]) * (y[r] * t[r] + w[r] * u);
-    dgdc[2 * r] = first ? dg : dgdc[2 * r] + dg;
-    dgdc[2 * r + 1] = first ? dc : dgdc[2 * r + 1] + dc;
+    const float th = tanhf(o[2 * r]);
+    const float s = 1.f / (1.f + expf(-(o[2 * r + 1] + kBeta)));
+    const float d0 = dg * g[r] * 0.5f * (1.f - th * th);
+    const float d1 = dc * kCMax * s * (1.f - s);
+    if (p < LO) dO[2 * r + p] = p ? d1 : d0;
+#pragma unroll
+    for (int j = 0; j < LH / 16; ++j) {
+        const int k = 16 * j + 4 * p;
+        v4f v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = fmaf(d0, w32[OFF_WO + k + i], d1 * w32[OFF_WO + LH + k + i]);
+        *reinterpret_cast<v4f*>(dh + LH * (long)r + k) = v;
+    }
 }
 
 // ---- training: backward through the network (FP32) -------------------------
-__global__ __launch_bounds__(kBlock) void k_lpc_head_bwd(int nu, const float* __restrict__ w32,
-                                                         const float* __restrict__ o,
-                                                         const float* __restrict__ g,
-                                                         const float* __restrict__ dgdc, float* dO,
-                                                         float* dh)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nu) return;
-    const float th = tanhf(o[2 * r]);
-    const float s = 1.f / (1.f + expf(-(o[2 * r + 1] + kBeta)));
-    const float d0 = dgdc[2 * r] * g[r] * 0.5f * (1.f - th * th);
-    const float d1 = dgdc[2 * r + 1] * kCMax * s * (1.f - s);
-    dO[2 * r] = d0;
-    dO[2 * r + 1] = d1;
-    for (int k = 0; k < LH; ++k) dh[LH * (long)r + k] = fmaf(d0, w32[OFF_WO + k], d1 * w32[OFF_WO + LH + k]);
-}
+// dpre = dh * [h > 0] is formed where it is read.
+__device__ __forceinline__ float relu_grad(float dh, uint16_t h) { return bf2f(h) > 0.f ? dh : 0.f; }
 
-// dpre = dh * [h > 0]; for layers >= 1 also dh_prev = dpre U (direct part)
-// and dmh = (dpre V) / sum_k O_rk (the aggregation's input gradient, scaled).
+// dh_prev = dpre U (the direct part) and dmh = (dpre V) / sum_k O_rk (the
+// aggregation's input gradient, scaled) of layer l >= 1: one 16-row tile per
+// wave, 80 output columns, on v_mfma_f32_16x16x4_f32 (operands: lane l holds
+// A[row l%16][k l/16] and B[k l/16][col l%16], D[row 4*(l/16)+i][col l%16]). k is
+// taken so that lane group g holds inputs 16 g .. 16 g + 15: contiguous loads.
+// 14.6k rows 57 (one thread per row, weights read from LDS) -> 7.4 us.
 __global__ __launch_bounds__(kBlock) void k_lpc_dense_bwd(int nu, int l, const uint16_t* __restrict__ w16,
                                                           const uint16_t* __restrict__ h,
                                                           const float* __restrict__ dh,
-                                                          const float* __restrict__ inv_osum,
-                                                          float* dpre, float* dmh, float* dh_prev)
+                                                          const float* __restrict__ inv_osum, float* dmh,
+                                                          float* dh_prev)
 {
-    __shared__ float sU[LH * LH];
-    __shared__ float sV[LH * LM];
-    if (l > 0) {
-        for (int k = threadIdx.x; k < LH * LH; k += kBlock) sU[k] = bf2f(w16[off_U(l) + k]);
-        for (int k = threadIdx.x; k < LH * LM; k += kBlock) sV[k] = bf2f(w16[off_V(l) + k]);
+    constexpr int NC = LH + LM;
+    __shared__ __align__(16) uint16_t wt[NC][LH + 8];  // [output column][input]
+    for (int k = threadIdx.x; k < LH * NC / 8; k += kBlock) {
+        const int o = k / (NC / 8), c = (k % (NC / 8)) * 8;
+        const v8s v = c < LH ? ld8(w16 + off_U(l) + o * LH + c) : ld8(w16 + off_V(l) + o * LM + (c - LH));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) wt[c + i][o] = (uint16_t)v[i];
     }
     __syncthreads();
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nu) return;
-    float dp[LH];
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+    if (row0 >= nu) return;
+    const long in = LH * (long)min(row0 + n, nu - 1) + 16 * g;
+    float dp[16];
 #pragma unroll
-    for (int o = 0; o < LH; ++o) {
-        const float hv = bf2f(h[LH * (long)r + o]);
-        dp[o] = hv > 0.f ? dh[LH * (long)r + o] : 0.f;
-        dpre[LH * (long)r + o] = dp[o];
+    for (int q = 0; q < 4; ++q) {
+        const v4f v = *reinterpret_cast<const v4f*>(dh + in + 4 * q);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dp[4 * q + i] = v[i];
     }
-    if (l == 0) return;
-    for (int k = 0; k < LH; ++k) {
-        float acc = 0.f;
 #pragma unroll
-        for (int o = 0; o < LH; ++o) acc = fmaf(dp[o], sU[o * LH + k], acc);
-        dh_prev[LH * (long)r + k] = acc;
+    for (int q = 0; q < 2; ++q) {
+        const v8s v = ld8(h + in + 8 * q);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dp[8 * q + i] = relu_grad(dp[8 * q + i], (uint16_t)v[i]);
     }
-    const float io = inv_osum[r];
-    for (int j = 0; j < LM; ++j) {
-        float acc = 0.f;
+    for (int nt = 0; nt < NC / 16; ++nt) {
+        v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int o = 0; o < LH; ++o) acc = fmaf(dp[o], sV[o * LM + j], acc);
-        dmh[LM * (long)r + j] = acc * io;
+        for (int q = 0; q < 2; ++q) {
+            const v8s v = *reinterpret_cast<const v8s*>(&wt[16 * nt + n][16 * g + 8 * q]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(dp[8 * q + i], bf2f((uint16_t)v[i]), acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = row0 + 4 * g + i;
+            if (r >= nu) continue;
+            if (nt < LH / 16) dh_prev[LH * (long)r + 16 * nt + n] = acc[i];
+            else dmh[LM * (long)r + n] = acc[i] * inv_osum[r];
+        }
     }
 }
 
-// ds_k = sum_r O_kr dmh_r (transpose of the aggregation; O is symmetric) and
-// dh_prev_k += ds_k P_l.
+// ds_k = sum_r O_kr dmh_r (transpose of the aggregation; O is symmetric), 8
+// lanes per row with 2 of the 16 channels each, and dh_prev_k += ds_k P_l.
+// 14.6k rows 165 (one thread per row) -> 33 us.
 __global__ __launch_bounds__(kBlock) void k_lpc_agg_bwd(int nu, int cap, const int32_t* __restrict__ rowlen,
                                                         const int32_t* __restrict__ acol,
                                                         const float* __restrict__ aval, int l,
@@ -615,95 +707,128 @@ __global__ __launch_bounds__(kBlock) void k_lpc_agg_bwd(int nu, int cap, const i
                                                         const float* __restrict__ dmh, float* ds,
                                                         float* dh_prev)
 {
+    constexpr int R = kBlock / 8;                      // rows of a block
     __shared__ float sP[LM * LH];
+    __shared__ float sd[R][LM];
     for (int k = threadIdx.x; k < LM * LH; k += kBlock) sP[k] = bf2f(w16[off_P(l) + k]);
+    const int q = threadIdx.x & 7, lr = threadIdx.x >> 3;
+    const int row0 = xcd_block() * R, r = row0 + lr;
+    float a0 = 0.f, a1 = 0.f;
+    if (r < nu) {
+        const float2* __restrict__ d = reinterpret_cast<const float2*>(dmh);
+        const long b = mx_index(r, 0, cap);
+        walk_row<8>(acol + b, aval + b, rowlen[r], [&](int c) { return d[8L * c + q]; },
+                    [&](int, float v, float2 x) {
+                        a0 = fmaf(-v, x.x, a0);
+                        a1 = fmaf(-v, x.y, a1);
+                    });
+        *reinterpret_cast<float2*>(ds + LM * (long)r + 2 * q) = make_float2(a0, a1);
+    }
+    sd[lr][2 * q] = a0;
+    sd[lr][2 * q + 1] = a1;
     __syncthreads();
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nu) return;
-    float acc[LM];
+    for (int k = threadIdx.x; k < R * LH; k += kBlock) {
+        const int i = k / LH, c = k % LH;
+        if (row0 + i >= nu) break;
+        float v = dh_prev[LH * (long)(row0 + i) + c];
 #pragma unroll
-    for (int q = 0; q < LM; ++q) acc[q] = 0.f;
-    const long b = mx_index(r, 0, cap);
-    for (int k = 0; k < rowlen[r]; ++k) {
-        const float o = -aval[b + 64L * k];
-        const v4f* p = reinterpret_cast<const v4f*>(dmh + LM * (long)acol[b + 64L * k]);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            const v4f v = p[h];
-            acc[4 * h + 0] = fmaf(o, v.x, acc[4 * h + 0]);
-            acc[4 * h + 1] = fmaf(o, v.y, acc[4 * h + 1]);
-            acc[4 * h + 2] = fmaf(o, v.z, acc[4 * h + 2]);
-            acc[4 * h + 3] = fmaf(o, v.w, acc[4 * h + 3]);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < LM; ++q) ds[LM * (long)r + q] = acc[q];
-    for (int k = 0; k < LH; ++k) {
-        float v = dh_prev[LH * (long)r + k];
-#pragma unroll
-        for (int q = 0; q < LM; ++q) v = fmaf(acc[q], sP[q * LH + k], v);
-        dh_prev[LH * (long)r + k] = v;
+        for (int j = 0; j < LM; ++j) v = fmaf(sd[i][j], sP[j * LH + c], v);
+        dh_prev[LH * (long)(row0 + i) + c] = v;
     }
 }
 
-// Partial sums over a block's rows of X_r (na) outer Y_r (nb): Y is bf16
-// (YK 0), FP32 rounded to bf16 (YK 1) or all ones (YK 2, nb = 1).
-template <int YK>
-__global__ __launch_bounds__(kBlock) void k_lpc_outer(int nu, int na, int nb, const float* __restrict__ X,
-                                                      const void* __restrict__ Yv, float* part)
+// Weight gradients of one layer over a block's rows, all in one launch: sums of
+// outer products of row vectors, matrix products with the graph's rows as the
+// inner index (4 rows an instruction); wave w takes the 16 outputs 16 w .. 16 w
+// + 15. MODE 0: encoder (dpre x features, bias); 1: message layer (dpre x h, dpre
+// x m, bias, ds x h); 2: head (dO x h, bias). Partials in the parameters' order.
+// 14.6k rows, a message layer: four products and their reductions 270 -> 11 us,
+// the one reduction of all layers' partials 50 a product -> 6 us.
+struct WGradArgs {
+    int nu, chunk, layer;
+    const float* __restrict__ dh;          // gradient of the layer's output
+    const uint16_t* __restrict__ hl;       // the layer's output
+    const uint16_t* __restrict__ hp;       // the layer's input
+    const uint16_t* __restrict__ mp;       // and messages
+    const float* __restrict__ ds;
+    const float* __restrict__ feat;
+    float* part;
+};
+
+template <int MODE>
+__global__ __launch_bounds__(kBlock) void k_lpc_wgrad(WGradArgs a)
 {
-    __shared__ float sX[32][LH];
-    __shared__ float sY[32][LH];
-    const int E = na * nb;
-    constexpr int Q = kOuterMax / kBlock;
-    float acc[Q];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, n = lane & 15, g = lane >> 4;
+    const int r0 = blockIdx.x * a.chunk, r1 = min(a.nu, r0 + a.chunk);
+    constexpr int NU = MODE == 1 ? 4 : 1;
+    v4f cu[NU], cv = {0.f, 0.f, 0.f, 0.f}, cp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q] = 0.f;
-    const int chunk = (nu + gridDim.x - 1) / gridDim.x;
-    const int r0 = blockIdx.x * chunk, r1 = min(nu, r0 + chunk);
-    for (int t0 = r0; t0 < r1; t0 += 32) {
-        const int nt = min(32, r1 - t0);
-        for (int k = threadIdx.x; k < 32 * na; k += kBlock) {
-            const int rr = k / na, i = k % na;
-            sX[rr][i] = rr < nt ? X[(long)(t0 + rr) * na + i] : 0.f;
-        }
-        if (YK != 2) {
-            for (int k = threadIdx.x; k < 32 * nb; k += kBlock) {
-                const int rr = k / nb, j = k % nb;
-                float v = 0.f;
-                if (rr < nt) {
-                    if (YK == 0) v = bf2f(reinterpret_cast<const uint16_t*>(Yv)[(long)(t0 + rr) * nb + j]);
-                    else v = bf2f(f2bf(reinterpret_cast<const float*>(Yv)[(long)(t0 + rr) * nb + j]));
-                }
-                sY[rr][j] = v;
-            }
-        }
-        __syncthreads();
+    for (int t = 0; t < NU; ++t) cu[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    float bias = 0.f;
+#pragma unroll 8
+    for (int s = r0; s < r1; s += 4) {
+        const bool ok = s + g < r1;
+        const long r = ok ? s + g : r0;
+        float x;
+        if (MODE == 2) x = a.dh[LO * r + (n & (LO - 1))];
+        else x = relu_grad(a.dh[LH * r + 16 * w + n], a.hl[LH * r + 16 * w + n]);
+        if (!ok || (MODE == 2 && n >= LO)) x = 0.f;
+        bias += x;
+        if (MODE == 0) {
+            float y = bf2f(f2bf(a.feat[LF * r + (n & (LF - 1))]));
+            if (n >= LF) y = 0.f;
+            cu[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, cu[0], 0, 0, 0);
+        } else if (MODE == 2) {
+            cu[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, bf2f(a.hp[LH * r + 16 * w + n]), cu[0], 0, 0, 0);
+        } else {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const int e = threadIdx.x + q * kBlock;
-            if (e < E) {
-                const int i = e / nb, j = e % nb;
-                float s = acc[q];
-                for (int rr = 0; rr < nt; ++rr) s = fmaf(sX[rr][i], YK == 2 ? 1.f : sY[rr][j], s);
-                acc[q] = s;
-            }
+            for (int t = 0; t < NU; ++t)
+                cu[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, bf2f(a.hp[LH * r + 16 * t + n]), cu[t], 0, 0, 0);
+            cv = __builtin_amdgcn_mfma_f32_16x16x4f32(x, bf2f(a.mp[LM * r + n]), cv, 0, 0, 0);
+            float d = a.ds[LM * r + n];
+            if (!ok) d = 0.f;
+            cp = __builtin_amdgcn_mfma_f32_16x16x4f32(d, bf2f(a.hp[LH * r + 16 * w + n]), cp, 0, 0, 0);
         }
-        __syncthreads();
     }
+    bias += __shfl_xor(bias, 16);
+    bias += __shfl_xor(bias, 32);
+    float* __restrict__ p = a.part + (long)blockIdx.x * NPARAM;
+    const int l = a.layer;
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int e = threadIdx.x + q * kBlock;
-        if (e < E) part[(long)blockIdx.x * E + e] = acc[q];
+    for (int i = 0; i < 4; ++i) {
+        const int q = 4 * g + i, o = 16 * w + q;
+        if (MODE == 0) {
+            if (n < LF) p[OFF_W0 + o * LF + n] = cu[0][i];
+        } else if (MODE == 2) {
+            if (q < LO) p[OFF_WO + q * LH + 16 * w + n] = cu[0][i];
+        } else {
+#pragma unroll
+            for (int t = 0; t < NU; ++t) p[off_U(l) + o * LH + 16 * t + n] = cu[t][i];
+            p[off_V(l) + o * LM + n] = cv[i];
+            p[off_P(l) + q * LH + 16 * w + n] = cp[i];
+        }
     }
+    if (g != 0) return;
+    if (MODE == 0) p[OFF_B0 + 16 * w + n] = bias;
+    if (MODE == 1) p[off_c(l) + 16 * w + n] = bias;
+    if (MODE == 2 && w == 0 && n < LO) p[OFF_BO + n] = bias;
 }
 
-__global__ void k_lpc_reduce(int E, int nblk, const float* __restrict__ part, float* out)
+// The gradient: FP64 sums of the blocks' partials, 64 parameters x 16 shares of
+// the blocks a block.
+__global__ __launch_bounds__(1024) void k_lpc_reduce(int nblk, const float* __restrict__ part, float* out)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
+    __shared__ double lds[16][kWave];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int e = blockIdx.x * kWave + lane;
     double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += (double)part[(long)b * E + e];
+    if (e < NPARAM)
+#pragma unroll 4
+        for (int b = w; b < nblk; b += 16) s += (double)part[(long)b * NPARAM + e];
+    lds[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || e >= NPARAM) return;
+    for (int k = 1; k < 16; ++k) s += lds[k][lane];
     out[e] = (float)s;
 }
 
@@ -752,8 +877,9 @@ struct vox_lpc {
     int rows_cap = 0;
     uint16_t *h[4] = {}, *s[3] = {}, *m[3] = {};
     float *o = nullptr, *g = nullptr, *c = nullptr, *sc = nullptr;
-    float *wv = nullptr, *t = nullptr, *z = nullptr, *e = nullptr, *y = nullptr, *dgdc = nullptr,
-          *dO = nullptr, *dh[2] = {}, *dpre = nullptr, *dmh = nullptr, *ds = nullptr;
+    float *wv = nullptr, *vv = nullptr, *t = nullptr, *z = nullptr, *e = nullptr, *y = nullptr,
+          *ys = nullptr, *dO = nullptr, *dh[2] = {}, *dmh = nullptr, *ds = nullptr;
+    double* epart = nullptr;
     long adam_t = 0;
 };
 
@@ -807,29 +933,31 @@ static int lpc_training_buffers(vox_lpc* L, int rows)
     for (auto*& p : L->h) lfree(p);
     for (auto*& p : L->s) lfree(p);
     for (auto*& p : L->m) lfree(p);
-    for (float** p : {&L->o, &L->g, &L->c, &L->sc, &L->wv, &L->t, &L->z, &L->e, &L->y, &L->dgdc, &L->dO,
-                      &L->dh[0], &L->dh[1], &L->dpre, &L->dmh, &L->ds})
+    for (float** p : {&L->o, &L->g, &L->c, &L->sc, &L->wv, &L->vv, &L->t, &L->z, &L->e, &L->y, &L->ys,
+                      &L->dO, &L->dh[0], &L->dh[1], &L->dmh, &L->ds})
         lfree(*p);
+    lfree(L->epart);
     const size_t n = (size_t)rows;
     for (auto*& p : L->h) VOX_TRY(lalloc(&p, n * LH));
     for (auto*& p : L->s) VOX_TRY(lalloc(&p, n * LM));
     for (auto*& p : L->m) VOX_TRY(lalloc(&p, n * LM));
     VOX_TRY(lalloc(&L->o, n * LO));
-    for (float** p : {&L->g, &L->c, &L->sc, &L->wv, &L->t, &L->z, &L->e, &L->y}) VOX_TRY(lalloc(p, n));
-    VOX_TRY(lalloc(&L->dgdc, n * 2));
+    for (float** p : {&L->g, &L->c, &L->sc}) VOX_TRY(lalloc(p, n));
+    for (float** p : {&L->wv, &L->vv, &L->t, &L->z, &L->e, &L->y, &L->ys}) VOX_TRY(lalloc(p, n * kProbes));
+    VOX_TRY(lalloc(&L->epart, (size_t)kProbes * grid_for((long)kProbes * rows)));
     VOX_TRY(lalloc(&L->dO, n * 2));
     VOX_TRY(lalloc(&L->dh[0], n * LH));
     VOX_TRY(lalloc(&L->dh[1], n * LH));
-    VOX_TRY(lalloc(&L->dpre, n * LH));
     VOX_TRY(lalloc(&L->dmh, n * LM));
     VOX_TRY(lalloc(&L->ds, n * LM));
     L->rows_cap = rows;
     return VOX_OK;
 }
 
-// Network forward over `rows` rows (multiple of 64) of a graph with nu rows;
-// h[0..3], s[0..2], m[0..2] may alias as long as layer l's inputs differ from
-// its outputs.
+// Rows from which the aggregation takes 4 lanes a row (fewer instructions an
+// entry) instead of 8 (more waves).
+constexpr int kAggRows = 32768;
+
 // Network forward over `rows` rows (multiple of 64) of a graph with nu rows;
 // h[0..3], s[0..2], m[0..2] may alias as long as layer l's inputs differ from
 // its outputs.
@@ -845,7 +973,8 @@ static int lpc_forward(hipStream_t st, const vox_lpc* L, int rows, AggArgs ag, c
     for (int l = 1; l <= LNL; ++l) {
         ag.s = s[l - 1];
         ag.m = m[l - 1];
-        k_lpc_agg<<<grid_for(ag.nu), kBlock, 0, st>>>(ag);
+        if (ag.nu < kAggRows) k_lpc_agg<8><<<grid_for(8L * ag.nu), kBlock, 0, st>>>(ag);
+        else k_lpc_agg<4><<<grid_for(4L * ag.nu), kBlock, 0, st>>>(ag);
         d.layer = l; d.hin = h[l - 1]; d.min = m[l - 1]; d.hout = h[l];
         d.sout = (l < LNL) ? s[l] : nullptr;
         k_lpc_dense<1><<<nblk, kBlock, 0, st>>>(d);
@@ -865,17 +994,6 @@ static int lpc_forward_sys(vox_lpc* L, const LpcSys& S)
     return VOX_OK;
 }
 
-template <int YK>
-static int outer(vox_lpc* L, int nu, int na, int nb, const float* X, const void* Y, int off)
-{
-    const int nblk = std::max(1, std::min(kOuterBlocks, (nu + 63) / 64));
-    k_lpc_outer<YK><<<nblk, kBlock, 0, L->stream>>>(nu, na, nb, X, Y, L->gpart);
-    const int E = na * nb;
-    k_lpc_reduce<<<grid_for(E), kBlock, 0, L->stream>>>(E, nblk, L->gpart, L->grad + off);
-    VOX_HIP(hipGetLastError());
-    return VOX_OK;
-}
-
 // Loss (into dscal[LS_LOSS]) and gradient (into L->grad) on one system.
 static int lpc_loss_grad_sys(vox_lpc* L, const LpcSys& S, uint64_t seed)
 {
@@ -883,44 +1001,42 @@ static int lpc_loss_grad_sys(vox_lpc* L, const LpcSys& S, uint64_t seed)
     const int nu = S.nu;
     if (grid_for(nu) > kMaxPartials) return fail(VOX_ERR_ARG, "training system too large");
     VOX_TRY(lpc_forward_sys(L, S));
-    k_lpc_set<<<1, 1, 0, st>>>(L->dscal, LS_LOSS, 0.0);
     const OpView SO{nu, S.cap, S.slen, S.scol, S.sval};
     const OpView AO{nu, S.cap, S.rowlen, S.acol, S.aval};
-    const int nb = std::min(kMaxPartials, grid_for(nu));
-    for (int p = 0; p < kProbes; ++p) {
-        k_lpc_probe<<<grid_for(nu), kBlock, 0, st>>>(nu, p, seed, S.rhs, L->wv);
-        k_lpc_dot<<<nb, kBlock, 0, st>>>(nu, L->wv, L->dpart);
-        k_lpc_fin<<<1, kBlock, 0, st>>>(L->dpart, nb, L->dscal, 0);
-        k_lpc_mprobe<<<grid_for(nu), kBlock, 0, st>>>(SO, L->sc, L->g, S.inv_d, L->wv, L->t, L->z);
-        k_lpc_spmv<<<grid_for(nu), kBlock, 0, st>>>(AO, S.diag, L->z, L->wv, L->dscal, L->e, L->dpart);
-        k_lpc_fin<<<1, kBlock, 0, st>>>(L->dpart, grid_for(nu), L->dscal, 1);
-        k_lpc_spmv<<<grid_for(nu), kBlock, 0, st>>>(AO, S.diag, L->e, nullptr, L->dscal, L->y, nullptr);
-        k_lpc_dgc<<<grid_for(nu), kBlock, 0, st>>>(SO, L->sc, S.inv_d, L->wv, L->t, L->y, L->dgdc, p == 0);
-    }
-    k_lpc_head_bwd<<<grid_for(nu), kBlock, 0, st>>>(nu, L->w32, L->o, L->g, L->dgdc, L->dO, L->dh[0]);
+    const int nb = grid_for(nu), nb4 = grid_for((long)kProbes * nu);
+    k_lpc_probe<<<nb, kBlock, 0, st>>>(nu, seed, S.rhs, L->sc, reinterpret_cast<v4f*>(L->wv),
+                                       reinterpret_cast<v4f*>(L->vv), L->dpart);
+    k_lpc_mprobe<<<nb4, kBlock, 0, st>>>(SO, L->sc, L->g, S.inv_d, L->wv, L->vv, L->t, L->z);
+    k_lpc_residual<<<nb4, kBlock, 0, st>>>(AO, S.diag, L->z, L->wv, L->e, L->epart);
+    k_lpc_fin<<<1, kBlock, 0, st>>>(nu, L->dpart, nb, L->epart, nb4, L->dscal);
+    k_lpc_adjoint<<<nb4, kBlock, 0, st>>>(AO, S.diag, L->e, L->sc, L->dscal, L->y, L->ys);
+    k_lpc_dgc<<<nb4, kBlock, 0, st>>>(SO, L->sc, S.inv_d, L->wv, L->t, L->y, L->ys, L->w32, L->o, L->g,
+                                      L->dO, L->dh[0]);
     VOX_HIP(hipGetLastError());
-    VOX_TRY(outer<0>(L, nu, LO, LH, L->dO, L->h[LNL], OFF_WO));
-    VOX_TRY(outer<2>(L, nu, LO, 1, L->dO, nullptr, OFF_BO));
+    // weight gradients: a block sums at least 64 rows, a multiple of 4
+    WGradArgs wg{};
+    wg.nu = nu;
+    wg.chunk = ((std::max(64, (nu + kOuterBlocks - 1) / kOuterBlocks)) + 3) & ~3;
+    wg.part = L->gpart;
+    const int nw = grid_for(nu, wg.chunk);
+    wg.dh = L->dO; wg.hp = L->h[LNL];
+    k_lpc_wgrad<2><<<nw, kBlock, 0, st>>>(wg);
     int cur = 0;
     for (int l = LNL; l >= 1; --l) {
         float* dh = L->dh[cur];
         float* dhp = L->dh[cur ^ 1];
-        k_lpc_dense_bwd<<<grid_for(nu), kBlock, 0, st>>>(nu, l, L->w16, L->h[l], dh, S.inv_osum, L->dpre,
-                                                         L->dmh, dhp);
-        k_lpc_agg_bwd<<<grid_for(nu), kBlock, 0, st>>>(nu, S.cap, S.rowlen, S.acol, S.aval, l, L->w16,
-                                                       L->dmh, L->ds, dhp);
-        VOX_HIP(hipGetLastError());
-        VOX_TRY(outer<0>(L, nu, LH, LH, L->dpre, L->h[l - 1], off_U(l)));
-        VOX_TRY(outer<0>(L, nu, LH, LM, L->dpre, L->m[l - 1], off_V(l)));
-        VOX_TRY(outer<2>(L, nu, LH, 1, L->dpre, nullptr, off_c(l)));
-        VOX_TRY(outer<0>(L, nu, LM, LH, L->ds, L->h[l - 1], off_P(l)));
+        k_lpc_dense_bwd<<<grid_for(nu, 64), kBlock, 0, st>>>(nu, l, L->w16, L->h[l], dh, S.inv_osum, L->dmh,
+                                                             dhp);
+        k_lpc_agg_bwd<<<grid_for(8L * nu), kBlock, 0, st>>>(nu, S.cap, S.rowlen, S.acol, S.aval, l, L->w16,
+                                                            L->dmh, L->ds, dhp);
+        wg.layer = l; wg.dh = dh; wg.hl = L->h[l]; wg.hp = L->h[l - 1]; wg.mp = L->m[l - 1]; wg.ds = L->ds;
+        k_lpc_wgrad<1><<<nw, kBlock, 0, st>>>(wg);
         cur ^= 1;
     }
-    k_lpc_dense_bwd<<<grid_for(nu), kBlock, 0, st>>>(nu, 0, L->w16, L->h[0], L->dh[cur], S.inv_osum,
-                                                     L->dpre, nullptr, nullptr);
+    wg.layer = 0; wg.dh = L->dh[cur]; wg.hl = L->h[0]; wg.feat = S.feat;
+    k_lpc_wgrad<0><<<nw, kBlock, 0, st>>>(wg);
+    k_lpc_reduce<<<grid_for(NPARAM, kWave), 1024, 0, st>>>(nw, L->gpart, L->grad);
     VOX_HIP(hipGetLastError());
-    VOX_TRY(outer<1>(L, nu, LH, LF, L->dpre, S.feat, OFF_W0));
-    VOX_TRY(outer<2>(L, nu, LH, 1, L->dpre, nullptr, OFF_B0));
     return VOX_OK;
 }
 
@@ -979,7 +1095,7 @@ static void ctx_features(vox_ctx* c, int rows, v4f* upos, float* invd, float* fe
     fa.nu = c->nu; fa.cap = c->a_cap; fa.inv_re = (float)(1.0 / c->p.re_l); fa.thr = lpc_threshold(c);
     fa.rowlen = c->rowlen; fa.acol = c->acol; fa.aval = c->aval32; fa.upos = upos; fa.invd = invd;
     fa.feat = feat; fa.inv_osum = inv_osum; fa.slen = slen; fa.scol = scol; fa.sval = sval;
-    k_lpc_features<<<grid_for(c->nu), kBlock, 0, c->stream>>>(fa);
+    k_lpc_features<<<grid_for(4L * c->nu), kBlock, 0, c->stream>>>(fa);
 }
 
 int lpc_prepare(vox_ctx* c)
@@ -1028,7 +1144,7 @@ int lpc_prepare(vox_ctx* c)
     uint16_t* const m[3] = {c->lpc_m, c->lpc_m, c->lpc_m};
     VOX_TRY(lpc_forward(c->stream, c->lpc, frows, ag, c->lpc_feat, h, s, m, c->lpc_o));
     k_lpc_gc_inf<<<grid_for(nu), kBlock, 0, c->stream>>>(nu, c->lpc_o, c->lpc_invd, c->lpc_gd, c->lpc_t);
-    k_lpc_scale<<<grid_for(nu), kBlock, 0, c->stream>>>(nu, c->a_cap, c->lpc_slen, c->lpc_scol, c->lpc_t,
+    k_lpc_scale<<<grid_for(nu, kWave), kBlock, 0, c->stream>>>(nu, c->a_cap, c->lpc_slen, c->lpc_scol, c->lpc_t,
                                                         c->lpc_sval);
     VOX_HIP(hipGetLastError());
     return VOX_OK;
@@ -1054,7 +1170,7 @@ int vox_lpc_create(vox_lpc** out, uint64_t seed)
     int rc;
     if ((rc = lalloc(&L->w32, NPARAM)) || (rc = lalloc(&L->grad, NPARAM)) || (rc = lalloc(&L->am, NPARAM)) ||
         (rc = lalloc(&L->av, NPARAM)) || (rc = lalloc(&L->w16, NPARAM)) ||
-        (rc = lalloc(&L->gpart, (size_t)kOuterBlocks * kOuterMax)) ||
+        (rc = lalloc(&L->gpart, (size_t)kOuterBlocks * NPARAM)) ||
         (rc = lalloc(&L->dpart, (size_t)kMaxPartials)) || (rc = lalloc(&L->dscal, LS_COUNT)))
         return bail(rc);
     if (hipHostMalloc((void**)&L->hscal, sizeof(double) * LS_COUNT, hipHostMallocDefault) != hipSuccess)
@@ -1078,10 +1194,11 @@ int vox_lpc_destroy(vox_lpc* L)
     for (auto*& p : L->h) lfree(p);
     for (auto*& p : L->s) lfree(p);
     for (auto*& p : L->m) lfree(p);
-    for (float** p : {&L->o, &L->g, &L->c, &L->sc, &L->wv, &L->t, &L->z, &L->e, &L->y, &L->dgdc, &L->dO,
-                      &L->dh[0], &L->dh[1], &L->dpre, &L->dmh, &L->ds, &L->w32, &L->grad, &L->am, &L->av,
+    for (float** p : {&L->o, &L->g, &L->c, &L->sc, &L->wv, &L->vv, &L->t, &L->z, &L->e, &L->y, &L->ys,
+                      &L->dO, &L->dh[0], &L->dh[1], &L->dmh, &L->ds, &L->w32, &L->grad, &L->am, &L->av,
                       &L->gpart})
         lfree(*p);
+    lfree(L->epart);
     lfree(L->w16); lfree(L->dpart); lfree(L->dscal);
     if (L->hscal) (void)hipHostFree(L->hscal);
     if (L->stream) (void)hipStreamDestroy(L->stream);
@@ -1230,7 +1347,7 @@ int vox_lpc_train(vox_lpc* L, int32_t epochs, double lr, uint64_t seed, double* 
         for (int k = 0; k < ns; ++k) {
             const int i = order[k];
             VOX_TRY(lpc_loss_grad_sys(L, L->sys[i], seed + (uint64_t)ep * 1000003ull + (uint64_t)i));
-            k_lpc_fin<<<1, kBlock, 0, L->stream>>>(L->dpart, 0, L->dscal, 2);
+            k_lpc_epoch<<<1, 1, 0, L->stream>>>(L->dscal);
             ++L->adam_t;
             const float bc1 = 1.f - std::pow(b1, (float)L->adam_t);
             const float bc2 = 1.f - std::pow(b2, (float)L->adam_t);
