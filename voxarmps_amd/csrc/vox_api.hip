@@ -4,8 +4,11 @@
 // per-stage host routines (functions.cuh:56-111) and vox_step replays the
 // body of its time loop (main.cu:1027-1363) in the same order.
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstring>
 #include <mutex>
+#include <thread>
 
 #include "vox_internal.hpp"
 
@@ -79,10 +82,168 @@ int prof_drain(vox_ctx* c)
     return VOX_OK;
 }
 
-int read_flags(vox_ctx* c)
+// ---- device to host ---------------------------------------------------------
+// Kernels store to pinned host memory and then a signal word, which the host
+// polls: a copy on the stream and a wait for the stream leave the GPU idle for
+// 20 to 35 us, and a step waits four or five times. Ten steps of 1.2k fluid
+// particles 5.1 -> 4.5 ms with it.
+
+// Everything stored by the block before is visible to the host when this is.
+__device__ __forceinline__ void signal_host(uint32_t* sig, uint32_t ticket)
 {
-    VOX_HIP(hipMemcpyAsync(c->hstat, c->dstat, kStatBytes, hipMemcpyDeviceToHost, c->stream));
+    __hip_atomic_store(sig, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kBlock) void k_fetch(const uint32_t* __restrict__ src, uint32_t* dst, int n,
+                                                  uint32_t* sig, uint32_t ticket)
+{
+    for (int k = threadIdx.x; k < n; k += kBlock) dst[k] = src[k];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) signal_host(sig, ticket);
+}
+
+// n 4-byte words in pieces of `piece`, `parts` blocks each; the last block of a
+// piece signals it.
+__global__ __launch_bounds__(kBlock) void k_to_host(const uint32_t* __restrict__ src, uint32_t* dst, long n,
+                                                    int piece, int parts, int32_t* done, uint32_t* sig,
+                                                    uint32_t ticket)
+{
+    const int q = blockIdx.x / parts, part = blockIdx.x % parts, each = piece / parts;
+    const long lo = (long)q * piece + (long)part * each, hi = min(n, lo + each);
+    for (long k = lo + 4 * threadIdx.x; k + 4 <= hi; k += 4 * kBlock)
+        *reinterpret_cast<v4u*>(dst + k) = *reinterpret_cast<const v4u*>(src + k);
+    const long k = (hi & ~3L) + threadIdx.x;           // (each, piece and lo: multiples of 4)
+    if (k >= lo && k < hi) dst[k] = src[k];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(&done[q], 1) == parts - 1) {
+        done[q] = 0;
+        signal_host(sig + q, ticket);
+    }
+}
+
+// Waits until *sig is the ticket: polls for up to a millisecond, then lets the
+// runtime wait for the stream.
+static int await_signal(vox_ctx* c, const uint32_t* sig, uint32_t ticket)
+{
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int k = 1;; ++k) {
+        if (__atomic_load_n(sig, __ATOMIC_ACQUIRE) == ticket) return VOX_OK;
+        __builtin_ia32_pause();
+        if ((k & 255) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) break;
+    }
     VOX_HIP(hipStreamSynchronize(c->stream));
+    if (__atomic_load_n(sig, __ATOMIC_ACQUIRE) != ticket) return fail(VOX_ERR_HIP, "device to host copy");
+    return VOX_OK;
+}
+
+static int fetch(vox_ctx* c, void* dst, const void* src, size_t bytes)
+{
+    const uint32_t ticket = ++c->ticket;
+    k_fetch<<<1, kBlock, 0, c->stream>>>((const uint32_t*)src, (uint32_t*)dst, (int)(bytes / 4), c->hsig, ticket);
+    VOX_HIP(hipGetLastError());
+    return await_signal(c, c->hsig, ticket);
+}
+
+int read_flags(vox_ctx* c) { return fetch(c, c->hstat, c->dstat, kStatBytes); }
+
+int read_i32(vox_ctx* c, const int32_t* src, int32_t* value)
+{
+    VOX_TRY(fetch(c, c->hsig + kSigWord, src, sizeof(int32_t)));
+    *value = (int32_t)c->hsig[kSigWord];
+    return VOX_OK;
+}
+
+// Device memory to the caller's array, through the context's pinned buffer. A
+// copy straight to pageable memory moves it piece by piece with one thread, 17
+// GB/s; here each piece is copied on as soon as it is in the buffer, by up to
+// three threads from 1 MB on. 9.4 MB 524 -> 330 us (420 with one thread; the
+// kernel alone 202), 3.4 MB 193 -> 125, 1.3 MB 78 -> 60, 40 kB 28 -> 13.
+// Memory that the runtime knows already (pinned, managed) is copied to directly.
+constexpr size_t kStageBytes = 16u << 20;              // of a context at most
+constexpr int kParts = 8;                              // blocks a piece
+constexpr size_t kHelpBytes = 1u << 20;
+constexpr int kHelpers = 2;
+constexpr size_t kPiece = kStageBytes / kSigPieces;
+
+static bool stage_ready(vox_ctx* c)
+{
+    HostStage& h = c->stage;
+    if (h.buf) return true;
+    if (h.failed) return false;
+    const size_t want = std::min(kStageBytes, (8 * (size_t)c->tp + 4095) & ~(size_t)4095);
+    if (hipHostMalloc((void**)&h.buf, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        h.buf = nullptr;
+        h.failed = true;                               // direct copies from here on
+        return false;
+    }
+    h.size = want;
+    return true;
+}
+
+// One buffer's worth; every helper has ended when it returns.
+static int stage_pass(vox_ctx* c, char* dst, const char* src, size_t bytes)
+{
+    HostStage& h = c->stage;
+    const int n = (int)((bytes + kPiece - 1) / kPiece);
+    const uint32_t ticket = ++c->ticket;
+    uint32_t* const sig = c->hsig + kSigPiece0;
+    k_to_host<<<n * kParts, kBlock, 0, c->stream>>>((const uint32_t*)src, (uint32_t*)h.buf, (long)(bytes / 4),
+                                                    (int)(kPiece / 4), kParts, c->dpiece, sig, ticket);
+    VOX_HIP(hipGetLastError());
+    auto copy_one = [&](int k) {
+        const size_t o = (size_t)k * kPiece;
+        std::memcpy(dst + o, h.buf + o, std::min(kPiece, bytes - o));
+    };
+    // pieces in the buffer, and the next to copy; n stops the helpers
+    std::atomic<int> there{0}, next{0};
+    auto take = [&]() {                                // copies a piece if there is one
+        int k = next.load();
+        if (k >= there.load(std::memory_order_acquire) || !next.compare_exchange_strong(k, k + 1)) return false;
+        copy_one(k);
+        return true;
+    };
+    auto helper = [&]() {
+        while (next.load() < n)
+            if (!take()) __builtin_ia32_pause();
+    };
+    std::thread help[kHelpers];
+    int nh = 0, rc = VOX_OK;
+    if (bytes >= kHelpBytes) {
+        try {
+            for (; nh < kHelpers; ++nh) help[nh] = std::thread(helper);
+        } catch (...) {                                // with the threads there are
+        }
+    }
+    for (int k = 0; k < n;) {
+        rc = await_signal(c, sig + k, ticket);
+        if (rc != VOX_OK) break;
+        while (k < n && __atomic_load_n(sig + k, __ATOMIC_ACQUIRE) == ticket) ++k;
+        there.store(k, std::memory_order_release);
+        take();
+    }
+    if (rc != VOX_OK) next.store(n);
+    while (next.load() < n) take();
+    for (int k = 0; k < nh; ++k) help[k].join();
+    return rc;
+}
+
+int to_host(vox_ctx* c, void* host, const void* src, size_t bytes)
+{
+    hipPointerAttribute_t at{};
+    const bool pageable = hipPointerGetAttributes(&at, host) != hipSuccess ||
+                          at.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(c->stage.m);
+    if (!pageable || !stage_ready(c)) {
+        VOX_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, c->stream));
+        VOX_HIP(hipStreamSynchronize(c->stream));
+        return VOX_OK;
+    }
+    for (size_t o = 0; o < bytes; o += c->stage.size)
+        VOX_TRY(stage_pass(c, (char*)host + o, (const char*)src + o, std::min(c->stage.size, bytes - o)));
     return VOX_OK;
 }
 
@@ -474,9 +635,11 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
     if ((rc = dalloc(&c->partials, kPartialSlots * (size_t)kMaxPartials)) ||
         (rc = dalloc(&c->dstat, kStatBytes)))
         return bail(rc);
-    if (hipHostMalloc((void**)&c->hstat, kStatBytes, hipHostMallocDefault) != hipSuccess)
+    if ((rc = dalloc(&c->dpiece, (size_t)kSigPieces))) return bail(rc);
+    if (hipHostMalloc((void**)&c->hstat, kStatBytes + 4 * kSigCount, hipHostMallocDefault) != hipSuccess)
         return bail(fail(VOX_ERR_HIP, "hipHostMalloc"));
-    std::memset(c->hstat, 0, kStatBytes);
+    std::memset(c->hstat, 0, kStatBytes + 4 * kSigCount);
+    c->hsig = reinterpret_cast<uint32_t*>(c->hstat + kStatBytes);
     c->dscal = reinterpret_cast<double*>(c->dstat);
     c->dflags = reinterpret_cast<int32_t*>(c->dstat + kStatFlags);
     c->dspread = reinterpret_cast<int32_t*>(c->dstat + kStatSpread);
@@ -484,6 +647,7 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
     c->hflags = reinterpret_cast<int32_t*>(c->hstat + kStatFlags);
     c->hspread = reinterpret_cast<int32_t*>(c->hstat + kStatSpread);
     if (hipDeviceSynchronize() != hipSuccess) return bail(fail(VOX_ERR_HIP, "initial sync"));
+    (void)stage_ready(c);
     *out = c;
     return VOX_OK;
 }
@@ -512,6 +676,8 @@ int vox_destroy(vox_ctx* c)
     dfree(c->scan_blocks); dfree(c->scan_blocks2); dfree(c->partials); dfree(c->dstat);
     lpc_free_ctx(c);
     if (c->hstat) (void)hipHostFree(c->hstat);
+    if (c->stage.buf) (void)hipHostFree(c->stage.buf);
+    dfree(c->dpiece);
     for (auto& r : c->prof_pending) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto e : c->prof_free) (void)hipEventDestroy(e);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
@@ -576,9 +742,7 @@ int vox_download(vox_ctx* c, int field, void* host)
                       : field == VOX_F_BCON ? (const void*)c->bcon
                                             : (const void*)c->f[field];
     size_t bytes = (int_field(field) ? sizeof(int32_t) : sizeof(double)) * (size_t)c->tp;
-    VOX_HIP(hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    VOX_HIP(hipStreamSynchronize(c->stream));
-    return VOX_OK;
+    return to_host(c, host, src, bytes);
 }
 
 int vox_upload_state(vox_ctx* c, const double* x, const double* y, const double* z,

@@ -8,6 +8,8 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -100,6 +102,8 @@ constexpr int kSpreadLine = 32;        // int32 per copy: 128 bytes
 // The status block that read_flags copies to the host in one piece: scalars,
 // flags, spread counters.
 constexpr int kStatFlags = 128, kStatSpread = 256;        // byte offsets
+// signal words after the host's copy of it: status, one fetched word, pieces of a download
+constexpr int kSigWord = 16, kSigPiece0 = 32, kSigPieces = 64, kSigCount = kSigPiece0 + kSigPieces;
 constexpr int kStatBytes = kStatSpread + 4 * kSpread * kSpreadLine;
 
 // device scalar slots of ctx->dscal (double); the solver names its own
@@ -230,11 +234,23 @@ struct ProfRec { int kclass; hipEvent_t a, b; };
 }  // namespace vox
 
 // ---- the context -----------------------------------------------------------------
+// The pinned buffer that downloads go through (to_host).
+struct HostStage {
+    std::mutex m;
+    char* buf = nullptr;
+    size_t size = 0;
+    bool failed = false;           // no buffer to be had
+};
+
 struct vox_ctx {
     vox_params p{};
     int tp = 0, gp = 0, wp = 0, fp = 0;
     int device = 0;
     hipStream_t stream = nullptr;
+    HostStage stage;
+    uint32_t* hsig = nullptr;      // pinned signal words (kSigCount), after hstat
+    std::atomic<uint32_t> ticket{0};   // the last one given out
+    int32_t* dpiece = nullptr;     // blocks done of each piece of a download
 
     double* f[VOX_F_COUNT] = {};
     int32_t* ptype = nullptr;
@@ -450,6 +466,8 @@ int fill_i32(vox_ctx* c, int32_t* p, int32_t v, long n);
 int fill_f64(vox_ctx* c, double* p, double v, long n);
 int read_flags(vox_ctx* c);   // D2H of the status block into its pinned mirror (syncs)
 int32_t spread_max(const vox_ctx* c, int slot);       // of the last read_flags
+int to_host(vox_ctx* c, void* host, const void* src, size_t bytes);   // synchronous
+int read_i32(vox_ctx* c, const int32_t* src, int32_t* value);         // synchronous
 int32_t spread_sum(const vox_ctx* c, int slot);
 
 int autotune_lists(vox_ctx* c, int reps, int32_t* modes);

@@ -873,6 +873,8 @@ struct vox_lpc {
     float *w32 = nullptr, *grad = nullptr, *am = nullptr, *av = nullptr, *gpart = nullptr;
     uint16_t* w16 = nullptr;
     double *dpart = nullptr, *dscal = nullptr, *hscal = nullptr;
+    float* hgrad = nullptr;        // pinned: a pageable copy of the gradient takes 25 us
+    std::mutex hgrad_m;
     std::vector<LpcSys> sys;
     int rows_cap = 0;
     uint16_t *h[4] = {}, *s[3] = {}, *m[3] = {};
@@ -1173,7 +1175,8 @@ int vox_lpc_create(vox_lpc** out, uint64_t seed)
         (rc = lalloc(&L->gpart, (size_t)kOuterBlocks * NPARAM)) ||
         (rc = lalloc(&L->dpart, (size_t)kMaxPartials)) || (rc = lalloc(&L->dscal, LS_COUNT)))
         return bail(rc);
-    if (hipHostMalloc((void**)&L->hscal, sizeof(double) * LS_COUNT, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc((void**)&L->hscal, sizeof(double) * LS_COUNT, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&L->hgrad, sizeof(float) * NPARAM, hipHostMallocDefault) != hipSuccess)
         return bail(fail(VOX_ERR_HIP, "hipHostMalloc"));
     std::vector<float> w;
     init_weights(seed, w);
@@ -1201,6 +1204,7 @@ int vox_lpc_destroy(vox_lpc* L)
     lfree(L->epart);
     lfree(L->w16); lfree(L->dpart); lfree(L->dscal);
     if (L->hscal) (void)hipHostFree(L->hscal);
+    if (L->hgrad) (void)hipHostFree(L->hgrad);
     if (L->stream) (void)hipStreamDestroy(L->stream);
     delete L;
     return VOX_OK;
@@ -1319,8 +1323,10 @@ int vox_lpc_loss_grad(vox_lpc* L, int32_t index, uint64_t seed, double* loss, fl
     VOX_TRY(check_index(L, index));
     VOX_TRY(lpc_loss_grad_sys(L, L->sys[index], seed));
     VOX_HIP(hipMemcpyAsync(L->hscal, L->dscal, sizeof(double) * LS_COUNT, hipMemcpyDeviceToHost, L->stream));
-    if (grad) VOX_HIP(hipMemcpyAsync(grad, L->grad, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, L->stream));
+    std::lock_guard<std::mutex> lock(L->hgrad_m);
+    if (grad) VOX_HIP(hipMemcpyAsync(L->hgrad, L->grad, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, L->stream));
     VOX_HIP(hipStreamSynchronize(L->stream));
+    if (grad) std::memcpy(grad, L->hgrad, sizeof(float) * NPARAM);
     if (loss) *loss = L->hscal[LS_LOSS];
     return VOX_OK;
 }

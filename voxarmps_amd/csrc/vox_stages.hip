@@ -1618,9 +1618,7 @@ int st_collision(vox_ctx* c)
                                                               c->coll_cnt, nullptr, nullptr, 0);
         VOX_TRY(scan_exclusive(c, c->coll_cnt, c->coll_off, n, c->coll_off + n));
         int32_t total = 0;
-        VOX_HIP(hipMemcpyAsync(&total, c->coll_off + n, sizeof(int32_t), hipMemcpyDeviceToHost,
-                               c->stream));
-        VOX_HIP(hipStreamSynchronize(c->stream));
+        VOX_TRY(read_i32(c, c->coll_off + n, &total));
         c->st.collision_cand = total;
         if (total == 0) { c->st.collisions = 0; return VOX_OK; }
         VOX_TRY(coll_reserve(c, total));
