@@ -706,28 +706,32 @@ __global__ __launch_bounds__(BS) void k_prediction_dg(PredArgs a)
 }
 
 // The predictor with 16 lanes per particle, four particles per wave: a lane
-// evaluates one of the row's next 16 entries and each sum adds the lanes' terms
-// in lane order (row16_add), which is the list's; the entries within re_s go to
-// the row's queue in LDS in list order and their gradient terms are added 16 at
-// a time when it fills and at the end. The same bits as the walks above.
+// evaluates one of the row's next 16 entries, its terms go through LDS to the
+// lane that holds their component, which adds them in lane order: the list's.
+// The entries within re_s go to the row's queue in LDS in list order and their
+// gradient terms are added 16 at a time when it fills and at the end. The same
+// bits as the walks above.
 // Why: one thread per particle (188 VGPRs, 2 waves per SIMD) waits for its
-// gathers; the lanes of a row gather records that lie side by side, and a
-// small system still fills the chip. The ordered sums cost 16 multiply-adds
-// each; those weighted with the eddy viscosity are left out where every
-// particle of the wave has none.
-// Measured against the walk of variant 6: 820k rows of 122 entries 1544 us
-// (1690), 103k rows 233 us (324), 2D two-phase of 12k particles 20 us (41), 2D
-// of 3k 6.4 us (31). Bound by the FP64 instructions (73 % of the cycles) and
-// the L1 lookups of the gathers (83 %); records brought to LDS four lanes a
-// record need a third of those lookups and were slower (1690 us, 267 us), and
-// 96 registers for a fifth wave spill (3566 us).
+// gathers; the lanes of a row gather records that lie side by side, and a small
+// system still fills the chip. The sums weighted with the eddy viscosity are left
+// out where every particle of the wave has none.
+// Measured against the walk of variant 6: 820k rows of 222 entries 1472 us
+// (1690), 103k rows 215 us (324), 2D two-phase of 22k particles 20 us (41), 2D of
+// 1.2k 6.6 us (31). At 820k rows bound by the L1 lookups of the gathers (3 a
+// record, 86 % of the cycles). Adding in every lane by lane broadcast: 1545 us,
+// 236 us; with that, records brought to LDS four lanes a record (a third of the
+// lookups) 1690 us, 267 us; 96 registers for a fifth wave spill (3566 us).
 constexpr int kPredSlots = 80;                     // queued entries of a row
 constexpr int kPredStride = kBlock / 16 + 4;       // rows of a slot, padded
+// terms of a wave's four rows: padded so that the twelve sums read 16 bytes each
+// from different banks
+constexpr int kTermsRow = 18, kTermsComp = 4 * kTermsRow, kTermsWave = 3 * kTermsComp;
 
 template <bool kUniform, int KT>
 __global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
 {
     __shared__ int32_t queue[kPredSlots * kPredStride];
+    __shared__ __align__(16) double terms[kBlock / kWave * kTermsWave];
     const int lane = threadIdx.x & (kWave - 1), sub = threadIdx.x & 15, lr = threadIdx.x >> 4;
     const int t = xcd_block() * (kBlock / 16) + lr;
     const bool live = t < a.n;
@@ -749,7 +753,27 @@ __global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
     const double inv_rhoN = 1.0 / rhoN;
     const double inv_re_s = 1.0 / a.re_s, inv_re_l = 1.0 / a.re_l;
     const bool eddy = __any(fluid && nt != 0.0);
-    double s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0, s6 = 0, s7 = 0, s8 = 0, s9 = 0;
+    // lane c of the row (c < dim) holds component c of the sums
+    double sg = 0.0, sl = 0.0, se = 0.0;
+    double* const put = terms + (threadIdx.x >> 6) * kTermsWave + (lane >> 4) * kTermsRow + sub;
+    const double2* const take = reinterpret_cast<const double2*>(put - sub + (sub < 3 ? sub : 0) * kTermsComp);
+    // s + the row's 16 terms of each component, in lane order
+    auto add = [&](double& s, double v0, double v1, double v2) {
+        put[0] = v0;
+        put[kTermsComp] = v1;
+        if (dim == 3) put[2 * kTermsComp] = v2;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (sub < dim) {
+            double2 v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = take[k];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) { s = s + v[k].x; s = s + v[k].y; }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     const unsigned long long seg = 0xffffull << (lane & 48);
     const unsigned long long below = seg & ((1ull << lane) - 1ull);
     int32_t* const gq = queue + lr;
@@ -772,9 +796,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
                 g2 = div_by(div_by(dp * dy * wg, D, inv_D), D, inv_D);
                 g3 = div_by(div_by(dp * dz * wg, D, inv_D), D, inv_D);
             }
-            s1 = row16_add(s1, g1);
-            s2 = row16_add(s2, g2);
-            if (dim == 3) s3 = row16_add(s3, g3);
+            add(sg, g1, g2, g3);
         }
         nq = 0;
         __builtin_amdgcn_wave_barrier();
@@ -814,14 +836,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
         // sum that starts at +0 is never -0)
         const double wl = wfun_h<KT>(D, h, a.ktype, a.re_l, inv_re_l);
         const double tu = wl * (rj.u - ui), tv = wl * (rj.v - vi), tw = wl * (rj.w - wi);
-        s4 = row16_add(s4, use ? tu * NEU : 0.0);
-        s5 = row16_add(s5, use ? tv * NEU : 0.0);
-        if (dim == 3) s6 = row16_add(s6, use ? tw * NEU : 0.0);
-        if (eddy) {
-            s7 = row16_add(s7, use ? tu : 0.0);
-            s8 = row16_add(s8, use ? tv : 0.0);
-            if (dim == 3) s9 = row16_add(s9, use ? tw : 0.0);
-        }
+        add(sl, use ? tu * NEU : 0.0, use ? tv * NEU : 0.0, use ? tw * NEU : 0.0);
+        if (eddy) add(se, use ? tu : 0.0, use ? tv : 0.0, use ? tw : 0.0);
     };
     if (most > 0) {
         // two groups a turn, each group's records on the way during the other
@@ -848,9 +864,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_prediction_l16(PredArgs a)
     // lane c of the row finishes component c (with no eddy viscosity its
     // product is 0 times the other sum: 0, or NaN where that one is not finite)
     if (!fluid || sub >= dim) return;
-    const double sl = (sub == 0) ? s4 : (sub == 1) ? s5 : s6;
-    const double se = !eddy ? sl : (sub == 0) ? s7 : (sub == 1) ? s8 : s9;
-    const double sg = (sub == 0) ? s1 : (sub == 1) ? s2 : s3;
+    if (!eddy) se = sl;
     const double v0 = (sub == 0) ? ui : (sub == 1) ? vi : wi;
     const double x0 = (sub == 0) ? xi : (sub == 1) ? yi : zi;
     const double gr = (sub == 0) ? a.gx : (sub == 1) ? a.gy : a.gz;
