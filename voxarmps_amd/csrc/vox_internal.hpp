@@ -127,8 +127,8 @@ struct DevList {
     int32_t* ids = nullptr;        // sliced rows, entry l of row i at sl_index(i, l, cap)
     int32_t* cell = nullptr;       // tp
     int32_t* cell_start = nullptr; // tnc + 1
-    int32_t* cell_fill = nullptr;  // tnc
-    int32_t* order_raw = nullptr;  // tp (atomic scatter result)
+    int32_t* cell_fill = nullptr;  // tnc: particles of a cell, zero between searches
+    int32_t* order_raw = nullptr;  // tp (ids by cell, unsorted within)
     PosRec* rec = nullptr;         // tp: positions + id sorted by (cell, id)
     bool sorted = false;           // rec holds a sort (a NEIGHBOR call has run)
     long tnc_alloc = 0;
@@ -460,7 +460,8 @@ inline const DevList& list_of(const vox_ctx* c, int which)
 }
 
 // host-side helpers implemented in the .hip files
-int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t* total_dev);
+int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t* total_dev,
+                   int32_t* clear = nullptr);
 int ensure_acol(vox_ctx* c);                                    // vox_ppe.hip
 int fill_i32(vox_ctx* c, int32_t* p, int32_t v, long n);
 int fill_f64(vox_ctx* c, double* p, double v, long n);
