@@ -482,6 +482,84 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
     }
 }
 
+// The same walk with 16 lanes per particle: a run of records is tested 16
+// candidates at a time, the accepted ones keep their order (ballot) and wait in
+// LDS for stores of whole pieces of the row. One thread per particle is a chain
+// of some ten round trips whatever the size; here a chain is a third of that, and
+// a small system has 16 times the waves (kLanesMax2d has the figures).
+constexpr int kRowBuf = 64;                            // accepted ids a row holds in LDS
+constexpr int kRowBufStride = kRowBuf + 1;
+
+__global__ __launch_bounds__(kBlock) void k_build_list_l16(
+    Grid g, int n, double R, const int32_t* __restrict__ start, const PosRec* __restrict__ rec,
+    int cap, int32_t* __restrict__ ids, int32_t* __restrict__ cnt, int32_t* __restrict__ spread,
+    int slot_max)
+{
+    __shared__ int32_t buf_all[kBlock / 16 * kRowBufStride];
+    __shared__ int wmax[kBlock / kWave];
+    const int lane = threadIdx.x & (kWave - 1), sub = threadIdx.x & 15;
+    int32_t* const buf = buf_all + (threadIdx.x >> 4) * kRowBufStride;
+    const int t = xcd_block() * (kBlock / 16) + (threadIdx.x >> 4);
+    const unsigned long long seg = 0xffffull << (lane & 48);
+    const unsigned long long below = seg & ((1ull << lane) - 1ull);
+    int k = 0;
+    if (t < n) {                                       // (uniform in a row of 16 lanes)
+        const PosRec me = rec[t];
+        const int i = me.id;
+        const int ni = inner_cells(g);
+        const int row = me.aux / ni, in = me.aux % ni;
+        const int ix = (g.dim == 3) ? row / g.ncy : row, iy = (g.dim == 3) ? row % g.ncy : 0;
+        const int x1 = max(ix - 1, 0), x2 = min(ix + 1, g.ncx - 1);
+        const int y1 = (g.dim == 3) ? max(iy - 1, 0) : 0;
+        const int y2 = (g.dim == 3) ? min(iy + 1, g.ncy - 1) : 0;
+        const int ny = (g.dim == 3) ? g.ncy : 1, nyb = y2 - y1 + 1, runs = (x2 - x1 + 1) * nyb;
+        const int i1 = max(in - 1, 0), i2 = min(in + 1, ni - 1) + 1;
+        const double R2 = R * R;
+        const double lo = R2 * (1.0 - 1e-10), hi = R2 * (1.0 + 1e-10);
+        int32_t* __restrict__ out = ids + sl_index(i, 0, cap);
+        int stored = 0;
+        auto flush = [&]() {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (int e = stored + sub; e < k; e += 16)
+                if (e < cap) out[((long)(e >> 3) << 9) + (e & 7)] = buf[e - stored];
+            stored = k;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        // lane q holds the bounds of run q (at most 9), all loaded at once
+        const int q = min(sub, runs - 1);
+        const int cn = ((x1 + q / nyb) * ny + y1 + q % nyb) * ni;
+        const int qs = start[cn + i1], qe = start[cn + i2];
+        for (int r = 0; r < runs; ++r) {
+            const int s = __shfl(qs, r, 16), e = __shfl(qe, r, 16);
+            for (int j0 = s; j0 < e; j0 += 16) {
+                const PosRec cu = rec[min(j0 + sub, e - 1)];
+                const double dx = cu.x - me.x, dy = cu.y - me.y, dz = cu.z - me.z;
+                const double d2 = dx * dx + dy * dy + dz * dz;
+                bool acc = d2 < lo;
+                if (!acc && !(d2 > hi))                // rare band: exact sqrt decides
+                    acc = g.incl ? (sqrt(d2) <= R) : (sqrt(d2) < R);
+                acc = acc && (j0 + sub < e) && (g.incl || cu.id != i);
+                const unsigned long long m = __ballot(acc) & seg;
+                if (acc) buf[k - stored + __popcll(m & below)] = cu.id;
+                k += __popcll(m);
+                if (k - stored > kRowBuf - 16) flush();
+            }
+        }
+        flush();
+        if (sub == 0) cnt[i] = k;
+    }
+    const int m = wave_max_i32(k);
+    if (lane == 0) wmax[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int b = wmax[0];
+        for (int w = 1; w < kBlock / kWave; ++w) b = max(b, wmax[w]);
+        atomicMax(spread_at(spread, slot_max), b);
+    }
+}
+
 // Stencil walk for cells that hold many particles (3D list L: 64-80 a cell),
 // on the matrix cores. A wave takes 64 consecutive particles of the
 // cell-sorted order: one or a few cells of one row of cells along the innermost
@@ -888,6 +966,17 @@ static int launch_one(vox_ctx* c, int which, double re)
     return search_one(c, which, re);
 }
 
+// The walk per particle takes 16 lanes up to this many particles. NEIGHBOR calls,
+// one thread and 16 lanes, us: 2D 2k particles 42 / 31, 26k 53 / 44, 69k 54 / 50,
+// 250k 78 / 92; 3D 15k 135 / 56, 61k 145 / 109, 201k 309 / 260, 485k 561 / 574.
+constexpr int kLanesMax2d = 1 << 16, kLanesMax3d = 1 << 18;
+// and against the matrix cores up to this many (16 lanes, matrix): 10k 69 / 171,
+// 43k 134 / 196, 94k 229 / 238, 133k 304 / 244 at 4 spacings, 149 / 176 and 193 /
+// 195 for the last two at 3.1. Half as many for list L, whose consumers read the
+// rows of positions that only the matrix walk stores faster (steps, 16 lanes and
+// matrix: 25k 790 / 832 us, 61k 1070 / 1063, 94k 1261 / 1220).
+constexpr int kLanesMaxMm = 3 << 15;
+
 // One search pass over the sorted cells of list `which` (rows at the list's
 // current capacity), on c->stream.
 static int search_one(vox_ctx* c, int which, double re)
@@ -903,7 +992,8 @@ static int search_one(vox_ctx* c, int which, double re)
     L.compact = compact;
     L.epoch = c->pos_epoch;
     // The matrix-core walk where a cell is expected (cell volume / DL^dim) to
-    // hold 24 particles or more, else the walk per particle. NEIGHBOR calls
+    // hold 24 particles or more and the system fills the chip with it, else the
+    // walk per particle (here by one thread). NEIGHBOR calls
     // measured with either, matrix against per particle, us: 3D 67 a cell 1500
     // against 2480 (1,185,000 particles), 330 against 590 (201,000), 200 against
     // 270 (15,500); 35 a cell 1005 / 1420, 250 / 370, 170 / 190; 10 a cell 650 /
@@ -912,7 +1002,8 @@ static int search_one(vox_ctx* c, int which, double re)
         ? L.g.hx * L.g.hx * L.g.hz / (c->p.dl * c->p.dl * c->p.dl)
         : L.g.hx * L.g.hx / (c->p.dl * c->p.dl);
     const int mode = c->tuned_mode[which] ? c->tuned_mode[which] : c->p.list_mode;
-    const bool cell_walk = (mode == 2 || (mode == 0 && per_cell >= 24.0));
+    const bool cell_walk = (mode == 2 || (mode == 0 && per_cell >= 24.0 &&
+                                          n > (compact ? kLanesMaxMm / 2 : kLanesMaxMm)));
     ProfScope ps(c, which == 0 ? KC_LIST : KC_LIST_L);
     // Compact rows of the cell walk hold positions in the cell-sorted records
     // (and sit at the particle's position): their consumers gather from
@@ -926,6 +1017,9 @@ static int search_one(vox_ctx* c, int which, double re)
         else
             k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
                 gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
+    } else if (n <= (c->p.dim == 3 ? kLanesMax3d : kLanesMax2d)) {
+        k_build_list_l16<<<grid_for(16L * n), kBlock, 0, c->stream>>>(
+            gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
     } else {
         k_build_list<<<grid_for(n), kBlock, 0, c->stream>>>(gg, n, R, L.cell_start, L.rec, L.cap,
                                                             L.ids, L.cnt, c->dspread, sm);
