@@ -169,7 +169,8 @@ typedef struct vox_status {
     int32_t product_col_bytes;/* bytes per column the last PPE product read: 2
                                  (16-bit steps or window ranks) or 4           */
     int32_t product_window_cols; /* columns the last product staged in its LDS
-                                 windows, summed over its blocks (0: none)     */
+                                 windows, summed over its blocks (0: none); all
+                                 unknowns where one block runs a whole solve   */
 } vox_status;
 
 typedef struct vox_ctx vox_ctx;

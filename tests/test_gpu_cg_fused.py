@@ -3,7 +3,8 @@ direction) against the three-kernel form: the same bits, iteration counts and
 residuals, when the solve stops at its limit after 1, 2 or 3 iterations, is
 read every iteration or in batches, starts warm, refines in mixed precision, has
 a zero right-hand side, or takes the learned preconditioner. Product variant 0
-is the one form, 4 the other; sizes lie around whole blocks of rows."""
+is the one form (for the smaller 2D systems the whole solve in one block), 4 the
+other; sizes lie around whole blocks of rows and the one block's limits."""
 import numpy as np
 import pytest
 
@@ -29,7 +30,7 @@ def _same(a, b, what):
     assert np.array_equal(a[1], b[1], equal_nan=True) and a[3] == b[3], what
 
 
-@pytest.mark.parametrize("shape", [(10, 10, 0), (16, 16, 0), (31, 33, 0), (8, 8, 8), (20, 13, 11)],
+@pytest.mark.parametrize("shape", [(10, 10, 0), (16, 16, 0), (31, 33, 0), (33, 31, 0), (40, 48, 0), (48, 48, 0), (8, 8, 8), (20, 13, 11)],
                          ids=str)
 @pytest.mark.parametrize("precision", [vx._abi.PREC_FP64, vx._abi.PREC_MIXED], ids=["fp64", "mixed"])
 def test_fused_and_plain_iterations_agree(hip, shape, precision):

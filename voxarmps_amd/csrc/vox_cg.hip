@@ -634,6 +634,160 @@ __global__ __launch_bounds__(kWave) void k_cg_test(CgArgs<VT, MT> a)
     cg_goes_on(a, wave_partials<8>(PSLOT(a, P_RR), a.nvb), a.it, threadIdx.x == 0);
 }
 
+// ---- a whole solve in one block -------------------------------------------------------
+// Small systems: three launches an iteration cost 15 us whatever their size, an
+// iteration of this kernel the time in which one CU reads the matrix (64 bytes a
+// cycle) and two reductions. Rows t and t + 1024 belong to thread t, p is in LDS,
+// columns come as 16-bit steps; every sum is formed as by the kernels above (256
+// rows a product block, 1024 a vector block), so the solve is the same bits.
+// (Both rows' entries loaded together measured the same, 12 % slower on systems
+// of one row a thread; one_block has the figures.)
+constexpr int kOneRows = 2 * kVecThreads;
+constexpr int kOnePq = kOneRows / kBlock;              // product blocks
+constexpr int kMaxOneParts = kOnePq > 2 ? kOnePq : 2;
+static_assert(kOnePq <= kVecThreads / kWave, "a wave per product block");
+
+// block_sum_n's value of the `NT` terms from v[0] on, in every lane of a wave.
+template <int NT>
+__device__ __forceinline__ double wave_sum_of(const double* v)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    double w[NT / kWave];
+#pragma unroll
+    for (int j = 0; j < NT / kWave; ++j) w[j] = v[lane + kWave * j];
+#pragma unroll
+    for (int h = NT / kWave / 2; h > 0; h >>= 1)
+#pragma unroll
+        for (int j = 0; j < h; ++j) w[j] = w[j] + w[j + h];
+    return wave_tree(w[0]);
+}
+
+template <class VT, class MT>
+__global__ __launch_bounds__(kVecThreads) void k_cg_one(CgArgs<VT, MT> a)
+{
+    __shared__ VT pv[kOneRows];
+    __shared__ double ta[kOneRows], tb[kOneRows];      // terms of two sums
+    __shared__ double part[2][kMaxOneParts];
+    const int t = threadIdx.x, wave = t >> 6, lane = t & (kWave - 1);
+    // sum of the first `n` partials of a slot, as wave_partials does it
+    auto total = [&](int slot, int n) {
+        const double s = wave_tree(0.0 + (lane < n ? part[slot][lane] : 0.0));
+        return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(s)),
+                                __builtin_amdgcn_readfirstlane(__double2loint(s)));
+    };
+    // the vector blocks' sums of ta and tb
+    auto vec_sums = [&](double& sa, double& sb) {
+        __syncthreads();
+        if (wave < 4) {
+            const double s = wave_sum_of<kVecThreads>(((wave & 1) ? tb : ta) + (wave >> 1) * kVecThreads);
+            if (lane == 0) part[wave & 1][wave >> 1] = s;
+        }
+        __syncthreads();
+        sa = total(0, a.nvb);
+        sb = total(1, a.nvb);
+    };
+    double d[2], nz[2];
+    VT x[2], r[2], z[2], p[2];
+    int len[2], base[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int row = t + h * kVecThreads;
+        const bool on = row < a.nu;
+        const double b = on ? a.rhs[row] : 0.0;
+        d[h] = on ? a.diag[row] : 1.0;
+        len[h] = on ? a.rowlen[row] : 0;
+        base[h] = len[h] > 0 ? a.cbase[row] : 0;
+        x[h] = (VT)0;
+        r[h] = (VT)b;
+        z[h] = p[h] = r[h] / (VT)d[h];
+        ta[row] = on ? 0.0 + b * b : 0.0;
+        tb[row] = on ? 0.0 + (double)r[h] * (double)z[h] : 0.0;
+        nz[h] = on ? (double)(len[h] + 1) : 0.0;
+        pv[row] = p[h];
+    }
+    double bb, rz, nnz, none;
+    vec_sums(bb, rz);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) ta[t + h * kVecThreads] = nz[h];
+    vec_sums(nnz, none);
+    const double bn = sqrt(bb);
+    if (t == 0) cg_start(a, bn, rz, nnz);
+    for (int it = 1; bn != 0.0 && it <= a.maxit; ++it) {
+        VT q[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int row = t + h * kVecThreads;
+            VT acc = (VT)d[h] * p[h];
+            const v4u* __restrict__ dc = a.dcol + dc_index(row, 0, a.cap);
+            const MT* __restrict__ val = a.aval + mx_index(row, 0, a.cap);
+            int cj = base[h];
+            for (int k = 0; k < len[h]; k += 8) {
+                const v4u w = dc[8L * k];
+                MT vv[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) vv[u] = val[64L * min(k + u, len[h] - 1)];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (k + u < len[h]) {
+                        cj += u16_of(w, u);
+                        acc = acc + (VT)vv[u] * pv[cj];
+                    }
+            }
+            q[h] = acc;
+            ta[row] = row < a.nu ? (double)p[h] * (double)acc : 0.0;
+        }
+        __syncthreads();
+        if (wave < kOnePq) {
+            const double s = wave_sum_of<kBlock>(ta + wave * kBlock);
+            if (lane == 0) part[0][wave] = s;
+        }
+        __syncthreads();
+        const double pq = total(0, a.npq);
+        if (!(pq > 0.0) || !isfinite(pq)) {
+            if (t == 0) {
+                a.flags[FLAG_CG_BREAK] = 1;
+                a.flags[FLAG_CG_DONE] = 1;
+                a.flags[FLAG_CG_ITERS] = it - 1;
+            }
+            break;
+        }
+        const VT alpha = (VT)(rz / pq);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int row = t + h * kVecThreads;
+            x[h] = x[h] + alpha * p[h];
+            r[h] = r[h] - alpha * q[h];
+            z[h] = r[h] / (VT)d[h];
+            const bool on = row < a.nu;
+            ta[row] = on ? 0.0 + (double)r[h] * (double)r[h] : 0.0;
+            tb[row] = on ? 0.0 + (double)r[h] * (double)z[h] : 0.0;
+        }
+        double rr, rzn;
+        vec_sums(rr, rzn);
+        const double rel = sqrt(rr) / bn;
+        const bool conv = rel <= a.tol, stop = it >= a.maxit || !isfinite(rel);
+        if (t == 0) {
+            a.scal[S_RELRES] = rel;
+            a.flags[FLAG_CG_ITERS] = it;
+            if (conv) a.flags[FLAG_CG_CONV] = 1;
+            if (conv || stop) a.flags[FLAG_CG_DONE] = 1;
+        }
+        if (conv || stop) break;
+        const VT beta = (VT)(rzn / rz);
+        rz = rzn;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            p[h] = z[h] + beta * p[h];
+            pv[t + h * kVecThreads] = p[h];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        if (t + h * kVecThreads < a.nu) a.x[t + h * kVecThreads] = x[h];
+}
+
 // ---- flexible CG ---------------------------------------------------------------------------
 template <class VT, class MT>
 __global__ __launch_bounds__(kVecThreads) void k_fcg_init(CgArgs<VT, MT> a)
@@ -953,6 +1107,21 @@ __global__ void k_scatter_x(int nu, const int32_t* __restrict__ urow, const doub
 }
 
 // ---- host ------------------------------------------------------------------------------------
+// Whether Jacobi-CG runs in one block (k_cg_one): few and short rows, a matrix that
+// one CU reads in the time the launches of an iteration take. Solves of 12
+// iterations, three kernels and one block: 2D 107 rows 121 -> 88 us, 744 rows 140
+// -> 98, 1421 rows of 26 entries 156 -> 139 (2443 rows of 34: 177 both), and no LDS
+// windows to build, 40 us a step; mixed precision 744 rows 285 -> 167, 1421 rows 297
+// -> 204; 3D rows of 97 entries, 179 rows 130 -> 188, so rows are bounded too. Ten
+// steps of 1.2k fluid particles 4.5 -> 3.9 ms.
+constexpr long kOneEntries = 1L << 17;
+constexpr int kOneRowCap = 96;
+static bool one_block(const vox_ctx* c)
+{
+    return c->tune_spmv == 0 && c->dcol_ok && c->nu > 0 && c->nu <= kOneRows &&
+           c->a_cap <= kOneRowCap && (long)c->nu * c->a_cap <= kOneEntries;
+}
+
 // Whether the products update p (k_cg_spmv_win). Measured per solve of 11 to 14
 // iterations, without and with: 2D rows 0.9k 192 -> 176 us, 12k 221 -> 180, 80k
 // 226 -> 194, 377k 449 -> 405; 3D rows 64k 617 -> 578, 139k 1028 -> 1010, 179k to
@@ -1026,6 +1195,20 @@ static void next_direction(CgArgs<VT, MT>& a, VT* const buf[2])
 template <class VT, class MT>
 static int run_cg(vox_ctx* c, CgArgs<VT, MT>& a, int* iters_out)
 {
+    if (one_block(c)) {
+        c->st.product_col_bytes = 2;
+        c->st.product_window_cols = c->nu;             // all of p is in LDS
+        a.z = nullptr;
+        {
+            ProfScope ps(c, KC_SPMV);
+            k_cg_one<VT, MT><<<1, kVecThreads, 0, c->stream>>>(a);
+            VOX_HIP(hipGetLastError());
+        }
+        VOX_TRY(read_flags(c));
+        c->nnz_total = (long)c->hscal[S_NNZ];
+        *iters_out = c->hflags[FLAG_CG_ITERS];
+        return VOX_OK;
+    }
     // the products that gather from LDS windows update p themselves
     const bool fused = updates_p(c, a);
     VT* const buf[2] = {a.p, reinterpret_cast<VT*>(c->cg_pn)};
@@ -1189,8 +1372,9 @@ static int ensure_window(vox_ctx* c)
 
 // The windows when the product variant in use (or being timed) reads them,
 // and the 32-bit columns when it reads those.
-static int prepare_product(vox_ctx* c, bool all_variants = false)
+static int prepare_product(vox_ctx* c, bool all_variants = false, bool fcg = false)
 {
+    if (!all_variants && !fcg && one_block(c)) return VOX_OK;
     const int v = c->tune_spmv;
     if (all_variants || v == 1 || v == 2 || v == 3 || !c->dcol_ok) VOX_TRY(ensure_acol(c));
     if (all_variants || v == 0) return ensure_window(c);
@@ -1243,7 +1427,7 @@ static int finish(vox_ctx* c, vox_solve_info* info, int iters, int conv, double 
 
 static int solve_fp64(vox_ctx* c, vox_solve_info* info, bool fcg, int maxit)
 {
-    VOX_TRY(prepare_product(c));
+    VOX_TRY(prepare_product(c, false, fcg));
     CgArgs<double, double> a;
     fill_args(c, a, (const double*)c->aval, c->cg_x, c->cg_r, c->cg_p, c->cg_q, c->rhs,
               c->p.cg_tol, maxit);
@@ -1304,7 +1488,7 @@ static int solve_refined(vox_ctx* c, vox_solve_info* info, const MT* aval, VT* x
     const int nu = c->nu;
     const int npq = grid_for(nu > 0 ? nu : 1);
     if (npq > kMaxPartials) return fail(VOX_ERR_ARG, "PPE larger than the solver's row limit");
-    VOX_TRY(prepare_product(c));
+    VOX_TRY(prepare_product(c, false, fcg));
     if (warm && nu > 0) {
         k_gather_x0<<<grid_for(nu), kBlock, 0, c->stream>>>(nu, c->urow, c->f[VOX_F_P], c->cg_x);
         VOX_HIP(hipGetLastError());
