@@ -531,12 +531,12 @@ namespace vox {
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.
 // This remap hands every XCD one contiguous range of logical blocks, so the
 // spatially adjacent particles of neighbouring blocks share an L2.
-__device__ __forceinline__ int xcd_block()
+__device__ __forceinline__ int xcd_block_of(int nb, int b)
 {
-    const int nb = gridDim.x, b = blockIdx.x;
     const int q = nb >> 3, r = nb & 7, x = b & 7;
     return x * q + min(x, r) + (b >> 3);
 }
+__device__ __forceinline__ int xcd_block() { return xcd_block_of(gridDim.x, blockIdx.x); }
 __device__ __forceinline__ int xcd_tid() { return xcd_block() * blockDim.x + threadIdx.x; }
 
 
