@@ -54,6 +54,46 @@ __global__ void k_pack_pos(int n, int dim, const double* __restrict__ x,
     rec[i] = r;
 }
 
+// The row walks of the lighter stages come in two forms: one thread per particle,
+// and for small systems 16 lanes per particle, where a lane evaluates one of the
+// row's next 16 entries and every sum adds the lanes' terms in lane order (the
+// row's; an entry that is left out adds +0, which changes no bit of a sum that
+// starts at +0). One thread per particle is a chain of some six round trips
+// whatever the size. The figures are at kStageLanes2d.
+struct LaneRow {
+    int i, sub;                                        // particle, lane of its row
+    bool live;
+};
+__device__ __forceinline__ LaneRow lane_row(int first, int n)
+{
+    const int i = first + xcd_block() * (kBlock / 16) + (int)(threadIdx.x >> 4);
+    return {i < n ? i : first, (int)(threadIdx.x & 15), i < n};
+}
+// f(j, in) for the entries of a row (`self`'s, cnt of them) 16 at a time, j == self
+// and in == false beyond its end; every lane of the wave takes part.
+template <class F>
+__device__ __forceinline__ void walk16(const ListView& L, int self, int cnt, int sub, F f)
+{
+    const int most = row16_max(cnt);
+    const int32_t* __restrict__ row = L.ids + sl_index(self, 0, L.cap) + sl_step(sub);
+    int j = sub < cnt ? row[0] : self;
+    for (int g = 0; g < most; g += 16) {
+        row += 1024;
+        const int jn = g + 16 + sub < cnt ? row[0] : self;
+        f(j, g + sub < cnt);
+        j = jn;
+    }
+}
+// Up to this many particles 16 lanes take one. Stages (with their packing), one
+// thread and 16 lanes, us. PNUM / SPS / VISCOSITY (Herschel-Bulkley) / PRESSGRAD: 2D
+// 2k particles 10.6 23 12.3 13.7 / 10.9 10.7 6.4 10.8, 26k 10.8 24 12.8 13.9 / 10.9
+// 14.6 12.3 11.1, 69k 12.6 29 16.5 16.4 / 11.8 29 23.5 16.5; 3D 15k 21 122 71 32 /
+// 10.9 22 23 10.9, 61k 23 124 74 33 / 20 65 63 17, 201k 52 225 168 54 / 51 212 190
+// 50, 485k 88 411 312 113 / 113 516 432 117.
+constexpr int kStageLanes2d = 3 << 14, kStageLanes3d = 1 << 17;
+static bool by_lanes(int dim, long n) { return n <= (dim == 3 ? kStageLanes3d : kStageLanes2d); }
+static int lane_blocks(long n) { return grid_for(16 * n); }
+
 // n_i = sum over the row of W(d_ij), j != i, in row order. Branch-free per
 // entry with 8 record loads in flight; the 3-term distance equals the 2D one
 // bit for bit (dz = 0).
@@ -98,6 +138,30 @@ __global__ __launch_bounds__(kBlock) void k_pnd(int n, int ktype, double re, dou
     if (pnew) pnew[i] = p[i];
 }
 
+__global__ __launch_bounds__(kBlock) void k_pnd_l16(int n, int ktype, double re, double ncorr,
+                                                    ListView L, const PosRec* __restrict__ rec,
+                                                    const int32_t* __restrict__ self_of,
+                                                    double* __restrict__ out,
+                                                    const double* __restrict__ p,
+                                                    double* __restrict__ pnew)
+{
+    const LaneRow r = lane_row(0, n);
+    const int self = self_of ? self_of[r.i] : r.i;
+    const PosRec me = rec[self];
+    const double inv_re = 1.0 / re;
+    double sum = 0.0;
+    walk16(L, self, r.live ? L.cnt[self] : 0, r.sub, [&](int j, bool in) {
+        const PosRec q = rec[j];
+        const double dx = q.x - me.x, dy = q.y - me.y, dz = q.z - me.z;
+        const double w = wfun_r(sqrt(dx * dx + dy * dy + dz * dz), ktype, re, inv_re);
+        sum = row16_add(sum, (in && j != self) ? w : 0.0);
+    });
+    if (!r.live || r.sub != 0) return;
+    if (ktype != 2) sum = sum * ncorr;
+    out[r.i] = sum;
+    if (pnew) pnew[r.i] = p[r.i];
+}
+
 // Rows of positions (list L's compact rows) index the list's own sorted
 // records, which hold the positions of its search: the caller passes those
 // positions (n0 right after NEIGHBOR).
@@ -115,9 +179,13 @@ static void launch_pnd(vox_ctx* c, const DevList& L, double re, double ncorr, co
     // (a kernel specialised on the kernel type holds fewer registers, runs
     // more waves and measured 11% slower: the gathers then share the caches
     // among more rows)
-    k_pnd<<<grid_for(c->tp), kBlock, 0, c->stream>>>(c->tp, c->p.ktype, re, ncorr,
-                                                      ListView{L.cnt, L.ids, L.cap}, rec, self_of,
-                                                      out, p, pnew);
+    if (by_lanes(c->p.dim, c->tp))
+        k_pnd_l16<<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(
+            c->tp, c->p.ktype, re, ncorr, ListView{L.cnt, L.ids, L.cap}, rec, self_of, out, p, pnew);
+    else
+        k_pnd<<<grid_for(c->tp), kBlock, 0, c->stream>>>(c->tp, c->p.ktype, re, ncorr,
+                                                          ListView{L.cnt, L.ids, L.cap}, rec, self_of,
+                                                          out, p, pnew);
 }
 
 int st_pnd(vox_ctx* c, int on_star, int loopstarted)
@@ -165,6 +233,25 @@ int st_n0(vox_ctx* c)
 // ---- strain rate: SPS functions.cu:1738-1790, VISCOSITY 2095-2150 ---------------------------------
 struct Strain { double s11, s12, s22, s13, s23, s33; };
 
+__device__ __forceinline__ Strain strain_of(int dim, double n0, double s1, double s2, double s3, double s4,
+                                            double s5, double s6, double s7, double s8, double s9)
+{
+    double Uxx = (2.0 / n0) * s1, Uyy = (2.0 / n0) * s2, Uxy = (2.0 / n0) * s3, Uyx = (2.0 / n0) * s4;
+    Strain S;
+    S.s12 = 0.5 * (Uxy + Uyx);
+    S.s11 = 0.5 * (Uxx + Uxx);
+    S.s22 = 0.5 * (Uyy + Uyy);
+    S.s13 = S.s23 = S.s33 = 0.0;
+    if (dim == 3) {
+        double Uzz = (2.0 / n0) * s5, Uxz = (2.0 / n0) * s6, Uyz = (2.0 / n0) * s7;
+        double Uzx = (2.0 / n0) * s8, Uzy = (2.0 / n0) * s9;
+        S.s33 = 0.5 * (Uzz + Uzz);
+        S.s13 = 0.5 * (Uxz + Uzx);
+        S.s23 = 0.5 * (Uyz + Uzy);
+    }
+    return S;
+}
+
 __device__ __forceinline__ Strain strain_row(int i, int dim, int ktype, double re, double n0,
                                              double dmin, bool use_dmin, ListView L,
                                              const double* __restrict__ x,
@@ -207,20 +294,43 @@ __device__ __forceinline__ Strain strain_row(int i, int dim, int ktype, double r
             }
         }
     }
-    double Uxx = (2.0 / n0) * s1, Uyy = (2.0 / n0) * s2, Uxy = (2.0 / n0) * s3, Uyx = (2.0 / n0) * s4;
-    Strain S;
-    S.s12 = 0.5 * (Uxy + Uyx);
-    S.s11 = 0.5 * (Uxx + Uxx);
-    S.s22 = 0.5 * (Uyy + Uyy);
-    S.s13 = S.s23 = S.s33 = 0.0;
-    if (dim == 3) {
-        double Uzz = (2.0 / n0) * s5, Uxz = (2.0 / n0) * s6, Uyz = (2.0 / n0) * s7;
-        double Uzx = (2.0 / n0) * s8, Uzy = (2.0 / n0) * s9;
-        S.s33 = 0.5 * (Uzz + Uzz);
-        S.s13 = 0.5 * (Uxz + Uzx);
-        S.s23 = 0.5 * (Uyz + Uzy);
-    }
-    return S;
+    return strain_of(dim, n0, s1, s2, s3, s4, s5, s6, s7, s8, s9);
+}
+// The same by the 16 lanes of a row (every lane gets the sums).
+__device__ __forceinline__ Strain strain_row16(int i, int cnt, int sub, int dim, int ktype, double re,
+                                               double n0, double dmin, bool use_dmin, const ListView& L,
+                                               const double* __restrict__ x,
+                                               const double* __restrict__ y,
+                                               const double* __restrict__ z,
+                                               const double* __restrict__ u,
+                                               const double* __restrict__ v,
+                                               const double* __restrict__ w)
+{
+    const double xi = x[i], yi = y[i], zi = (dim == 3) ? z[i] : 0.0;
+    const double ui = u[i], vi = v[i], wi = (dim == 3) ? w[i] : 0.0;
+    double s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0, s6 = 0, s7 = 0, s8 = 0, s9 = 0;
+    walk16(L, i, cnt, sub, [&](int j, bool in) {
+        const double dx = x[j] - xi, dy = y[j] - yi;
+        double dz = 0.0, d;
+        if (dim == 3) { dz = z[j] - zi; d = sqrt(dx * dx + dy * dy + dz * dz); }
+        else d = sqrt(dx * dx + dy * dy);
+        const bool use = in && j != i && !(use_dmin && !(d > dmin));
+        const double wv = wfun(d, ktype, re);
+        const double du = u[j] - ui, dv = v[j] - vi;
+        s1 = row16_add(s1, use ? du * dx * wv / d / d : 0.0);
+        s2 = row16_add(s2, use ? dv * dy * wv / d / d : 0.0);
+        s3 = row16_add(s3, use ? du * dy * wv / d / d : 0.0);
+        s4 = row16_add(s4, use ? dv * dx * wv / d / d : 0.0);
+        if (dim == 3) {
+            const double dw = w[j] - wi;
+            s5 = row16_add(s5, use ? dw * dz * wv / d / d : 0.0);
+            s6 = row16_add(s6, use ? du * dz * wv / d / d : 0.0);
+            s7 = row16_add(s7, use ? dv * dz * wv / d / d : 0.0);
+            s8 = row16_add(s8, use ? dw * dx * wv / d / d : 0.0);
+            s9 = row16_add(s9, use ? dw * dy * wv / d / d : 0.0);
+        }
+    });
+    return strain_of(dim, n0, s1, s2, s3, s4, s5, s6, s7, s8, s9);
 }
 
 // ---- SPS: functions.cu:1719-1841 -------------------------------------------------------------
@@ -232,12 +342,22 @@ struct SpsArgs {
     double *s11, *s12, *s22, *s13, *s23, *s33, *neut, *t1, *t2, *t3;
 };
 
+template <bool kLanes>
 __global__ __launch_bounds__(kBlock) void k_sps1(SpsArgs a)
 {
-    int i = a.first + xcd_tid();
-    if (i >= a.n) return;
-    Strain S = strain_row(i, a.dim, a.ktype, a.re, a.n0, a.dmin, true, a.L, a.x, a.y, a.z, a.u,
-                          a.v, a.w);
+    int i;
+    Strain S;
+    if constexpr (kLanes) {
+        const LaneRow r = lane_row(a.first, a.n);
+        i = r.i;
+        S = strain_row16(i, r.live ? a.L.cnt[i] : 0, r.sub, a.dim, a.ktype, a.re, a.n0, a.dmin, true, a.L,
+                         a.x, a.y, a.z, a.u, a.v, a.w);
+        if (!r.live || r.sub != 0) return;
+    } else {
+        i = a.first + xcd_tid();
+        if (i >= a.n) return;
+        S = strain_row(i, a.dim, a.ktype, a.re, a.n0, a.dmin, true, a.L, a.x, a.y, a.z, a.u, a.v, a.w);
+    }
     a.s11[i] = S.s11; a.s12[i] = S.s12; a.s22[i] = S.s22;
     a.s13[i] = S.s13; a.s23[i] = S.s23; a.s33[i] = S.s33;
     double s = sqrt(2 * S.s11 * S.s11) + 2 * sqrt(2 * S.s12 * S.s12) + sqrt(2 * S.s22 * S.s22);
@@ -246,31 +366,52 @@ __global__ __launch_bounds__(kBlock) void k_sps1(SpsArgs a)
     a.neut[i] = a.csdl2 * s;
 }
 
+template <bool kLanes>
 __global__ __launch_bounds__(kBlock) void k_sps2(SpsArgs a)
 {
-    int i = a.first + xcd_tid();
-    if (i >= a.n) return;
-    double xi = a.x[i], yi = a.y[i], zi = (a.dim == 3) ? a.z[i] : 0.0, ni = a.neut[i];
+    int i;
     double s1 = 0, s2 = 0, s3 = 0;
-    int cnt = a.L.cnt[i];
-    const int32_t* __restrict__ rowp = a.L.ids + sl_index(i, 0, a.L.cap);
-    for (int g = 0; (g << 3) < cnt; ++g) {
-        int32_t jc[8];
-        load_chunk8(rowp, g, jc);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            if ((g << 3) + e >= cnt) break;
-            int j = jc[e];
-            if (j == i) continue;
-            double dx = a.x[j] - xi, dy = a.y[j] - yi, dz = 0.0, d;
+    if constexpr (kLanes) {
+        const LaneRow r = lane_row(a.first, a.n);
+        i = r.i;
+        const double xi = a.x[i], yi = a.y[i], zi = (a.dim == 3) ? a.z[i] : 0.0, ni = a.neut[i];
+        walk16(a.L, i, r.live ? a.L.cnt[i] : 0, r.sub, [&](int j, bool in) {
+            const double dx = a.x[j] - xi, dy = a.y[j] - yi;
+            double dz = 0.0, d;
             if (a.dim == 3) { dz = a.z[j] - zi; d = sqrt(dx * dx + dy * dy + dz * dz); }
             else d = sqrt(dx * dx + dy * dy);
-            if (!(d > a.dmin)) continue;
-            double wv = wfun(d, a.ktype, a.re);
-            double dn = a.neut[j] - ni;
-            s1 = s1 + dn * dx * wv / d / d;
-            s2 = s2 + dn * dy * wv / d / d;
-            if (a.dim == 3) s3 = s3 + dn * dz * wv / d / d;
+            const bool use = in && j != i && d > a.dmin;
+            const double wv = wfun(d, a.ktype, a.re);
+            const double dn = a.neut[j] - ni;
+            s1 = row16_add(s1, use ? dn * dx * wv / d / d : 0.0);
+            s2 = row16_add(s2, use ? dn * dy * wv / d / d : 0.0);
+            if (a.dim == 3) s3 = row16_add(s3, use ? dn * dz * wv / d / d : 0.0);
+        });
+        if (!r.live || r.sub != 0) return;
+    } else {
+        i = a.first + xcd_tid();
+        if (i >= a.n) return;
+        double xi = a.x[i], yi = a.y[i], zi = (a.dim == 3) ? a.z[i] : 0.0, ni = a.neut[i];
+        int cnt = a.L.cnt[i];
+        const int32_t* __restrict__ rowp = a.L.ids + sl_index(i, 0, a.L.cap);
+        for (int g = 0; (g << 3) < cnt; ++g) {
+            int32_t jc[8];
+            load_chunk8(rowp, g, jc);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if ((g << 3) + e >= cnt) break;
+                int j = jc[e];
+                if (j == i) continue;
+                double dx = a.x[j] - xi, dy = a.y[j] - yi, dz = 0.0, d;
+                if (a.dim == 3) { dz = a.z[j] - zi; d = sqrt(dx * dx + dy * dy + dz * dz); }
+                else d = sqrt(dx * dx + dy * dy);
+                if (!(d > a.dmin)) continue;
+                double wv = wfun(d, a.ktype, a.re);
+                double dn = a.neut[j] - ni;
+                s1 = s1 + dn * dx * wv / d / d;
+                s2 = s2 + dn * dy * wv / d / d;
+                if (a.dim == 3) s3 = s3 + dn * dz * wv / d / d;
+            }
         }
     }
     double s11 = a.s11[i], s12 = a.s12[i], s22 = a.s22[i];
@@ -302,8 +443,13 @@ int st_sps(vox_ctx* c)
     a.t1 = c->f[VOX_F_TURB1]; a.t2 = c->f[VOX_F_TURB2]; a.t3 = c->f[VOX_F_TURB3];
     int m = c->tp - c->gp;
     if (m <= 0) return VOX_OK;
-    k_sps1<<<grid_for(m), kBlock, 0, c->stream>>>(a);
-    k_sps2<<<grid_for(m), kBlock, 0, c->stream>>>(a);
+    if (by_lanes(a.dim, m)) {
+        k_sps1<true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
+        k_sps2<true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
+    } else {
+        k_sps1<false><<<grid_for(m), kBlock, 0, c->stream>>>(a);
+        k_sps2<false><<<grid_for(m), kBlock, 0, c->stream>>>(a);
+    }
     VOX_HIP(hipGetLastError());
     return VOX_OK;
 }
@@ -342,6 +488,30 @@ __global__ __launch_bounds__(kBlock) void k_vfraction(int n, int dim, int ktype,
     C[i] = cv;
 }
 
+__global__ __launch_bounds__(kBlock) void k_vfraction_l16(int n, int dim, int ktype, double re,
+                                                          ListView L, const int32_t* __restrict__ pt,
+                                                          const double* __restrict__ x,
+                                                          const double* __restrict__ y,
+                                                          const double* __restrict__ z,
+                                                          double* __restrict__ C)
+{
+    const LaneRow r = lane_row(0, n);
+    const int i = r.i;
+    const double xi = x[i], yi = y[i], zi = (dim == 3) ? z[i] : 0.0;
+    double s1 = 0, s2 = 0;
+    walk16(L, i, r.live ? L.cnt[i] : 0, r.sub, [&](int j, bool in) {
+        const int tj = pt[j];
+        const bool use = in && j != i && tj > 0;
+        const double wv = wfun(pdist(dim, x, y, z, i, j, xi, yi, zi), ktype, re);
+        s1 = row16_add(s1, use ? wv : 0.0);
+        s2 = row16_add(s2, (use && tj == 2) ? wv : 0.0);
+    });
+    if (!r.live || r.sub != 0) return;
+    double cv = s2 / s1;
+    if (s1 == 0) cv = 0;
+    C[i] = cv;
+}
+
 int st_vfraction(vox_ctx* c)
 {
     ProfScope ps(c, KC_VFRAC);
@@ -349,7 +519,12 @@ int st_vfraction(vox_ctx* c)
     // is 0 / s1 = +0 (or the s1 == 0 case, also +0): the same bits as the walk.
     if (c->n_fluid2 == 0) return fill_f64(c, c->f[VOX_F_C], 0.0, c->tp);
     if (c->p.precision == VOX_PREC_MIXED) return st_vfraction32(c);
-    k_vfraction<<<grid_for(c->tp), kBlock, 0, c->stream>>>(
+    if (by_lanes(c->p.dim, c->tp))
+        k_vfraction_l16<<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(
+            c->tp, c->p.dim, c->p.ktype, c->p.re_s, view(c, VOX_LIST_S), c->ptype, c->f[VOX_F_X],
+            c->f[VOX_F_Y], c->f[VOX_F_Z], c->f[VOX_F_C]);
+    else
+        k_vfraction<<<grid_for(c->tp), kBlock, 0, c->stream>>>(
         c->tp, c->p.dim, c->p.ktype, c->p.re_s, view(c, VOX_LIST_S), c->ptype, c->f[VOX_F_X],
         c->f[VOX_F_Y], c->f[VOX_F_Z], c->f[VOX_F_C]);
     VOX_HIP(hipGetLastError());
@@ -376,13 +551,25 @@ struct HbArgs {
     double* meu;
 };
 
+template <bool kLanes>
 __global__ __launch_bounds__(kBlock) void k_visc_hb(HbArgs a)
 {
-    int i = xcd_tid();
-    if (i >= a.n) return;
-    if (a.pt[i] == 1) { a.meu[i] = a.m1; return; }
-    Strain S = strain_row(i, a.dim, a.ktype, a.re, a.n0, 0.0, false, a.L, a.x, a.y, a.z, a.u, a.v,
-                          a.w);
+    int i;
+    Strain S;
+    if constexpr (kLanes) {
+        const LaneRow r = lane_row(0, a.n);
+        i = r.i;
+        const bool other = a.pt[i] != 1;
+        S = strain_row16(i, (r.live && other) ? a.L.cnt[i] : 0, r.sub, a.dim, a.ktype, a.re, a.n0, 0.0, false,
+                         a.L, a.x, a.y, a.z, a.u, a.v, a.w);
+        if (!r.live || r.sub != 0) return;
+        if (!other) { a.meu[i] = a.m1; return; }
+    } else {
+        i = xcd_tid();
+        if (i >= a.n) return;
+        if (a.pt[i] == 1) { a.meu[i] = a.m1; return; }
+        S = strain_row(i, a.dim, a.ktype, a.re, a.n0, 0.0, false, a.L, a.x, a.y, a.z, a.u, a.v, a.w);
+    }
     // phi reads C[I] with the caller's I == 0 (main.cu:211): always phi = 0 (2154-2155)
     double cz = 0.0;
     double phi = (cz - 0.25) * a.phi_param / (1 - 0.25);
@@ -417,7 +604,8 @@ int st_viscosity(vox_ctx* c)
         a.x = c->f[VOX_F_X]; a.y = c->f[VOX_F_Y]; a.z = c->f[VOX_F_Z];
         a.u = c->f[VOX_F_UNEW]; a.v = c->f[VOX_F_VNEW]; a.w = c->f[VOX_F_WNEW];
         a.phat = c->f[VOX_F_PHAT]; a.meu = c->f[VOX_F_MEU];
-        k_visc_hb<<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
+        if (by_lanes(c->p.dim, c->tp)) k_visc_hb<true><<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(a);
+        else k_visc_hb<false><<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
     }
     VOX_HIP(hipGetLastError());
     return VOX_OK;
@@ -1076,44 +1264,65 @@ __global__ void k_pack_grad(GradArgs a)
 
 // Branch-free per entry with 8 records in flight; the 3-term distance equals
 // the 2D one bit for bit, and the z sum is only read in 3D.
-template <int KT>
+template <int KT, bool kLanes>
 __global__ __launch_bounds__(kBlock) void k_pressgrad(GradArgs a)
 {
-    int i = a.first + xcd_tid();
-    if (i >= a.n) return;
+    int i;
     const int dim = a.dim;
-    const GradRec me = a.rec[i];
-    const double xi = me.x, yi = me.y, zi = me.z, pi_ = me.pn, phi_ = me.ph;
     double s1 = 0, s2 = 0, s3 = 0;
     const double inv_re = 1.0 / a.re;
-    int cnt = a.L.cnt[i];
-    const int32_t* __restrict__ rowp = a.L.ids + sl_index(i, 0, a.L.cap);
-    for (int g = 0; (g << 3) < cnt; ++g) {
-        int32_t jc[8];
-        load_chunk8(rowp, g, jc);
-        double px[8], py[8], pz[8], pp[8], ph[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) jc[e] = ((g << 3) + e < cnt) ? jc[e] : i;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const GradRec* r = a.rec + jc[e];
-            px[e] = r->x; py[e] = r->y; pz[e] = r->z; pp[e] = r->pn; ph[e] = r->ph;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool use = (jc[e] != i);
-            const double dx = px[e] - xi, dy = py[e] - yi, dz = pz[e] - zi;
+    // kh 1: p_j + p_i - (p^_i + p^_j) (functions.cu:275-278); kh 2, the
+    // reference's CUDA kernel: p_j + p_i - 2 p^_i (382-385); kh 0: p_j - p^_i
+    auto pressure = [&](double pj, double phj, double pi_, double phi_) {
+        return (a.kh == 1) ? (pj + pi_ - (phi_ + phj)) : (a.kh == 2) ? (pj + pi_ - 2.0 * phi_) : (pj - phi_);
+    };
+    if constexpr (kLanes) {
+        const LaneRow r = lane_row(a.first, a.n);
+        i = r.i;
+        const GradRec me = a.rec[i];
+        walk16(a.L, i, r.live ? a.L.cnt[i] : 0, r.sub, [&](int j, bool in) {
+            const GradRec q = a.rec[j];
+            const bool use = in && j != i;
+            const double dx = q.x - me.x, dy = q.y - me.y, dz = q.z - me.z;
             const double D = sqrt(dx * dx + dy * dy + dz * dz);
             const double wv = wfun_k<KT>(D, a.ktype, a.re, inv_re);
-            // kh 1: p_j + p_i - (p^_i + p^_j) (functions.cu:275-278); kh 2, the
-            // reference's CUDA kernel: p_j + p_i - 2 p^_i (382-385); kh 0: p_j - p^_i
-            const double dp = (a.kh == 1)   ? (pp[e] + pi_ - (phi_ + ph[e]))
-                              : (a.kh == 2) ? (pp[e] + pi_ - 2.0 * phi_)
-                                            : (pp[e] - phi_);
-            const double inv_D = 1.0 / D;                 // x / D / D via div_by
-            s1 = use ? s1 + div_by(div_by(dp * dx * wv, D, inv_D), D, inv_D) : s1;
-            s2 = use ? s2 + div_by(div_by(dp * dy * wv, D, inv_D), D, inv_D) : s2;
-            s3 = use ? s3 + div_by(div_by(dp * dz * wv, D, inv_D), D, inv_D) : s3;
+            const double dp = pressure(q.pn, q.ph, me.pn, me.ph);
+            const double inv_D = 1.0 / D;                     // x / D / D via div_by
+            s1 = row16_add(s1, use ? div_by(div_by(dp * dx * wv, D, inv_D), D, inv_D) : 0.0);
+            s2 = row16_add(s2, use ? div_by(div_by(dp * dy * wv, D, inv_D), D, inv_D) : 0.0);
+            if (dim == 3) s3 = row16_add(s3, use ? div_by(div_by(dp * dz * wv, D, inv_D), D, inv_D) : 0.0);
+        });
+        if (!r.live || r.sub != 0) return;
+    } else {
+        i = a.first + xcd_tid();
+        if (i >= a.n) return;
+        const GradRec me = a.rec[i];
+        const double xi = me.x, yi = me.y, zi = me.z, pi_ = me.pn, phi_ = me.ph;
+        int cnt = a.L.cnt[i];
+        const int32_t* __restrict__ rowp = a.L.ids + sl_index(i, 0, a.L.cap);
+        for (int g = 0; (g << 3) < cnt; ++g) {
+            int32_t jc[8];
+            load_chunk8(rowp, g, jc);
+            double px[8], py[8], pz[8], pp[8], ph[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) jc[e] = ((g << 3) + e < cnt) ? jc[e] : i;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const GradRec* r = a.rec + jc[e];
+                px[e] = r->x; py[e] = r->y; pz[e] = r->z; pp[e] = r->pn; ph[e] = r->ph;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool use = (jc[e] != i);
+                const double dx = px[e] - xi, dy = py[e] - yi, dz = pz[e] - zi;
+                const double D = sqrt(dx * dx + dy * dy + dz * dz);
+                const double wv = wfun_k<KT>(D, a.ktype, a.re, inv_re);
+                const double dp = pressure(pp[e], ph[e], pi_, phi_);
+                const double inv_D = 1.0 / D;                 // x / D / D via div_by
+                s1 = use ? s1 + div_by(div_by(dp * dx * wv, D, inv_D), D, inv_D) : s1;
+                s2 = use ? s2 + div_by(div_by(dp * dy * wv, D, inv_D), D, inv_D) : s2;
+                s3 = use ? s3 + div_by(div_by(dp * dz * wv, D, inv_D), D, inv_D) : s3;
+            }
         }
     }
     double g = a.relaxp * (a.gnum * a.dt / a.n0 / a.rho[i]);
@@ -1151,10 +1360,15 @@ int st_pressgrad(vox_ctx* c)
     int m = c->tp - a.first;
     if (m <= 0) return VOX_OK;
     k_pack_grad<<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
+    auto go = [&](auto kt) {
+        constexpr int KT = decltype(kt)::value;
+        if (by_lanes(a.dim, m)) k_pressgrad<KT, true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
+        else k_pressgrad<KT, false><<<grid_for(m), kBlock, 0, c->stream>>>(a);
+    };
     switch (kt_of(a.ktype)) {
-    case 2: k_pressgrad<2><<<grid_for(m), kBlock, 0, c->stream>>>(a); break;
-    case 6: k_pressgrad<6><<<grid_for(m), kBlock, 0, c->stream>>>(a); break;
-    default: k_pressgrad<0><<<grid_for(m), kBlock, 0, c->stream>>>(a); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    default: go(std::integral_constant<int, 0>{}); break;
     }
     VOX_HIP(hipGetLastError());
     return VOX_OK;
@@ -1296,6 +1510,32 @@ __global__ __launch_bounds__(kBlock) void k_coll_screen(int n, double rc, ListVi
         }
     }
     if (!off) cnt[i] = k;
+}
+
+__global__ __launch_bounds__(kBlock) void k_coll_screen_l16(int n, double rc, ListView L,
+                                                            const PosRec* __restrict__ rec,
+                                                            const int32_t* __restrict__ off,
+                                                            int32_t* __restrict__ cnt,
+                                                            int32_t* __restrict__ ci,
+                                                            int32_t* __restrict__ cj, long cap)
+{
+    const LaneRow r = lane_row(0, n);
+    const int lane = threadIdx.x & (kWave - 1);
+    const unsigned long long seg = 0xffffull << (lane & 48);
+    const unsigned long long below = seg & ((1ull << lane) - 1ull);
+    const PosRec me = rec[r.i];
+    const long pos = off ? off[r.i] : 0;
+    int k = 0;
+    walk16(L, r.i, r.live ? L.cnt[r.i] : 0, r.sub, [&](int j, bool in) {
+        const PosRec q = rec[j];
+        const double dx = q.x - me.x, dy = q.y - me.y, dz = q.z - me.z;
+        const bool hit = in && j != r.i && sqrt(dx * dx + dy * dy + dz * dz) < rc;
+        const unsigned long long m = __ballot(hit);
+        const long at = pos + k + __popcll(m & below);
+        if (hit && off && at < cap) { ci[at] = r.i; cj[at] = j; }
+        k += __popcll(m & seg);
+    });
+    if (r.live && r.sub == 0 && !off) cnt[r.i] = k;
 }
 
 struct CollArgs {
@@ -1628,17 +1868,27 @@ int st_collision(vox_ctx* c)
         const bool every_pair = p.coll + margin > list_r;
         const double rc = every_pair ? HUGE_VAL : p.coll + margin;
         k_pack_pos<<<grid_for(n), kBlock, 0, c->stream>>>(n, p.dim, X, Y, Z, c->pos_rec);
-        k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
-                                                              c->coll_cnt, nullptr, nullptr, 0);
+        const bool lanes = by_lanes(p.dim, n);
+        if (lanes)
+            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
+                                                                        c->coll_cnt, nullptr, nullptr, 0);
+        else
+            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
+                                                                  c->coll_cnt, nullptr, nullptr, 0);
         VOX_TRY(scan_exclusive(c, c->coll_cnt, c->coll_off, n, c->coll_off + n));
         int32_t total = 0;
         VOX_TRY(read_i32(c, c->coll_off + n, &total));
         c->st.collision_cand = total;
         if (total == 0) { c->st.collisions = 0; return VOX_OK; }
         VOX_TRY(coll_reserve(c, total));
-        k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, c->coll_off,
-                                                              nullptr, c->coll_i, c->coll_j,
-                                                              c->coll_cap);
+        if (lanes)
+            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, c->coll_off,
+                                                                        nullptr, c->coll_i, c->coll_j,
+                                                                        c->coll_cap);
+        else
+            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, c->coll_off,
+                                                                  nullptr, c->coll_i, c->coll_j,
+                                                                  c->coll_cap);
         CollArgs a;
         a.dim = p.dim; a.coll = p.coll; a.cc = p.cc; a.rho1 = p.rho1; a.rho2 = p.rho2; a.dt = p.dt;
         a.half_margin = every_pair ? HUGE_VAL : 0.45 * margin;
