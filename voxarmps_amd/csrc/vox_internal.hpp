@@ -460,6 +460,12 @@ inline const DevList& list_of(const vox_ctx* c, int which)
 }
 
 // host-side helpers implemented in the .hip files
+// Entries expected in a row of radius re at spacing dl.
+inline double row_entries(const vox_params& p, double re)
+{
+    const double k = re / p.dl;
+    return p.dim == 3 ? 4.19 * k * k * k : 3.14 * k * k;
+}
 int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t* total_dev,
                    int32_t* clear = nullptr);
 int ensure_acol(vox_ctx* c);                                    // vox_ppe.hip

@@ -969,6 +969,8 @@ static int launch_one(vox_ctx* c, int which, double re)
 // The walk per particle takes 16 lanes up to this many particles. NEIGHBOR calls,
 // one thread and 16 lanes, us: 2D 2k particles 42 / 31, 26k 53 / 44, 69k 54 / 50,
 // 250k 78 / 92; 3D 15k 135 / 56, 61k 145 / 109, 201k 309 / 260, 485k 561 / 574.
+// (in 2D twice as many where rows are longer than one group of 16: five weakly
+// compressible steps of 69k particles at 4 spacings 1360 -> 1320 us).
 constexpr int kLanesMax2d = 1 << 16, kLanesMax3d = 1 << 18;
 // and against the matrix cores up to this many (16 lanes, matrix): 10k 69 / 171,
 // 43k 134 / 196, 94k 229 / 238, 133k 304 / 244 at 4 spacings, 149 / 176 and 193 /
@@ -1017,7 +1019,7 @@ static int search_one(vox_ctx* c, int which, double re)
         else
             k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
                 gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
-    } else if (n <= (c->p.dim == 3 ? kLanesMax3d : kLanesMax2d)) {
+    } else if (n <= (c->p.dim == 3 ? kLanesMax3d : kLanesMax2d * (row_entries(c->p, re) > 16.0 ? 2 : 1))) {
         k_build_list_l16<<<grid_for(16L * n), kBlock, 0, c->stream>>>(
             gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
     } else {

@@ -59,7 +59,7 @@ __global__ void k_pack_pos(int n, int dim, const double* __restrict__ x,
 // row's next 16 entries and every sum adds the lanes' terms in lane order (the
 // row's; an entry that is left out adds +0, which changes no bit of a sum that
 // starts at +0). One thread per particle is a chain of some six round trips
-// whatever the size. The figures are at kStageLanes2d.
+// whatever the size. The figures are at kStageLanesShort.
 struct LaneRow {
     int i, sub;                                        // particle, lane of its row
     bool live;
@@ -90,8 +90,14 @@ __device__ __forceinline__ void walk16(const ListView& L, int self, int cnt, int
 // 14.6 12.3 11.1, 69k 12.6 29 16.5 16.4 / 11.8 29 23.5 16.5; 3D 15k 21 122 71 32 /
 // 10.9 22 23 10.9, 61k 23 124 74 33 / 20 65 63 17, 201k 52 225 168 54 / 51 212 190
 // 50, 485k 88 411 312 113 / 113 516 432 117.
-constexpr int kStageLanes2d = 3 << 14, kStageLanes3d = 1 << 17;
-static bool by_lanes(int dim, long n) { return n <= (dim == 3 ? kStageLanes3d : kStageLanes2d); }
+// Rows of one group of 16 (13 entries: 2D at 2.1 spacings) end earlier than longer
+// ones (37: 3D at 2.1, 50: 2D at 4; five weakly compressible 2D steps of 69k 1360 ->
+// 1240 us).
+constexpr int kStageLanesShort = 3 << 14, kStageLanesLong = 1 << 17;
+static bool by_lanes(const vox_params& p, double re, long n)
+{
+    return n <= (row_entries(p, re) > 16.0 ? kStageLanesLong : kStageLanesShort);
+}
 static int lane_blocks(long n) { return grid_for(16 * n); }
 
 // n_i = sum over the row of W(d_ij), j != i, in row order. Branch-free per
@@ -179,7 +185,7 @@ static void launch_pnd(vox_ctx* c, const DevList& L, double re, double ncorr, co
     // (a kernel specialised on the kernel type holds fewer registers, runs
     // more waves and measured 11% slower: the gathers then share the caches
     // among more rows)
-    if (by_lanes(c->p.dim, c->tp))
+    if (by_lanes(c->p, re, c->tp))
         k_pnd_l16<<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(
             c->tp, c->p.ktype, re, ncorr, ListView{L.cnt, L.ids, L.cap}, rec, self_of, out, p, pnew);
     else
@@ -443,7 +449,7 @@ int st_sps(vox_ctx* c)
     a.t1 = c->f[VOX_F_TURB1]; a.t2 = c->f[VOX_F_TURB2]; a.t3 = c->f[VOX_F_TURB3];
     int m = c->tp - c->gp;
     if (m <= 0) return VOX_OK;
-    if (by_lanes(a.dim, m)) {
+    if (by_lanes(c->p, c->p.re_s, m)) {
         k_sps1<true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
         k_sps2<true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
     } else {
@@ -519,7 +525,7 @@ int st_vfraction(vox_ctx* c)
     // is 0 / s1 = +0 (or the s1 == 0 case, also +0): the same bits as the walk.
     if (c->n_fluid2 == 0) return fill_f64(c, c->f[VOX_F_C], 0.0, c->tp);
     if (c->p.precision == VOX_PREC_MIXED) return st_vfraction32(c);
-    if (by_lanes(c->p.dim, c->tp))
+    if (by_lanes(c->p, c->p.re_s, c->tp))
         k_vfraction_l16<<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(
             c->tp, c->p.dim, c->p.ktype, c->p.re_s, view(c, VOX_LIST_S), c->ptype, c->f[VOX_F_X],
             c->f[VOX_F_Y], c->f[VOX_F_Z], c->f[VOX_F_C]);
@@ -604,7 +610,7 @@ int st_viscosity(vox_ctx* c)
         a.x = c->f[VOX_F_X]; a.y = c->f[VOX_F_Y]; a.z = c->f[VOX_F_Z];
         a.u = c->f[VOX_F_UNEW]; a.v = c->f[VOX_F_VNEW]; a.w = c->f[VOX_F_WNEW];
         a.phat = c->f[VOX_F_PHAT]; a.meu = c->f[VOX_F_MEU];
-        if (by_lanes(c->p.dim, c->tp)) k_visc_hb<true><<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(a);
+        if (by_lanes(c->p, c->p.re_s, c->tp)) k_visc_hb<true><<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(a);
         else k_visc_hb<false><<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
     }
     VOX_HIP(hipGetLastError());
@@ -1362,7 +1368,7 @@ int st_pressgrad(vox_ctx* c)
     k_pack_grad<<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
     auto go = [&](auto kt) {
         constexpr int KT = decltype(kt)::value;
-        if (by_lanes(a.dim, m)) k_pressgrad<KT, true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
+        if (by_lanes(c->p, c->p.re_s, m)) k_pressgrad<KT, true><<<lane_blocks(m), kBlock, 0, c->stream>>>(a);
         else k_pressgrad<KT, false><<<grid_for(m), kBlock, 0, c->stream>>>(a);
     };
     switch (kt_of(a.ktype)) {
@@ -1868,7 +1874,7 @@ int st_collision(vox_ctx* c)
         const bool every_pair = p.coll + margin > list_r;
         const double rc = every_pair ? HUGE_VAL : p.coll + margin;
         k_pack_pos<<<grid_for(n), kBlock, 0, c->stream>>>(n, p.dim, X, Y, Z, c->pos_rec);
-        const bool lanes = by_lanes(p.dim, n);
+        const bool lanes = by_lanes(p, p.re_s, n);
         if (lanes)
             k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
                                                                         c->coll_cnt, nullptr, nullptr, 0);
