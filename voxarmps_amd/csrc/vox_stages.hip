@@ -1467,6 +1467,18 @@ int st_euler(vox_ctx* c)
     return VOX_OK;
 }
 
+// The least double whose correctly rounded square root is not below rc: sqrt(x) < rc
+// exactly when x is below it, so the screen needs no root (1.2 million particles 222
+// -> 194 us; the gathers' cache lookups remain).
+static double square_bound(double rc)
+{
+    if (!(rc > 0.0)) return 0.0;
+    double x = rc * rc;
+    while (x > 0.0 && std::sqrt(x) >= rc) x = std::nextafter(x, 0.0);
+    while (std::sqrt(x) < rc) x = std::nextafter(x, HUGE_VAL);
+    return x;
+}
+
 // ---- COLLISION2: functions.cu:1523-1601 ------------------------------------------------------------
 // The reference updates particles i and j in place while it walks i = 1..TP and
 // each row in order, so a later pair sees earlier updates. That order is
@@ -1481,7 +1493,7 @@ int st_euler(vox_ctx* c)
 // Positions come as packed 32-byte records (z = 0 in 2D: the 3-term distance
 // equals the 2D one bit for bit); 8 record loads are in flight per row chunk
 // and candidates are emitted in slot order.
-__global__ __launch_bounds__(kBlock) void k_coll_screen(int n, double rc, ListView L,
+__global__ __launch_bounds__(kBlock) void k_coll_screen(int n, double rc2, ListView L,
                                                         const PosRec* __restrict__ rec,
                                                         const int32_t* __restrict__ off,
                                                         int32_t* __restrict__ cnt,
@@ -1509,8 +1521,7 @@ __global__ __launch_bounds__(kBlock) void k_coll_screen(int n, double rc, ListVi
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const double dx = px[e] - me.x, dy = py[e] - me.y, dz = pz[e] - me.z;
-            const double d = sqrt(dx * dx + dy * dy + dz * dz);
-            const bool hit = (jc[e] != i) && (d < rc);
+            const bool hit = (jc[e] != i) && (dx * dx + dy * dy + dz * dz < rc2);
             if (hit && off && pos + k < cap) { ci[pos + k] = i; cj[pos + k] = jc[e]; }
             k += hit ? 1 : 0;
         }
@@ -1518,7 +1529,7 @@ __global__ __launch_bounds__(kBlock) void k_coll_screen(int n, double rc, ListVi
     if (!off) cnt[i] = k;
 }
 
-__global__ __launch_bounds__(kBlock) void k_coll_screen_l16(int n, double rc, ListView L,
+__global__ __launch_bounds__(kBlock) void k_coll_screen_l16(int n, double rc2, ListView L,
                                                             const PosRec* __restrict__ rec,
                                                             const int32_t* __restrict__ off,
                                                             int32_t* __restrict__ cnt,
@@ -1535,7 +1546,7 @@ __global__ __launch_bounds__(kBlock) void k_coll_screen_l16(int n, double rc, Li
     walk16(L, r.i, r.live ? L.cnt[r.i] : 0, r.sub, [&](int j, bool in) {
         const PosRec q = rec[j];
         const double dx = q.x - me.x, dy = q.y - me.y, dz = q.z - me.z;
-        const bool hit = in && j != r.i && sqrt(dx * dx + dy * dy + dz * dz) < rc;
+        const bool hit = in && j != r.i && dx * dx + dy * dy + dz * dz < rc2;
         const unsigned long long m = __ballot(hit);
         const long at = pos + k + __popcll(m & below);
         if (hit && off && at < cap) { ci[at] = r.i; cj[at] = j; }
@@ -1872,14 +1883,14 @@ int st_collision(vox_ctx* c)
     for (int attempt = 0; attempt < 8; ++attempt) {
         double margin = p.coll * c->coll_margin;
         const bool every_pair = p.coll + margin > list_r;
-        const double rc = every_pair ? HUGE_VAL : p.coll + margin;
+        const double rc2 = every_pair ? HUGE_VAL : square_bound(p.coll + margin);
         k_pack_pos<<<grid_for(n), kBlock, 0, c->stream>>>(n, p.dim, X, Y, Z, c->pos_rec);
         const bool lanes = by_lanes(p, p.re_s, n);
         if (lanes)
-            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
+            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc2, L, c->pos_rec, nullptr,
                                                                         c->coll_cnt, nullptr, nullptr, 0);
         else
-            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, nullptr,
+            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc2, L, c->pos_rec, nullptr,
                                                                   c->coll_cnt, nullptr, nullptr, 0);
         VOX_TRY(scan_exclusive(c, c->coll_cnt, c->coll_off, n, c->coll_off + n));
         int32_t total = 0;
@@ -1888,11 +1899,11 @@ int st_collision(vox_ctx* c)
         if (total == 0) { c->st.collisions = 0; return VOX_OK; }
         VOX_TRY(coll_reserve(c, total));
         if (lanes)
-            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, c->coll_off,
+            k_coll_screen_l16<<<lane_blocks(n), kBlock, 0, c->stream>>>(n, rc2, L, c->pos_rec, c->coll_off,
                                                                         nullptr, c->coll_i, c->coll_j,
                                                                         c->coll_cap);
         else
-            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc, L, c->pos_rec, c->coll_off,
+            k_coll_screen<<<grid_for(n), kBlock, 0, c->stream>>>(n, rc2, L, c->pos_rec, c->coll_off,
                                                                   nullptr, c->coll_i, c->coll_j,
                                                                   c->coll_cap);
         CollArgs a;
