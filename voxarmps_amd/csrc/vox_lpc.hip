@@ -80,23 +80,32 @@ __device__ __forceinline__ double rademacher(uint64_t seed, int probe, int r)
 }
 
 // ---- row walks ---------------------------------------------------------------
-// The first `len` entries of a SELL-64 row in order: f(column, value, gathered)
-// for each, gathered = get(column). U entries' gathers are in flight together,
-// and the next U columns and values are loaded before they are used; loads past
-// the row's end take its last entry again, so none sits in a branch.
+// The first `len` entries of row r of a SELL-64 matrix in order: f(column, value,
+// gathered) for each, gathered = get(column). U entries' gathers are in flight
+// together, and the next U columns and values are loaded before they are used;
+// loads past the row's end take its last entry again, so none sits in a branch.
+// A wave's rows are of one slice, whose start is a scalar: a lane's offsets in it
+// (256 bytes an entry) are 32 bits for column and value alike. With 64-bit
+// addresses of each load, a third of the loop's instructions, the walks of 14.6k
+// rows took 6 to 14 % longer. (Loads that leave no cache lines: 22 to 45 % slower,
+// the four or eight lanes of a row then fetch an entry's line again.)
 template <int U, class Get, class F>
-__device__ __forceinline__ void walk_row(const int32_t* __restrict__ col, const float* __restrict__ val,
-                                         int len, Get get, F f)
+__device__ __forceinline__ void walk_row(const int32_t* __restrict__ cols, const float* __restrict__ vals,
+                                         int r, int cap, int len, Get get, F f)
 {
     if (len <= 0) return;
+    const long slice = mx_index((long)__builtin_amdgcn_readfirstlane(r >> 6) << 6, 0, cap);
+    const char* __restrict__ col = reinterpret_cast<const char*>(cols + slice);
+    const char* __restrict__ val = reinterpret_cast<const char*>(vals + slice);
+    const uint32_t first = 4u * (r & 63), last = first + 256u * (uint32_t)(len - 1);
     int32_t c[U], cn[U];
     float v[U], vn[U];
     auto next = [&](int k) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const long i = 64L * min(k + u, len - 1);
-            cn[u] = col[i];
-            vn[u] = val[i];
+            const uint32_t i = min(first + 256u * (uint32_t)(k + u), last);
+            cn[u] = *reinterpret_cast<const int32_t*>(col + i);
+            vn[u] = *reinterpret_cast<const float*>(val + i);
         }
     };
     decltype(get(0)) x[U];
@@ -160,7 +169,7 @@ __global__ __launch_bounds__(kBlock) void k_lpc_rowprep(PrepArgs a)
 struct FeatArgs {
     int nu, cap;
     float inv_re;
-    double thr;
+    float thr;                  // the smallest float not below the threshold
     const int32_t* __restrict__ rowlen;
     const int32_t* __restrict__ acol;
     const float* __restrict__ aval;
@@ -175,13 +184,15 @@ struct FeatArgs {
 
 // Four lanes per row: x, y, z moments and the sum of magnitudes. Strong
 // couplings wait in LDS for whole-line stores at the end (a wave's stores hold up
-// its next gathers); a row's 49th and later are stored as they come.
-// 240 -> 154 us at 107k rows of 215 entries (254 with the stores in the walk).
-constexpr int kStrongLds = 48;
+// its next gathers), written without a branch: an entry that is not strong is
+// overwritten by the next. A row's 61st and later are stored as they come; a
+// lattice has up to 56 within the threshold's distance, and 31 KB leave 5 blocks
+// to a CU. 107k rows of 215 entries: 240 us (one thread per row), 254 (stores in
+// the walk), 150 (a branch per strong entry), 135 (48 slots), 120.
+constexpr int kStrongLds = 60;
 __global__ __launch_bounds__(kBlock) void k_lpc_features(FeatArgs a)
 {
-    __shared__ int32_t qc[kStrongLds][kWave];
-    __shared__ float qv[kStrongLds][kWave];
+    __shared__ uint32_t qs[kStrongLds + 1][kWave][2];  // column, value; the last slot is not read
     __shared__ int sn[kWave];
     const int q = threadIdx.x & 3, lr = threadIdx.x >> 2;
     const int row0 = xcd_block() * kWave, r = row0 + lr;
@@ -189,22 +200,20 @@ __global__ __launch_bounds__(kBlock) void k_lpc_features(FeatArgs a)
         const float* __restrict__ pos = reinterpret_cast<const float*>(a.upos);
         const float own = pos[4L * r + q];
         const long b = mx_index(r, 0, a.cap);
+        uint32_t* __restrict__ out = (q & 1) ? reinterpret_cast<uint32_t*>(a.sval + b)
+                                             : reinterpret_cast<uint32_t*>(a.scol + b);
+        const int far = q < 2 ? kStrongLds : INT_MAX;  // lanes 2 and 3 hold 0's and 1's words
         float acc = 0.f;
         int n = 0;
-        walk_row<8>(a.acol + b, a.aval + b, a.rowlen[r], [&](int c) { return pos[4L * c + q]; },
+        walk_row<8>(a.acol, a.aval, r, a.cap, a.rowlen[r], [&](int c) { return pos[4L * c + q]; },
                     [&](int c, float v, float x) {
                         const float o = -v;
                         acc = fmaf(o, q < 3 ? x - own : 1.f, acc);
-                        if ((double)o >= a.thr) {
-                            if (n < kStrongLds) {
-                                if (q == 0) qc[n][lr] = c;
-                                if (q == 1) qv[n][lr] = o;
-                            } else {
-                                if (q == 0) a.scol[b + 64L * n] = c;
-                                if (q == 1) a.sval[b + 64L * n] = o;
-                            }
-                            ++n;
-                        }
+                        const bool strong = o >= a.thr;
+                        const uint32_t w = (q & 1) ? __float_as_uint(o) : (uint32_t)c;
+                        qs[min(n, kStrongLds)][lr][q & 1] = w;
+                        if (strong && n >= far) out[64L * n] = w;
+                        n += strong;
                     });
         const float osum = __shfl(acc, 3, 4);
         const float inv = (osum > 0.f) ? 1.f / osum : 0.f;
@@ -225,8 +234,8 @@ __global__ __launch_bounds__(kBlock) void k_lpc_features(FeatArgs a)
     const int i = threadIdx.x & (kWave - 1), n = sn[i];
     const long b = mx_index(row0 + i, 0, a.cap);
     for (int k = threadIdx.x >> 6; k < n; k += kBlock / kWave) {
-        a.scol[b + 64L * k] = qc[k][i];
-        a.sval[b + 64L * k] = qv[k][i];
+        a.scol[b + 64L * k] = (int32_t)qs[k][i][0];
+        a.sval[b + 64L * k] = __uint_as_float(qs[k][i][1]);
     }
 }
 
@@ -267,8 +276,8 @@ struct AggArgs {
 // with 16 / G of the message's channels.
 // Bound by the gathers' cache lookups: one thread per row, 32 bytes an entry,
 // made two a row and entry, the lanes of a row make one between them. 107k rows
-// of 215 entries 176 -> 103 us (8 lanes: the same within 3 %), 14.6k rows 134 ->
-// 21 us. 16 entries a batch measured the same, 4 slower.
+// of 215 entries 176 -> 102 us (8 lanes: the same within 3 %), 14.6k rows 134 ->
+// 19 us. 16 entries a batch measured the same, 4 slower.
 template <int G>
 __global__ __launch_bounds__(kBlock) void k_lpc_agg(AggArgs a)
 {
@@ -278,9 +287,8 @@ __global__ __launch_bounds__(kBlock) void k_lpc_agg(AggArgs a)
     if (r >= a.nu) return;
     struct Part { uint32_t w[D]; };
     const Part* __restrict__ s = reinterpret_cast<const Part*>(a.s);
-    const long b = mx_index(r, 0, a.cap);
     float acc[2 * D] = {};
-    walk_row<8>(a.acol + b, a.aval + b, a.rowlen[r], [&](int c) { return s[(long)G * c + q]; },
+    walk_row<8>(a.acol, a.aval, r, a.cap, a.rowlen[r], [&](int c) { return s[(long)G * c + q]; },
                 [&](int, float v, const Part& x) {
 #pragma unroll
                     for (int t = 0; t < D; ++t) {
@@ -536,17 +544,16 @@ struct OpView {   // a SELL-64 operator: rows, cap, lengths, columns, values
 __device__ __forceinline__ float row_product(const OpView& A, int r, int p, const float* __restrict__ x,
                                              float init)
 {
-    const long b = mx_index(r, 0, A.cap);
     float acc = init;
-    walk_row<8>(A.col + b, A.val + b, A.len[r], [&](int c) { return x[4L * c + p]; },
+    walk_row<8>(A.col, A.val, r, A.cap, A.len[r], [&](int c) { return x[4L * c + p]; },
                 [&](int, float v, float y) { acc = fmaf(v, y, acc); });
     return acc;
 }
 
 // One lane per row and probe in the kernels that follow, so that an operator is
 // walked once for the four probes and a gather takes their 16 bytes together.
-// 14.6k rows of 215 entries, all four probes: residual 4 x 87 -> 20 us, adjoint
-// 4 x 87 -> 17, mprobe 4 x 22 -> 7, dgc 4 x 36 -> 8.
+// 14.6k rows of 215 entries, all four probes: residual 4 x 87 -> 17 us, adjoint
+// 4 x 87 -> 15, mprobe 4 x 22 -> 7, dgc 4 x 36 -> 8.
 // t = Oh (sc w); z = g w / A_rr + sc t
 __global__ __launch_bounds__(kBlock) void k_lpc_mprobe(OpView S, const float* __restrict__ sc,
                                                        const float* __restrict__ g,
@@ -699,7 +706,7 @@ __global__ __launch_bounds__(kBlock) void k_lpc_dense_bwd(int nu, int l, const u
 
 // ds_k = sum_r O_kr dmh_r (transpose of the aggregation; O is symmetric), 8
 // lanes per row with 2 of the 16 channels each, and dh_prev_k += ds_k P_l.
-// 14.6k rows 165 (one thread per row) -> 33 us.
+// 14.6k rows 165 (one thread per row) -> 30 us.
 __global__ __launch_bounds__(kBlock) void k_lpc_agg_bwd(int nu, int cap, const int32_t* __restrict__ rowlen,
                                                         const int32_t* __restrict__ acol,
                                                         const float* __restrict__ aval, int l,
@@ -716,8 +723,7 @@ __global__ __launch_bounds__(kBlock) void k_lpc_agg_bwd(int nu, int cap, const i
     float a0 = 0.f, a1 = 0.f;
     if (r < nu) {
         const float2* __restrict__ d = reinterpret_cast<const float2*>(dmh);
-        const long b = mx_index(r, 0, cap);
-        walk_row<8>(acol + b, aval + b, rowlen[r], [&](int c) { return d[8L * c + q]; },
+        walk_row<8>(acol, aval, r, cap, rowlen[r], [&](int c) { return d[8L * c + q]; },
                     [&](int, float v, float2 x) {
                         a0 = fmaf(-v, x.x, a0);
                         a1 = fmaf(-v, x.y, a1);
@@ -1094,7 +1100,10 @@ static void ctx_features(vox_ctx* c, int rows, v4f* upos, float* invd, float* fe
     pa.upos = upos; pa.invd = invd; pa.feat = feat;
     k_lpc_rowprep<<<grid_for(rows), kBlock, 0, c->stream>>>(pa);
     FeatArgs fa;
-    fa.nu = c->nu; fa.cap = c->a_cap; fa.inv_re = (float)(1.0 / c->p.re_l); fa.thr = lpc_threshold(c);
+    fa.nu = c->nu; fa.cap = c->a_cap; fa.inv_re = (float)(1.0 / c->p.re_l);
+    const double thr = lpc_threshold(c);
+    fa.thr = (float)thr;
+    if ((double)fa.thr < thr) fa.thr = std::nextafter(fa.thr, INFINITY);
     fa.rowlen = c->rowlen; fa.acol = c->acol; fa.aval = c->aval32; fa.upos = upos; fa.invd = invd;
     fa.feat = feat; fa.inv_osum = inv_osum; fa.slen = slen; fa.scol = scol; fa.sval = sval;
     k_lpc_features<<<grid_for(4L * c->nu), kBlock, 0, c->stream>>>(fa);
