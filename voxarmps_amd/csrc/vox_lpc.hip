@@ -277,7 +277,8 @@ struct AggArgs {
 // Bound by the gathers' cache lookups: one thread per row, 32 bytes an entry,
 // made two a row and entry, the lanes of a row make one between them. 107k rows
 // of 215 entries 176 -> 102 us (8 lanes: the same within 3 %), 14.6k rows 134 ->
-// 19 us. 16 entries a batch measured the same, 4 slower.
+// 19 us. 16 entries a batch and 3 to 6 waves a SIMD measured the same, 4 entries
+// slower, 8 waves 6 to 20 % slower (107k rows, blocks of 128 to 1024 threads).
 template <int G>
 __global__ __launch_bounds__(kBlock) void k_lpc_agg(AggArgs a)
 {

@@ -915,6 +915,7 @@ __global__ __launch_bounds__(BS) void k_prediction_dg(PredArgs a)
 // record, 86 % of the cycles). Adding in every lane by lane broadcast: 1545 us,
 // 236 us; with that, records brought to LDS four lanes a record (a third of the
 // lookups) 1690 us, 267 us; 96 registers for a fifth wave spill (3566 us).
+// Blocks of 128, 512, 1024 threads: 1527, 1513, 1566 us (103k rows 209, 233, 250).
 constexpr int kPredSlots = 80;                     // queued entries of a row
 constexpr int kPredStride = kBlock / 16 + 4;       // rows of a slot, padded
 // terms of a wave's four rows: padded so that the twelve sums read 16 bytes each
