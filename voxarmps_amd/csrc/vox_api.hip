@@ -605,7 +605,8 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
     for (int w = 0; w < 2; ++w) {
         if (w == 1 && !c->two_lists) break;
         DevList& L = c->list[w];
-        if ((rc = dalloc(&L.cnt, n)) || (rc = dalloc(&L.cell, n)) || (rc = dalloc(&L.order_raw, n)) ||
+        if ((rc = dalloc(&L.cnt, n)) || (rc = dalloc(&L.cell, n)) || (rc = dalloc(&L.slot_of, n)) ||
+            (rc = dalloc(&L.order_raw, n)) ||
             (rc = dalloc(&L.rec, n)) || (rc = dalloc(&L.pos_of, n)))
             return bail(rc);
         double re = (w == 0) ? c->p.re_s : c->p.re_l;
@@ -661,7 +662,7 @@ int vox_destroy(vox_ctx* c)
     for (int w = 0; w < 2; ++w) {
         DevList& L = c->list[w];
         dfree(L.cnt); dfree(L.ids); dfree(L.cell); dfree(L.cell_start); dfree(L.cell_fill);
-        dfree(L.order_raw); dfree(L.rec); dfree(L.pos_of);
+        dfree(L.slot_of); dfree(L.order_raw); dfree(L.rec); dfree(L.pos_of);
     }
     for (int k = 0; k < 6; ++k) dfree(c->sps_s[k]);
     dfree(c->scratch_d); dfree(c->pred_rec); dfree(c->pt_sorted); dfree(c->pos_rec);

@@ -128,6 +128,9 @@ struct DevList {
     int32_t* cell = nullptr;       // tp
     int32_t* cell_start = nullptr; // tnc + 1
     int32_t* cell_fill = nullptr;  // tnc: particles of a cell, zero between searches
+    bool fill_clear = false;       //   while this is set
+    int32_t* slot_of = nullptr;    // tp: a particle's slot among its cell's
+    bool searched = false;         // the last search's sort was queued
     int32_t* order_raw = nullptr;  // tp (ids by cell, unsorted within)
     PosRec* rec = nullptr;         // tp: positions + id sorted by (cell, id)
     bool sorted = false;           // rec holds a sort (a NEIGHBOR call has run)

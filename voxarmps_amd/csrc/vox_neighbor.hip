@@ -178,6 +178,19 @@ __global__ __launch_bounds__(kScanOne) void k_scan_one(const int32_t* in, int32_
     if (total && threadIdx.x == 0) *total = before;
 }
 
+// Scratch for a scan of n items. A capacity is only ever that of a live buffer.
+static int reserve_scan(vox_ctx* c, long n)
+{
+    const long nb = (n + kScanTile - 1) / kScanTile;
+    if (n <= kScanOneMax || nb <= c->scan_blocks_cap) return VOX_OK;
+    if (c->scan_blocks) (void)hipFree(c->scan_blocks);
+    c->scan_blocks = nullptr;
+    c->scan_blocks_cap = 0;
+    VOX_HIP(hipMalloc(&c->scan_blocks, sizeof(int32_t) * (nb + 64)));
+    c->scan_blocks_cap = nb + 64;
+    return VOX_OK;
+}
+
 // out[0..n) = exclusive scan of in[0..n); out[n] = total if out has room (caller
 // passes total_dev to receive it; may alias out + n); clear: in, zeroed on the way.
 int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t* total_dev, int32_t* clear)
@@ -187,14 +200,8 @@ int scan_exclusive(vox_ctx* c, const int32_t* in, int32_t* out, long n, int32_t*
         VOX_HIP(hipGetLastError());
         return VOX_OK;
     }
-    long nb = (n + kScanTile - 1) / kScanTile;
-    if (nb < 1) nb = 1;
-    if (nb > c->scan_blocks_cap) {
-        if (c->scan_blocks) (void)hipFree(c->scan_blocks);
-        c->scan_blocks = nullptr;
-        VOX_HIP(hipMalloc(&c->scan_blocks, sizeof(int32_t) * (nb + 64)));
-        c->scan_blocks_cap = nb + 64;
-    }
+    VOX_TRY(reserve_scan(c, n));
+    const long nb = (n + kScanTile - 1) / kScanTile;
     k_scan_tile_sums<<<(int)nb, kBlock, 0, c->stream>>>(in, c->scan_blocks, n);
     k_scan_out<<<(int)nb, kBlock, 0, c->stream>>>(in, out, c->scan_blocks, n, total_dev, clear);
     VOX_HIP(hipGetLastError());
@@ -920,6 +927,7 @@ static int launch_one(vox_ctx* c, int which, double re)
     DevList& L = c->list[which];
     const int n = c->tp;
     L.re = re;
+    L.searched = false;                // until this search's sort is queued
     L.g = make_grid(c->p, re);
     if (L.g.tnc <= 0 || L.g.tnc > (1L << 30))
         return fail(VOX_ERR_ARG, "neighbour grid has an invalid number of cells");
@@ -927,17 +935,25 @@ static int launch_one(vox_ctx* c, int which, double re)
         if (L.cell_start) (void)hipFree(L.cell_start);
         if (L.cell_fill) (void)hipFree(L.cell_fill);
         L.cell_start = L.cell_fill = nullptr;
+        L.tnc_alloc = 0;
+        L.fill_clear = false;
         VOX_HIP(hipMalloc(&L.cell_start, sizeof(int32_t) * (L.g.tnc + 1)));
         VOX_HIP(hipMalloc(&L.cell_fill, sizeof(int32_t) * (L.g.tnc + 1)));
         L.tnc_alloc = L.g.tnc;
-        VOX_TRY(fill_i32(c, L.cell_fill, 0, L.g.tnc + 1));
     }
+    // The scan of the counts clears them for the next search. A search that ends
+    // between the count and that scan (an error of an earlier launch shows up there)
+    // leaves them raised: slots counted on top of them would lie past order_raw, so
+    // the next search clears them itself. What the scan needs is reserved first, and
+    // the slots have an array of their own: rec, pos_of and the rows stay those of the
+    // last search that got past here.
+    VOX_TRY(reserve_scan(c, L.g.tnc));
+    if (!L.fill_clear) VOX_TRY(fill_i32(c, L.cell_fill, 0, L.tnc_alloc + 1));
+    L.fill_clear = false;
     {
         ProfScope ps(c, KC_CELL);
-        // (the counts are zero: each scan clears them; pos_of holds the slots
-        // until the sort writes the positions)
         k_cell_keys<<<grid_for(n), kBlock, 0, c->stream>>>(L.g, n, c->f[VOX_F_X], c->f[VOX_F_Y],
-                                                             c->f[VOX_F_Z], L.cell, L.pos_of,
+                                                             c->f[VOX_F_Z], L.cell, L.slot_of,
                                                              L.cell_fill, c->dflags);
         VOX_HIP(hipGetLastError());
     }
@@ -945,7 +961,8 @@ static int launch_one(vox_ctx* c, int which, double re)
         ProfScope ps(c, KC_SORT);
         VOX_TRY(scan_exclusive(c, L.cell_fill, L.cell_start, L.g.tnc, L.cell_start + L.g.tnc,
                                L.cell_fill));
-        k_scatter<<<grid_for(n), kBlock, 0, c->stream>>>(n, L.cell, L.pos_of, L.cell_start,
+        L.fill_clear = true;
+        k_scatter<<<grid_for(n), kBlock, 0, c->stream>>>(n, L.cell, L.slot_of, L.cell_start,
                                                            L.order_raw);
         // cells of fewer than ~24 expected particles: one thread per particle
         if (few_per_cell(c, L)) {
@@ -962,7 +979,7 @@ static int launch_one(vox_ctx* c, int which, double re)
         }
         VOX_HIP(hipGetLastError());
     }
-    L.sorted = true;
+    L.sorted = L.searched = true;
     return search_one(c, which, re);
 }
 
@@ -1075,6 +1092,7 @@ int ensure_reference_list(vox_ctx* c, int which)
 {
     DevList& L = c->list[which];
     if (!L.compact) return VOX_OK;
+    if (!L.searched) return fail(VOX_ERR_STATE, "the last neighbour search did not finish");
     const int sm = which == 0 ? SPR_MAXCNT_S : SPR_MAXCNT_L;
     const double R = L.g.incl ? L.re + c->p.delta : L.re;
     const int n = c->tp;
