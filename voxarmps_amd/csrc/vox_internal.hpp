@@ -44,12 +44,16 @@ struct __align__(64) PredRec {
 void set_error(const std::string& msg);
 int fail(int code, const std::string& msg);
 
+// (a reported error is taken from the runtime too: the next call's launch checks
+// would report it again)
 #define VOX_HIP(call)                                                              \
     do {                                                                           \
         hipError_t e_ = (call);                                                    \
-        if (e_ != hipSuccess)                                                      \
+        if (e_ != hipSuccess) {                                                    \
+            (void)hipGetLastError();                                               \
             return ::vox::fail(VOX_ERR_HIP, std::string(#call) + ": " +            \
                                                 hipGetErrorString(e_));            \
+        }                                                                          \
     } while (0)
 
 #define VOX_TRY(expr)                                                              \

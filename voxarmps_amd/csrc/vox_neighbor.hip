@@ -849,6 +849,11 @@ __global__ __launch_bounds__(kWave, 4) void k_build_list_mm(
 }
 
 // ---- host side --------------------------------------------------------------------------
+// Empties the rows of a list whose search ended with rows longer than its storage
+// (no room for wider ones, or another error first): every stage then finds no
+// neighbours, and the next search starts from the storage there is.
+static int drop_rows(vox_ctx* c, int which) { return fill_i32(c, c->list[which].cnt, 0, c->tp); }
+
 int ensure_list_storage(vox_ctx* c, int which, int cap)
 {
     DevList& L = c->list[which];
@@ -856,7 +861,16 @@ int ensure_list_storage(vox_ctx* c, int which, int cap)
     if (cap <= L.cap && L.ids) return VOX_OK;
     if (L.ids) (void)hipFree(L.ids);
     L.ids = nullptr;
-    VOX_HIP(hipMalloc(&L.ids, sizeof(int32_t) * (size_t)sl_size(c->tp, cap)));
+    L.cap = 0;
+    const size_t bytes = sizeof(int32_t) * (size_t)sl_size(c->tp, cap);
+    const hipError_t e = hipMalloc(&L.ids, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        L.ids = nullptr;
+        VOX_TRY(drop_rows(c, which));
+        return fail(VOX_ERR_HIP, "neighbour rows of " + std::to_string(cap) + " entries (" +
+                                     std::to_string(bytes >> 20) + " MB): " + hipGetErrorString(e));
+    }
     L.cap = cap;
     return VOX_OK;
 }
@@ -1047,10 +1061,20 @@ static int search_one(vox_ctx* c, int which, double re)
     return VOX_OK;
 }
 
+// After read_flags, on the way out with an error: rows that were never searched
+// again with the storage they need.
+static int drop_long_rows(vox_ctx* c)
+{
+    for (int w = 0; w < (c->two_lists ? 2 : 1); ++w)
+        if (spread_max(c, w == 0 ? SPR_MAXCNT_S : SPR_MAXCNT_L) > c->list[w].cap) VOX_TRY(drop_rows(c, w));
+    return VOX_OK;
+}
+
 // After read_flags: the domain error, naming the first particle outside the
 // grid (its type, position and velocity).
 static int domain_error(vox_ctx* c)
 {
+    VOX_TRY(drop_long_rows(c));
     const int i = c->hflags[FLAG_DOMAIN_FIRST];
     double v[5] = {0, 0, 0, 0, 0};
     int32_t t = 0;
@@ -1081,6 +1105,7 @@ static int regrow_one(vox_ctx* c, int which, double re)
         VOX_TRY(search_one(c, which, re));
         VOX_TRY(read_flags(c));
     }
+    VOX_TRY(drop_rows(c, which));
     return fail(VOX_ERR_OVERFLOW, "neighbour row capacity could not be satisfied");
 }
 
@@ -1110,6 +1135,7 @@ int ensure_reference_list(vox_ctx* c, int which)
         }
         VOX_TRY(ensure_list_storage(c, which, ((need + need / 4) + 7) & ~7));
     }
+    VOX_TRY(drop_rows(c, which));
     return fail(VOX_ERR_OVERFLOW, "neighbour row capacity could not be satisfied");
 }
 
@@ -1202,7 +1228,11 @@ int build_neighbors(vox_ctx* c)
         VOX_HIP(hipStreamWaitEvent(c->stream, c->ev_join, 0));
         VOX_TRY(read_flags(c));
         if (c->hflags[FLAG_DOMAIN] != 0) return domain_error(c);
-        VOX_TRY(regrow_one(c, 0, c->p.re_s));
+        const int rc = regrow_one(c, 0, c->p.re_s);
+        if (rc != VOX_OK) {
+            VOX_TRY(drop_long_rows(c));
+            return rc;
+        }
         VOX_TRY(regrow_one(c, 1, c->p.re_l));
     } else {
         VOX_TRY(build_one(c, 0, c->p.re_s));
