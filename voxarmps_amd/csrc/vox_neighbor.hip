@@ -1154,6 +1154,7 @@ int list_l_for_consumer(vox_ctx* c)
 
 static int build_one(vox_ctx* c, int which, double re)
 {
+    VOX_TRY(clear_search_status(c));
     VOX_TRY(launch_one(c, which, re));
     VOX_TRY(read_flags(c));
     if (c->hflags[FLAG_DOMAIN] != 0) return domain_error(c);
@@ -1215,8 +1216,8 @@ static int launch_side(vox_ctx* c, int which, double re)
 
 int build_neighbors(vox_ctx* c)
 {
-    VOX_TRY(clear_search_status(c));
     if (c->two_lists && c->stream2) {
+        VOX_TRY(clear_search_status(c));
         // The two lists are independent: list L is built on a second stream
         // beside list S (the side stream first waits for everything queued so
         // far), and the main stream waits for it before the one flag read.
