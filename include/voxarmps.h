@@ -283,8 +283,8 @@ int vox_set_regions(vox_ctx* ctx, int nregion, const int32_t* region, const doub
 
 /* Tile-shape autotuner (no counterpart in the reference): times both
  * neighbour-search walks (1: one thread or, in small systems, 16 lanes per
- * particle, 2: one wave per 64 cell-sorted particles) over `reps` builds on the current positions and keeps the faster per
- * list (modes[2] receives the choice for lists S and L); then runs the step's
+ * particle, 2: one wave per 64 cell-sorted particles) over `reps` builds on the
+ * current positions and keeps the faster per list (modes[2] receives the choice for lists S and L); then runs the step's
  * stages up to MATRIX once and times the predictor's variants (FP64: records
  * gathered per group 4, 8 or 2 with 256 threads per block, 4 or 8 with 128;
  * variants 5-7: 8 records with 128 or 256 threads, 4 with 128, and the gradient
@@ -293,8 +293,10 @@ int vox_set_regions(vox_ctx* ctx, int nregion, const int32_t* region, const doub
  * per-block LDS window of the block's distinct columns; 1, 2, 3: 4, 16 and 8
  * entries on the 32-bit columns; 4: 8 entries on 16-bit column steps; 0 and 4
  * fall back to the next form where the assembly's rows do not allow theirs).
- * Every variant gives the same bits; the context keeps the fastest. Requires
- * vox_init. */
+ * Every variant gives the same bits; the context keeps the fastest. Product 0 is
+ * kept untimed where the solve then runs in one block or renews the direction in
+ * its products (up to 196,608 unknowns, and larger 2D systems): no other variant
+ * does either. Requires vox_init. */
 int vox_autotune(vox_ctx* ctx, int reps, int32_t* modes);
 /* The context's tuning (no counterpart in the reference): choice[4] = walk of
  * list S, walk of list L (0 = heuristic), predictor variant (0..8), product

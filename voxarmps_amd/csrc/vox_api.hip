@@ -347,7 +347,8 @@ namespace vox {
 // the choice is by time only. The step's stages up to MATRIX run once on the
 // current state (each field they write is rewritten by the next step before
 // it is read; the pressure is not touched), then each predictor variant
-// (FP64 path) and each PPE product variant is timed over `reps` launches.
+// (FP64 path) is timed over `reps` launches, and each PPE product variant where a
+// solve runs it as a product alone.
 int autotune_kernels(vox_ctx* c, int reps)
 {
     if (reps < 1) reps = 1;
@@ -387,13 +388,7 @@ int autotune_kernels(vox_ctx* c, int reps)
     VOX_TRY(st_bcon(c));
     VOX_TRY(ppe_assemble(c));
     if (c->nu <= 0) return VOX_OK;
-    float ms[kSpmvVariants] = {};
-    VOX_TRY(time_spmv_variants(c, reps, ms));
-    int pick = 0;
-    for (int v = 1; v < kSpmvVariants; ++v)
-        if (ms[v] < ms[pick]) pick = v;
-    c->tune_spmv = pick;
-    return VOX_OK;
+    return tune_product(c, reps);
 }
 
 }  // namespace vox

@@ -42,6 +42,8 @@
 // which stays a conjugate-direction method when M varies between solves or
 // is not exactly symmetric positive definite.
 
+#include <algorithm>
+
 #include "vox_internal.hpp"
 
 namespace vox {
@@ -1632,7 +1634,7 @@ static int solve_learned(vox_ctx* c, vox_solve_info* info)
 
 // Times each product variant on the assembled system (the context's solver
 // vectors hold p = D^-1 b afterwards, as after a solve's setup): ms[v] is the
-// mean of `reps` launches. Used by the autotuner; needs nu > 0.
+// mean of `reps` launches.
 template <class VT, class MT>
 static int time_spmv_t(vox_ctx* c, CgArgs<VT, MT>& a, int reps, float* ms)
 {
@@ -1660,23 +1662,46 @@ static int time_spmv_t(vox_ctx* c, CgArgs<VT, MT>& a, int reps, float* ms)
     return rc;
 }
 
-int time_spmv_variants(vox_ctx* c, int reps, float* ms)
+// The form a solve of this system takes with variant 0: whether the product does
+// more than a product there.
+template <class VT, class MT>
+static bool variant0_fused(const vox_ctx* c, const CgArgs<VT, MT>& a)
+{
+    const bool learned = c->p.solver == VOX_SOLVER_LEARNED_FCG;
+    return (!learned && one_block(c)) || (updates_p(c, a) && (!learned || a.npq <= kFusedBlocks));
+}
+
+// Picks the product variant of the assembled system (tune_spmv). Where a solve with
+// variant 0 runs in one block or renews the direction in its products, which no
+// other variant does, it is variant 0 untimed: the bare product would rank it
+// without what it saves. Solves of 7 to 13 iterations there, variant 0 and the best of
+// the others, us: 2D rows 1k 87 / 117, 20k 98 / 135, 130k 178 / 210, 900k 787 / 897;
+// 3D rows 1k 126 / 179, 30k 211 / 283, 110k 344 / 464, 190k 527 / 682; mixed
+// precision the same order (1k 125 / 175, 190k 488 / 602).
+int tune_product(vox_ctx* c, int reps)
 {
     if (c->nu <= 0) return fail(VOX_ERR_STATE, "no assembled PPE to time the product on");
     if (grid_for(c->nu) > kMaxPartials) return fail(VOX_ERR_ARG, "PPE larger than the solver's row limit");
+    c->tune_spmv = 0;
     VOX_TRY(prepare_product(c, true));
+    float ms[kSpmvVariants] = {};
     if (c->p.precision == VOX_PREC_MIXED) {
         if (!c->aval32_ok) VOX_TRY(ppe_make_aval32(c));
         CgArgs<float, float> a;
         fill_args(c, a, (const float*)c->aval32, c->cg_x32, c->cg_r32, c->cg_p32, c->cg_q32,
                   c->rhs, c->p.cg_tol, c->p.cg_maxit);
-        return time_spmv_t(c, a, reps, ms);
+        if (variant0_fused(c, a)) return VOX_OK;
+        VOX_TRY(time_spmv_t(c, a, reps, ms));
+    } else {
+        if (!c->aval64_ok) VOX_TRY(ppe_make_aval64(c));
+        CgArgs<double, double> a;
+        fill_args(c, a, (const double*)c->aval, c->cg_x, c->cg_r, c->cg_p, c->cg_q, c->rhs,
+                  c->p.cg_tol, c->p.cg_maxit);
+        if (variant0_fused(c, a)) return VOX_OK;
+        VOX_TRY(time_spmv_t(c, a, reps, ms));
     }
-    if (!c->aval64_ok) VOX_TRY(ppe_make_aval64(c));
-    CgArgs<double, double> a;
-    fill_args(c, a, (const double*)c->aval, c->cg_x, c->cg_r, c->cg_p, c->cg_q, c->rhs,
-              c->p.cg_tol, c->p.cg_maxit);
-    return time_spmv_t(c, a, reps, ms);
+    c->tune_spmv = (int)(std::min_element(ms, ms + kSpmvVariants) - ms);
+    return VOX_OK;
 }
 
 int ppe_solve(vox_ctx* c, vox_solve_info* info)

@@ -503,7 +503,7 @@ int st_viscosity(vox_ctx* c);
 int st_prediction(vox_ctx* c);
 const char* pred_variant_name(int v);
 int autotune_kernels(vox_ctx* c, int reps);   // predictor and PPE product variants (vox_api.hip)
-int time_spmv_variants(vox_ctx* c, int reps, float* ms);   // vox_cg.hip
+int tune_product(vox_ctx* c, int reps);                    // vox_cg.hip
 bool uniform_meu(const vox_ctx* c);
 int st_prediction32(vox_ctx* c);
 int st_phat32(vox_ctx* c);          // the FP32 twins of the mixed precision mode
