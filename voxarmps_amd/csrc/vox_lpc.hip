@@ -894,12 +894,15 @@ struct vox_lpc {
 
 namespace vox {
 
+// Zeroed memory for kernels on `stream`, cleared in that stream's order: the streams
+// here do not wait for the null stream, on which a clear of hundreds of megabytes would
+// still run when the first kernels write there.
 template <class T>
-static int lalloc(T** p, size_t n)
+static int lalloc(hipStream_t stream, T** p, size_t n)
 {
     if (n == 0) n = 1;
     VOX_HIP(hipMalloc((void**)p, sizeof(T) * n));
-    VOX_HIP(hipMemset(*p, 0, sizeof(T) * n));
+    VOX_HIP(hipMemsetAsync(*p, 0, sizeof(T) * n, stream));
     return VOX_OK;
 }
 template <class T>
@@ -947,18 +950,19 @@ static int lpc_training_buffers(vox_lpc* L, int rows)
         lfree(*p);
     lfree(L->epart);
     const size_t n = (size_t)rows;
-    for (auto*& p : L->h) VOX_TRY(lalloc(&p, n * LH));
-    for (auto*& p : L->s) VOX_TRY(lalloc(&p, n * LM));
-    for (auto*& p : L->m) VOX_TRY(lalloc(&p, n * LM));
-    VOX_TRY(lalloc(&L->o, n * LO));
-    for (float** p : {&L->g, &L->c, &L->sc}) VOX_TRY(lalloc(p, n));
-    for (float** p : {&L->wv, &L->vv, &L->t, &L->z, &L->e, &L->y, &L->ys}) VOX_TRY(lalloc(p, n * kProbes));
-    VOX_TRY(lalloc(&L->epart, (size_t)kProbes * grid_for((long)kProbes * rows)));
-    VOX_TRY(lalloc(&L->dO, n * 2));
-    VOX_TRY(lalloc(&L->dh[0], n * LH));
-    VOX_TRY(lalloc(&L->dh[1], n * LH));
-    VOX_TRY(lalloc(&L->dmh, n * LM));
-    VOX_TRY(lalloc(&L->ds, n * LM));
+    auto alloc = [&](auto** p, size_t k) { return lalloc(L->stream, p, k); };
+    for (auto*& p : L->h) VOX_TRY(alloc(&p, n * LH));
+    for (auto*& p : L->s) VOX_TRY(alloc(&p, n * LM));
+    for (auto*& p : L->m) VOX_TRY(alloc(&p, n * LM));
+    VOX_TRY(alloc(&L->o, n * LO));
+    for (float** p : {&L->g, &L->c, &L->sc}) VOX_TRY(alloc(p, n));
+    for (float** p : {&L->wv, &L->vv, &L->t, &L->z, &L->e, &L->y, &L->ys}) VOX_TRY(alloc(p, n * kProbes));
+    VOX_TRY(alloc(&L->epart, (size_t)kProbes * grid_for((long)kProbes * rows)));
+    VOX_TRY(alloc(&L->dO, n * 2));
+    VOX_TRY(alloc(&L->dh[0], n * LH));
+    VOX_TRY(alloc(&L->dh[1], n * LH));
+    VOX_TRY(alloc(&L->dmh, n * LM));
+    VOX_TRY(alloc(&L->ds, n * LM));
     L->rows_cap = rows;
     return VOX_OK;
 }
@@ -1121,27 +1125,28 @@ int lpc_prepare(vox_ctx* c)
     if (c->lpc_rows < rows) {
         lpc_free_ctx(c);
         const size_t n = (size_t)rows;
-        VOX_TRY(lalloc(&c->lpc_feat, n * LF));
-        VOX_TRY(lalloc(&c->lpc_inv_osum, n));
-        VOX_TRY(lalloc(&c->lpc_t, n));
-        VOX_TRY(lalloc(&c->lpc_invd, n));
-        VOX_TRY(lalloc(&c->lpc_upos, n));
-        VOX_TRY(lalloc(&c->lpc_h[0], n * LH));
-        VOX_TRY(lalloc(&c->lpc_h[1], n * LH));
-        VOX_TRY(lalloc(&c->lpc_s, n * LM));
-        VOX_TRY(lalloc(&c->lpc_m, n * LM));
-        VOX_TRY(lalloc(&c->lpc_o, n * LO));
-        VOX_TRY(lalloc(&c->lpc_gd, n));
-        VOX_TRY(lalloc(&c->lpc_slen, n));
-        VOX_TRY(lalloc(&c->cg_z, n));
-        VOX_TRY(lalloc(&c->cg_z32, n));
+        auto alloc = [&](auto** p, size_t k) { return lalloc(c->stream, p, k); };
+        VOX_TRY(alloc(&c->lpc_feat, n * LF));
+        VOX_TRY(alloc(&c->lpc_inv_osum, n));
+        VOX_TRY(alloc(&c->lpc_t, n));
+        VOX_TRY(alloc(&c->lpc_invd, n));
+        VOX_TRY(alloc(&c->lpc_upos, n));
+        VOX_TRY(alloc(&c->lpc_h[0], n * LH));
+        VOX_TRY(alloc(&c->lpc_h[1], n * LH));
+        VOX_TRY(alloc(&c->lpc_s, n * LM));
+        VOX_TRY(alloc(&c->lpc_m, n * LM));
+        VOX_TRY(alloc(&c->lpc_o, n * LO));
+        VOX_TRY(alloc(&c->lpc_gd, n));
+        VOX_TRY(alloc(&c->lpc_slen, n));
+        VOX_TRY(alloc(&c->cg_z, n));
+        VOX_TRY(alloc(&c->cg_z32, n));
         c->lpc_rows = rows;
     }
     if (c->lpc_scap != c->a_cap) {
         lfree(c->lpc_scol);
         lfree(c->lpc_sval);
-        VOX_TRY(lalloc(&c->lpc_scol, (size_t)sl_size(c->tp, c->a_cap)));
-        VOX_TRY(lalloc(&c->lpc_sval, (size_t)sl_size(c->tp, c->a_cap)));
+        VOX_TRY(lalloc(c->stream, &c->lpc_scol, (size_t)sl_size(c->tp, c->a_cap)));
+        VOX_TRY(lalloc(c->stream, &c->lpc_sval, (size_t)sl_size(c->tp, c->a_cap)));
         c->lpc_scap = c->a_cap;
     }
     if (nu == 0) return VOX_OK;
@@ -1180,10 +1185,11 @@ int vox_lpc_create(vox_lpc** out, uint64_t seed)
     if (hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(VOX_ERR_HIP, "hipStreamCreate"));
     int rc;
-    if ((rc = lalloc(&L->w32, NPARAM)) || (rc = lalloc(&L->grad, NPARAM)) || (rc = lalloc(&L->am, NPARAM)) ||
-        (rc = lalloc(&L->av, NPARAM)) || (rc = lalloc(&L->w16, NPARAM)) ||
-        (rc = lalloc(&L->gpart, (size_t)kOuterBlocks * NPARAM)) ||
-        (rc = lalloc(&L->dpart, (size_t)kMaxPartials)) || (rc = lalloc(&L->dscal, LS_COUNT)))
+    auto alloc = [&](auto** p, size_t n) { return lalloc(L->stream, p, n); };
+    if ((rc = alloc(&L->w32, NPARAM)) || (rc = alloc(&L->grad, NPARAM)) || (rc = alloc(&L->am, NPARAM)) ||
+        (rc = alloc(&L->av, NPARAM)) || (rc = alloc(&L->w16, NPARAM)) ||
+        (rc = alloc(&L->gpart, (size_t)kOuterBlocks * NPARAM)) || (rc = alloc(&L->dpart, (size_t)kMaxPartials)) ||
+        (rc = alloc(&L->dscal, LS_COUNT)))
         return bail(rc);
     if (hipHostMalloc((void**)&L->hscal, sizeof(double) * LS_COUNT, hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void**)&L->hgrad, sizeof(float) * NPARAM, hipHostMallocDefault) != hipSuccess)
@@ -1238,10 +1244,10 @@ int vox_lpc_set_weights(vox_lpc* L, const float* w)
     VOX_HIP(hipMemcpyAsync(L->w32, w, sizeof(float) * NPARAM, hipMemcpyHostToDevice, L->stream));
     k_lpc_cast<<<grid_for(NPARAM), kBlock, 0, L->stream>>>(NPARAM, L->w32, L->w16);
     VOX_HIP(hipGetLastError());
-    VOX_HIP(hipStreamSynchronize(L->stream));
     // a fresh set of weights restarts the optimiser
-    VOX_HIP(hipMemset(L->am, 0, sizeof(float) * NPARAM));
-    VOX_HIP(hipMemset(L->av, 0, sizeof(float) * NPARAM));
+    VOX_HIP(hipMemsetAsync(L->am, 0, sizeof(float) * NPARAM, L->stream));
+    VOX_HIP(hipMemsetAsync(L->av, 0, sizeof(float) * NPARAM, L->stream));
+    VOX_HIP(hipStreamSynchronize(L->stream));
     L->adam_t = 0;
     return VOX_OK;
 }
@@ -1271,10 +1277,11 @@ int vox_lpc_dump(vox_lpc* L, vox_ctx* c, int32_t* index)
         lfree(S.rowlen); lfree(S.acol); lfree(S.slen); lfree(S.scol); lfree(S.aval); lfree(S.diag);
         lfree(S.inv_d); lfree(S.inv_osum); lfree(S.feat); lfree(S.rhs); lfree(S.sval); lfree(upos);
     };
-    if ((rc = lalloc(&S.rowlen, nn)) || (rc = lalloc(&S.acol, mat)) || (rc = lalloc(&S.aval, mat)) ||
-        (rc = lalloc(&S.slen, nn)) || (rc = lalloc(&S.scol, mat)) || (rc = lalloc(&S.sval, mat)) ||
-        (rc = lalloc(&S.diag, nn)) || (rc = lalloc(&S.inv_d, nn)) || (rc = lalloc(&S.inv_osum, nn)) ||
-        (rc = lalloc(&S.feat, nn * LF)) || (rc = lalloc(&S.rhs, nn)) || (rc = lalloc(&upos, nn))) {
+    auto alloc = [&](auto** p, size_t n) { return lalloc(c->stream, p, n); };
+    if ((rc = alloc(&S.rowlen, nn)) || (rc = alloc(&S.acol, mat)) || (rc = alloc(&S.aval, mat)) ||
+        (rc = alloc(&S.slen, nn)) || (rc = alloc(&S.scol, mat)) || (rc = alloc(&S.sval, mat)) ||
+        (rc = alloc(&S.diag, nn)) || (rc = alloc(&S.inv_d, nn)) || (rc = alloc(&S.inv_osum, nn)) ||
+        (rc = alloc(&S.feat, nn * LF)) || (rc = alloc(&S.rhs, nn)) || (rc = alloc(&upos, nn))) {
         cleanup();
         return rc;
     }
