@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(
 // candidates at a time, the accepted ones keep their order (ballot) and wait in
 // LDS for stores of whole pieces of the row. One thread per particle is a chain
 // of some ten round trips whatever the size; here a chain is a third of that, and
-// a small system has 16 times the waves (kLanesMax2d has the figures).
+// a small system has 16 times the waves (lanes_max has the figures).
 constexpr int kRowBuf = 64;                            // accepted ids a row holds in LDS
 constexpr int kRowBufStride = kRowBuf + 1;
 
@@ -997,12 +997,19 @@ static int launch_one(vox_ctx* c, int which, double re)
     return search_one(c, which, re);
 }
 
-// The walk per particle takes 16 lanes up to this many particles. NEIGHBOR calls,
-// one thread and 16 lanes, us: 2D 2k particles 42 / 31, 26k 53 / 44, 69k 54 / 50,
-// 250k 78 / 92; 3D 15k 135 / 56, 61k 145 / 109, 201k 309 / 260, 485k 561 / 574.
-// (in 2D twice as many where rows are longer than one group of 16: five weakly
-// compressible steps of 69k particles at 4 spacings 1360 -> 1320 us).
-constexpr int kLanesMax2d = 1 << 16, kLanesMax3d = 1 << 18;
+// The walk per particle takes 16 lanes up to this many particles, by the entries
+// expected in a row (a short row leaves most of a group's last 16 lanes idle).
+// NEIGHBOR calls, one thread and 16 lanes, us: 2D rows of 14 entries 50k 49 / 47, 65k 53 /
+// 53, 100k 52 / 53, of 21 50k 47 / 47, 65k 51 / 52, 100k 59 / 65, of 30 65k 53 / 51, 100k
+// 61 / 62, 131k 68 / 74, of 50 80k 63 / 60, 100k 67 / 68, 131k 70 / 77; 3D rows of 17 60k
+// 71 / 65, 131k 86 / 84, 260k 123 / 132, of 39 60k 90 / 73, 100k 104 / 99, 131k 111 / 118, 260k
+// 157 / 177, of 65 60k 115 / 82, 131k 135 / 128, 220k 211 / 189, 320k 241 / 249.
+static int lanes_max(const vox_params& p, double re)
+{
+    const double e = row_entries(p, re);
+    if (p.dim == 3) return e > 48.0 ? 1 << 18 : 3 << 15;
+    return e > 24.0 ? 3 << 15 : 1 << 16;
+}
 // and against the matrix cores up to this many (16 lanes, matrix): 10k 69 / 171,
 // 43k 134 / 196, 94k 229 / 238, 133k 304 / 244 at 4 spacings, 149 / 176 and 193 /
 // 195 for the last two at 3.1. Half as many for list L, whose consumers read the
@@ -1050,7 +1057,7 @@ static int search_one(vox_ctx* c, int which, double re)
         else
             k_build_list_mm<false><<<(n + kWave - 1) / kWave, kWave, 0, c->stream>>>(
                 gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
-    } else if (n <= (c->p.dim == 3 ? kLanesMax3d : kLanesMax2d * (row_entries(c->p, re) > 16.0 ? 2 : 1))) {
+    } else if (n <= lanes_max(c->p, re)) {
         k_build_list_l16<<<grid_for(16L * n), kBlock, 0, c->stream>>>(
             gg, n, R, L.cell_start, L.rec, L.cap, L.ids, L.cnt, c->dspread, sm);
     } else {

@@ -59,7 +59,7 @@ __global__ void k_pack_pos(int n, int dim, const double* __restrict__ x,
 // row's next 16 entries and every sum adds the lanes' terms in lane order (the
 // row's; an entry that is left out adds +0, which changes no bit of a sum that
 // starts at +0). One thread per particle is a chain of some six round trips
-// whatever the size. The figures are at kStageLanesShort.
+// whatever the size. The figures are at by_lanes.
 struct LaneRow {
     int i, sub;                                        // particle, lane of its row
     bool live;
@@ -84,19 +84,20 @@ __device__ __forceinline__ void walk16(const ListView& L, int self, int cnt, int
         j = jn;
     }
 }
-// Up to this many particles 16 lanes take one. Stages (with their packing), one
-// thread and 16 lanes, us. PNUM / SPS / VISCOSITY (Herschel-Bulkley) / PRESSGRAD: 2D
-// 2k particles 10.6 23 12.3 13.7 / 10.9 10.7 6.4 10.8, 26k 10.8 24 12.8 13.9 / 10.9
-// 14.6 12.3 11.1, 69k 12.6 29 16.5 16.4 / 11.8 29 23.5 16.5; 3D 15k 21 122 71 32 /
-// 10.9 22 23 10.9, 61k 23 124 74 33 / 20 65 63 17, 201k 52 225 168 54 / 51 212 190
-// 50, 485k 88 411 312 113 / 113 516 432 117.
-// Rows of one group of 16 (13 entries: 2D at 2.1 spacings) end earlier than longer
-// ones (37: 3D at 2.1, 50: 2D at 4; five weakly compressible 2D steps of 69k 1360 ->
-// 1240 us).
-constexpr int kStageLanesShort = 3 << 14, kStageLanesLong = 1 << 17;
+// Up to this many particles 16 lanes take one, by the entries expected in a row. Time
+// with 16 lanes over time with one thread, all of PNUM, SPS, V_FRACTION, VISCOSITY
+// (Herschel-Bulkley), PRESSGRAD and COLLISION2 together: 2D rows of 14 entries 30k 0.80, 49k
+// 0.94, 65k 1.07, 131k 1.33, of 21 49k 0.97, 65k 1.12, of 30 80k 0.77, 100k 0.90, 131k
+// 1.06, of 50 80k 0.71, 100k 0.84, 131k 1.00; 3D rows of 17 49k 0.83, 80k 0.93, 131k
+// 1.28, of 39 80k 0.77, 131k 1.11, of 125 80k 0.63, 131k 0.88. 2D 30k particles of 50
+// entries, us: PNUM 19 -> 12, SPS 76 -> 33, V_FRACTION 27 -> 9, VISCOSITY 40 -> 20, PRESSGRAD
+// 29 -> 15, COLLISION2 36 -> 27.
+// VISCOSITY crosses earliest (of 14 entries 30k 0.89, 49k 1.18, of 30 80k 0.92, 100k
+// 1.11, of 50 100k 1.00, 131k 1.27): it counts a third more particles.
 static bool by_lanes(const vox_params& p, double re, long n)
 {
-    return n <= (row_entries(p, re) > 16.0 ? kStageLanesLong : kStageLanesShort);
+    const double e = row_entries(p, re);
+    return n <= (e > 48.0 ? 1 << 17 : e > 24.0 ? 3 << 15 : 3 << 14);
 }
 static int lane_blocks(long n) { return grid_for(16 * n); }
 
@@ -610,7 +611,7 @@ int st_viscosity(vox_ctx* c)
         a.x = c->f[VOX_F_X]; a.y = c->f[VOX_F_Y]; a.z = c->f[VOX_F_Z];
         a.u = c->f[VOX_F_UNEW]; a.v = c->f[VOX_F_VNEW]; a.w = c->f[VOX_F_WNEW];
         a.phat = c->f[VOX_F_PHAT]; a.meu = c->f[VOX_F_MEU];
-        if (by_lanes(c->p, c->p.re_s, c->tp)) k_visc_hb<true><<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(a);
+        if (by_lanes(c->p, c->p.re_s, c->tp + c->tp / 3)) k_visc_hb<true><<<lane_blocks(c->tp), kBlock, 0, c->stream>>>(a);
         else k_visc_hb<false><<<grid_for(c->tp), kBlock, 0, c->stream>>>(a);
     }
     VOX_HIP(hipGetLastError());
