@@ -14,9 +14,10 @@
 // rz is double-buffered by iteration parity (K3 of iteration k writes slot
 // k&1 while its blocks read slot (k-1)&1). The stop flag stays on the device;
 // kernels launched after convergence return at entry.
-// Up to kFusedBlocks product blocks K1 does K3's work itself, each block for
-// its window of p (two kernels an iteration); the smallest systems run the
-// whole solve in one block (k_cg_one). Same bits in every form.
+// Up to kFusedBlocks product blocks, and past them where the blocks' windows stage
+// at most 4 columns a row (2D), K1 does K3's work itself, each block for its window
+// of p (two kernels an iteration; updates_p); the smallest systems run the whole
+// solve in one block (k_cg_one). Same bits in every form.
 //
 // The kernels are templated on the vector type VT and the matrix value type
 // MT; dot products always accumulate in FP64. VT = MT = double is the FP64

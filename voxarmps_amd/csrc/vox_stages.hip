@@ -912,9 +912,9 @@ __global__ __launch_bounds__(BS) void k_prediction_dg(PredArgs a)
 // out where every particle of the wave has none.
 // Measured against the walk of variant 6: 820k rows of 222 entries 1472 us
 // (1690), 103k rows 215 us (324), 2D two-phase of 22k particles 20 us (41), 2D of
-// 1.2k 6.6 us (31). At 820k rows bound by the L1 lookups of the gathers (3 a
-// record, 86 % of the cycles). Adding in every lane by lane broadcast: 1545 us,
-// 236 us; with that, records brought to LDS four lanes a record (a third of the
+// 1.2k 6.6 us (31). At 820k rows no unit is at its limit (L1 lookups, 3 a record,
+// 0.66 a cycle of a CU, VALU 47 %, address path 51 %): latency of the gathers at 4
+// waves per SIMD. Adding in every lane by lane broadcast: 1545 us, 236 us; with that, records brought to LDS four lanes a record (a third of the
 // lookups) 1690 us, 267 us; 96 registers for a fifth wave spill (3566 us).
 // Blocks of 128, 512, 1024 threads: 1527, 1513, 1566 us (103k rows 209, 233, 250).
 constexpr int kPredSlots = 80;                     // queued entries of a row
