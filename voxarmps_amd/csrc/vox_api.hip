@@ -145,21 +145,24 @@ static int await_signal(vox_ctx* c, const uint32_t* sig, uint32_t ticket)
     return VOX_OK;
 }
 
-static int fetch(vox_ctx* c, void* dst, const void* src, size_t bytes)
+// One fetch of a context at a time: a second thread's ticket in the one signal word
+// would hide the first's.
+static int fetch(vox_ctx* c, void* dst, const void* src, size_t bytes, int32_t* word = nullptr)
 {
+    std::lock_guard<std::mutex> lock(c->fetch_m);
     const uint32_t ticket = ++c->ticket;
     k_fetch<<<1, kBlock, 0, c->stream>>>((const uint32_t*)src, (uint32_t*)dst, (int)(bytes / 4), c->hsig, ticket);
     VOX_HIP(hipGetLastError());
-    return await_signal(c, c->hsig, ticket);
+    VOX_TRY(await_signal(c, c->hsig, ticket));
+    if (word) *word = *static_cast<const int32_t*>(dst);
+    return VOX_OK;
 }
 
 int read_flags(vox_ctx* c) { return fetch(c, c->hstat, c->dstat, kStatBytes); }
 
 int read_i32(vox_ctx* c, const int32_t* src, int32_t* value)
 {
-    VOX_TRY(fetch(c, c->hsig + kSigWord, src, sizeof(int32_t)));
-    *value = (int32_t)c->hsig[kSigWord];
-    return VOX_OK;
+    return fetch(c, c->hsig + kSigWord, src, sizeof(int32_t), value);
 }
 
 // Device memory to the caller's array, through the context's pinned buffer. A

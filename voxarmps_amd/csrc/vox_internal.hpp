@@ -257,6 +257,7 @@ struct vox_ctx {
     HostStage stage;
     uint32_t* hsig = nullptr;      // pinned signal words (kSigCount), after hstat
     std::atomic<uint32_t> ticket{0};   // the last one given out
+    std::mutex fetch_m;            // held by a read of the status or of one word
     int32_t* dpiece = nullptr;     // blocks done of each piece of a download
 
     double* f[VOX_F_COUNT] = {};
