@@ -607,6 +607,7 @@ int vox_create(vox_ctx** out, const vox_params* pin, int tp, int gp, int wp, int
     if (c->p.pmax <= 0) c->p.pmax = (double)tp * 4.50;              // main.cu:548
     c->tp = tp; c->gp = gp; c->wp = wp; c->fp = fp;
     c->two_lists = (c->p.re_l != c->p.re_s);
+    c->tune_pred = default_predictor(c->p, tp);
     int rc = VOX_OK;
     auto bail = [&](int code) { vox_destroy(c); return code; };
     if (hipGetDevice(&c->device) != hipSuccess) return bail(fail(VOX_ERR_HIP, "hipGetDevice"));

@@ -272,8 +272,8 @@ struct vox_ctx {
     vox::DevList list[2];
     int max_count[2] = {0, 0};     // longest row of each list's last search
     int tuned_mode[2] = {0, 0};    // neighbour walk chosen by the autotuner (0: none)
-    int tune_pred = 8;             // predictor variant (vox::kPredVariants): 16 lanes per
-                                   // particle unless tuned
+    int tune_pred = 8;             // predictor variant (vox::kPredVariants): that of
+                                   // default_predictor unless tuned
     int tune_spmv = 0;             // PPE product variant (vox::kSpmvVariants)
     bool two_lists = false;
     double n0s = 0.0, n0l = 0.0;
@@ -485,6 +485,7 @@ int to_host(vox_ctx* c, void* host, const void* src, size_t bytes);   // synchro
 int read_i32(vox_ctx* c, const int32_t* src, int32_t* value);         // synchronous
 int32_t spread_sum(const vox_ctx* c, int slot);
 
+int default_predictor(const vox_params& p, long n);             // vox_stages.hip
 int autotune_lists(vox_ctx* c, int reps, int32_t* modes);
 int build_neighbors(vox_ctx* c);
 bool list_compact_ok(const vox_ctx* c);

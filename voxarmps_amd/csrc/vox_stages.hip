@@ -1091,6 +1091,22 @@ bool uniform_meu(const vox_ctx* c)
 static const int kPredR[kPredVariants] = {4, 8, 2, 4, 8, 8, 8, 4, 1};
 static const int kPredBS[kPredVariants] = {256, 256, 256, 128, 128, 128, 256, 128, 256};
 
+// The FP64 predictor of a context that is not tuned: 16 lanes per particle up to a size
+// that grows with the entries of both lists' rows, beyond it one thread per particle
+// with the gradient deferred. Us, variants 6, 7 and 8, entries of S + L: 2D 14 + 14 49k
+// 23 24 22, 80k 31 27 33, 131k 35 35 50, 600k 134 120 207; 14 + 30 65k 33 35 31, 98k 44
+// 39 44, 131k 47 44 56, 400k 129 115 153; 14 + 50 80k 54 47 43, 98k 57 48 50, 131k 60 55
+// 64, 400k 168 152 176; 50 + 50 98k 80 68 64, 131k 83 78 83, 196k 126 109 119, 600k 350
+// 323 364; 3D 17 + 17 60k 40 40 35, 98k 53 47 52, 131k 57 56 67, 400k 176 182 191; 39 + 39
+// 98k 81 69 68, 131k 84 83 88, 262k 163 199 167, 800k 554 607 561; 39 + 74 131k 100 97
+// 93, 800k 644 728 622; 39 + 268 130k 191 187 169, 500k 791 883 737.
+int default_predictor(const vox_params& p, long n)
+{
+    const double e = row_entries(p, p.re_s) + row_entries(p, p.re_l);
+    if (p.dim == 3) return (e > 100.0 || n <= 3 << 15) ? 8 : 6;
+    return n <= (e > 90.0 ? 1 << 17 : e > 55.0 ? 3 << 15 : e > 40.0 ? 1 << 16 : 3 << 14) ? 8 : 7;
+}
+
 template <bool kU>
 static void launch_pred_u(const PredArgs& a, int v, int n, hipStream_t s)
 {
